@@ -32,6 +32,9 @@ constexpr uint32_t ERR_SCRATCH = 1, ERR_BUCKET = 2, ERR_POOL = 4, ERR_HEADER = 8
 
 constexpr uint32_t kMaxEditLevels = 17;
 constexpr uint32_t kUndoCap = 1u << 20;
+constexpr uint32_t kSegColors = 4096;  // colours of one encoder segment
+// segments that staged colours of capacity `colors` over at most `tasks` tasks can need
+inline uint64_t encode_segments(uint64_t colors, uint64_t tasks) { return colors / kSegColors + tasks; }
 
 // An editor with its derived bounds (hash_dag_editors.h:57-127): box min/max = c -/+ r,
 // r2 = r * r, `single` = rgb101210 colour of add editors (sphere red, box magenta).
@@ -154,6 +157,12 @@ struct EditPass {
     uint64_t* colors;
     uint64_t* cmarks;  // per 64-colour chunk of `colors`: kUniformChunk | colour, or 0 (explicit)
     uint64_t color_cap;
+    // encoder: the task of every segment of kSegColors staged colours, and the segment's blocks
+    // and weight bits (counts, then offsets in the task's leaf)
+    uint32_t* seg_task;
+    uint2* seg_out;
+    uint32_t seg_cap;
+    uint32_t* seg_top;
     uint32_t* cnodes;
     uint32_t cnodes_cap;
     const uint64_t* offsets;
@@ -179,6 +188,9 @@ struct EditScratch {
     uint32_t* hset = nullptr;
     uint64_t* colors = nullptr;
     uint64_t* cmarks = nullptr;
+    uint32_t* seg_task = nullptr;
+    uint2* seg_out = nullptr;
+    uint32_t seg_cap = 0;
     uint32_t* dcount = nullptr;
     uint32_t* decount = nullptr;
     uint64_t* dstats = nullptr;

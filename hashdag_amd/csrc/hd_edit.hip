@@ -1332,9 +1332,8 @@ __global__ __launch_bounds__(256) void k_color_starts(EditPass P, uint32_t l) {
     d_color_starts(P, l, VGrid{blockIdx.x, gridDim.x});
 }
 
-// colour array of every task with colours: base offset in the colour scratch. Arrays start on
-// a 64-colour chunk; the chunk markers of the wave's range are cleared here (the colour
-// writers mark the chunks they fill with one colour).
+// colour array of every task with colours: base offset in the colour scratch (arrays start on a
+// 64-colour chunk) and its segments for the encoder
 __device__ __forceinline__ void d_color_alloc(const EditPass& P, VGrid G) {
     const uint32_t ctl = P.ctl;
     const uint32_t n = min(P.count[ctl], P.cap[ctl]);
@@ -1347,14 +1346,16 @@ __device__ __forceinline__ void d_color_alloc(const EditPass& P, VGrid G) {
         const uint64_t acnt = ((uint64_t)cnt + 63u) & ~63ull;
         const uint64_t base = wave_alloc64(P.color_top, acnt);
         wave_add64(P.stat_colors, cnt);
-        if (i < n) T.cbase[i] = base;
-        // the wave's arrays are contiguous: [base of lane 0, end of lane 63)
-        const uint64_t lo = shfl64(base, 0), hi = shfl64(base + acnt, 63);
-        if (hi > P.color_cap) {
-            if (lane == 0) set_error(P.errors, ERR_COLOR_SCRATCH);
-            continue;
+        const uint32_t nSeg = (cnt + kSegColors - 1u) / kSegColors;
+        const uint32_t seg = wave_alloc32(P.seg_top, nSeg);
+        if (i < n) {
+            T.cbase[i] = base;
+            T.hash[i] = seg;
         }
-        for (uint64_t k = lo / 64 + lane; k < hi / 64; k += 64) P.cmarks[k] = 0;
+        // colour arrays within the capacity never need more segments than seg_cap
+        if (base + acnt > P.color_cap || seg + nSeg > P.seg_cap) set_error(P.errors, ERR_COLOR_SCRATCH);
+        else
+            for (uint32_t k = 0; k < nSeg; ++k) P.seg_task[seg + k] = i;
     }
 }
 __global__ __launch_bounds__(256) void k_color_alloc(EditPass P) {
@@ -1372,7 +1373,7 @@ __device__ __forceinline__ LeafDesc task_leaf(const EditPass& P, uint32_t handle
 
 // DAGUtils::get_color (dag_utils.h:423-523) of voxel (x, y, z) in the DAG at `root`: the colour
 // at the voxel's rank in its colour subtree, CompressedColor{} (0) when absent. The colour
-// slots hold the pass's starting colours until k_encode writes the new leaves.
+// slots hold the pass's starting colours until k_enc_scan writes the new leaves.
 __device__ uint64_t source_color(const EditPass& P, uint32_t root, uint32_t x, uint32_t y, uint32_t z) {
     const uint32_t levels = P.levels, L = levels - 2, ctl = P.ctl;
     const uint32_t* __restrict__ vpool = P.vpool;
@@ -1844,6 +1845,11 @@ __global__ __launch_bounds__(256) void k_color_leaf(EditPass P) {
 // level-ctl node position), so they are written without atomics.
 __device__ __forceinline__ void d_color_tree(const EditPass& P, VGrid G) {
     if (*P.errors) return;
+    // the chunk markers of the staged colours start cleared: the colour writers (which run after
+    // this step) mark the chunks they fill with one colour
+    const uint64_t chunks = min((uint64_t)*P.color_top, P.color_cap) / 64;
+    for (uint64_t k = (uint64_t)G.block * blockDim.x + threadIdx.x; k < chunks; k += (uint64_t)G.nblocks * blockDim.x)
+        P.cmarks[k] = 0;
     const uint32_t ctl = P.ctl;
     const uint32_t n = min(P.count[ctl], P.cap[ctl]);
     const Items T = P.items[ctl];
@@ -1927,12 +1933,18 @@ __global__ __launch_bounds__(256) void k_gather_leaves(const LeafDesc* leaves, c
         out[k] = leaves[handles[k] & 0x7FFFFFFFu];
 }
 
-// Colour leaf encoder (k_encode): per task, a counting walk over the colours (blocks and weight
-// bits), then a writing walk in chunks of 64 with wave scans carried across chunks. Weight bits
-// of a chunk are gathered in LDS and each weight word is written once (the word a chunk leaves
-// partial is carried to the next chunk).
+// Colour leaf encoder. A task's staged colours are cut into segments of kSegColors colours, a
+// wavefront each, in three steps: k_enc_count counts every segment's blocks and weight bits,
+// k_enc_scan turns a task's counts into offsets, reserves its arena words and writes what lies
+// at segment starts (macro-block records, zeroed weight words that two segments share), and
+// k_enc_write writes blocks and weight words at those offsets. The walks are a chain of
+// dependent loads and scans, so they are bound by the longest chain: a wavefront per task (the
+// segments of a task one after another) took 171 us for one brush stroke's few tasks and 745 us
+// for a pass of 48 editors, with most of the chip idle.
 constexpr uint32_t kEncBlock = 256;
 constexpr uint32_t kEncWaves = kEncBlock / 64;
+constexpr uint32_t kSegChunks = 64;  // a marker per lane
+static_assert(kSegColors == kSegChunks * 64 && 16384 % kSegColors == 0, "macro blocks start at segment starts");
 
 __device__ __forceinline__ uint32_t wave_sum(uint32_t v) {
 #pragma unroll
@@ -1957,173 +1969,243 @@ __device__ __forceinline__ uint64_t shfl_up64(uint64_t v) {
     return ((uint64_t)__shfl_up((uint32_t)(v >> 32), 1, 64) << 32) | __shfl_up((uint32_t)v, 1, 64);
 }
 
-// One task's staged colours, chunk by chunk, in colour order. A block starts where the colour
-// index is a multiple of 16384 or the colour bits / bits per weight differ from the previous
-// colour's (the same rule as the leaf builder). Uniform chunks (markers) hold no weights and
-// can start a block only at their first colour, so a run of them is handled 64 chunks at a
-// time. kWrite = false counts blocks and weight bits; kWrite = true writes blocks, macro-block
-// records and weight words at the counted sizes. Weight bits of an explicit chunk are gathered
-// in LDS and each weight word is written once (the word a chunk leaves partial is carried).
+// Where a segment's output starts, and where it goes (kWrite only).
+struct EncOut {
+    uint64_t* blocks;
+    uint32_t* weights;
+    uint32_t block0, bit0, macroBit;  // offsets in the leaf; bit offset of the segment's macro block
+    uint32_t* buf;                    // LDS: weight words of one group
+};
+constexpr uint32_t kEncBuf = 34;  // 256 colours of at most 4 bits from an unaligned start
+
+// One segment (colours [s0, s0 + kSegColors) of a task's cnt), chunk by chunk in colour order. A
+// block starts where the colour index is a multiple of 16384 or the colour bits / bits per weight
+// differ from the previous colour's (the same rule as the leaf builder). Uniform chunks (markers)
+// hold no weights and can start a block only at their first colour, so a run of them is handled
+// at once. From an explicit chunk on, four chunks are taken together, four consecutive colours a
+// lane: one scan per 256 colours gives block and weight-bit offsets. kWrite = false counts blocks
+// and weight bits; kWrite = true writes them. Weight bits of a group are gathered in LDS and each
+// weight word is written once; the segment's first and last words may be shared with its
+// neighbours and are ORed into words that k_enc_scan has zeroed.
 template <bool kWrite>
-__device__ __forceinline__ void encode_colors(const uint64_t* __restrict__ cols, const uint64_t* __restrict__ marks,
-                                              uint32_t cnt, uint32_t lane, uint32_t* buf, uint64_t* blocks,
-                                              uint64_t* macro, uint32_t* weights, uint32_t& outBlocks,
-                                              uint32_t& outBits) {
-    uint32_t carryBlocks = 0, carryBits = 0, macroBit = 0, carryWord = 0, laneBits = 0;
-    uint64_t prev = 0;  // the colour before the current chunk (unused at colour 0)
-    const uint32_t nCh = (cnt + 63u) / 64u;
-    for (uint32_t g0 = 0; g0 < nCh; g0 += 64) {
-        const uint32_t gl = min(64u, nCh - g0);
-        const uint64_t mk = lane < gl ? marks[g0 + lane] : 0ull;
-        const uint64_t marked = __ballot((mk & kUniformChunk) != 0);
-        uint32_t j = 0;
-        while (j < gl) {
-            if ((marked >> j) & 1ull) {
-                // uniform chunks j .. e-1 (lane k: chunk g0 + k)
-                const uint64_t open = ~marked >> j;
-                const uint32_t e = min(open ? j + (uint32_t)__ffsll((long long)open) - 1u : 64u, gl);
-                const uint64_t col = mk & 0xFFFFFFFFull;
-                const uint32_t upc = __shfl_up((uint32_t)col, 1, 64);
-                const bool in = lane >= j && lane < e;
-                const uint32_t pos = (g0 + lane) * 64u;
-                const bool mstart = in && (pos & 16383u) == 0;
-                const bool st = mstart || (in && (lane == j ? ((prev ^ col) & kColorKey) != 0 : upc != (uint32_t)col));
-                const uint64_t sb = __ballot(st);
-                if constexpr (kWrite) {
-                    const uint32_t bi = carryBlocks + (uint32_t)__popcll(sb & (~0ull >> (63u - lane)));
-                    if (st) blocks[bi - 1] = (col << 32) | (0xFFFFu << 16) | (pos & 16383u);
-                    if (mstart) {
-                        macro[2 * (pos >> 14)] = bi - 1;
-                        macro[2 * (pos >> 14) + 1] = carryBits;
-                    }
-                    if (__ballot(mstart)) macroBit = carryBits;
-                }
-                carryBlocks += (uint32_t)__popcll(sb);
-                prev = __shfl((uint32_t)col, e - 1, 64);
-                j = e;
-                continue;
+__device__ __forceinline__ void encode_segment(const uint64_t* __restrict__ cols, const uint64_t* __restrict__ marks,
+                                               uint32_t cnt, uint32_t s0, uint32_t lane, const EncOut& O,
+                                               uint32_t& outBlocks, uint32_t& outBits) {
+    const uint32_t ch0 = s0 / 64u, gl = min(kSegChunks, (cnt + 63u) / 64u - ch0);
+    const uint64_t mk = lane < gl ? marks[ch0 + lane] : 0ull;
+    const uint64_t marked = __ballot((mk & kUniformChunk) != 0);
+    uint64_t prev = 0;  // the colour before the current chunk (unused where a macro block starts)
+    const bool macroStart = (s0 & 16383u) == 0;
+    if (!macroStart) {
+        const uint64_t pm = marks[ch0 - 1];
+        prev = (pm & kUniformChunk) ? (pm & 0xFFFFFFFFull) : cols[s0 - 1];
+    }
+    uint32_t nBlocks = kWrite ? O.block0 : 0u, nBits = kWrite ? O.bit0 : 0u, carryWord = 0;
+    uint32_t laneStarts = 0, laneBits = 0;
+    uint32_t j = 0;
+    while (j < gl) {
+        if ((marked >> j) & 1ull) {
+            // uniform chunks j .. e-1 (lane k: chunk ch0 + k)
+            const uint64_t open = ~marked >> j;
+            const uint32_t e = min(open ? j + (uint32_t)__ffsll((long long)open) - 1u : 64u, gl);
+            const uint64_t col = mk & 0xFFFFFFFFull;
+            const uint32_t upc = __shfl_up((uint32_t)col, 1, 64);
+            const bool in = lane >= j && lane < e;
+            const bool st = in && (lane == j ? ((macroStart && j == 0) || ((prev ^ col) & kColorKey) != 0)
+                                             : upc != (uint32_t)col);
+            const uint64_t sb = __ballot(st);
+            if constexpr (kWrite) {
+                if (st)
+                    O.blocks[nBlocks + (uint32_t)__popcll(sb & ((1ull << lane) - 1ull))] =
+                        (col << 32) | (0xFFFFu << 16) | ((s0 + lane * 64u) & 16383u);
             }
-            // explicit chunk
-            const uint32_t c0 = (g0 + j) * 64u, i = c0 + lane;
-            uint64_t c = 0;
-            uint32_t bpw = 0;
-            if (i < cnt) {
-                c = cols[i];
-                bpw = (uint32_t)(c >> 40) & 0xFFu;
+            nBlocks += (uint32_t)__popcll(sb);
+            prev = __shfl((uint32_t)col, e - 1, 64);
+            j = e;
+            continue;
+        }
+        // chunks j .. j+3: lane k takes colours 4 k .. 4 k + 3 of the 256, its chunk is j + k / 16
+        const uint32_t ck = j + (lane >> 4);
+        const uint32_t i0 = s0 + j * 64u + lane * 4u;
+        const uint32_t nv = ck < gl && i0 < cnt ? min(cnt - i0, 4u) : 0u;
+        const uint64_t cm = shfl64(mk, ck & 63u);
+        uint64_t c[4];
+        if (nv && (cm & kUniformChunk)) {
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q) c[q] = cm & 0xFFFFFFFFull;
+        } else {
+            const ulonglong2* p = reinterpret_cast<const ulonglong2*>(cols + i0);  // 32-byte aligned
+            ulonglong2 a{0, 0}, b{0, 0};
+            if (nv) {  // arrays are whole chunks: colours past cnt are in memory, and masked below
+                a = p[0];
+                b = p[1];
             }
-            const uint64_t up = shfl_up64(c);
-            const uint64_t p = lane == 0 ? prev : up;
-            const uint32_t start = i < cnt && ((i & 16383u) == 0 || ((p ^ c) & kColorKey) != 0);
-            prev = shfl64(c, 63);
-            ++j;
-            if constexpr (!kWrite) {
-                carryBlocks += (uint32_t)__popcll(__ballot(start));
-                laneBits += bpw;
-            } else {
-                const uint32_t sA = wave_incl_scan(start, lane), sB = wave_incl_scan(bpw, lane);
-                const uint32_t blockIdxIncl = carryBlocks + sA;  // block index + 1 if start
-                const uint32_t bitOff = carryBits + sB - bpw;    // exclusive bit offset
-                // only lane 0 can sit on a macro-block start (16384 is a multiple of 64)
-                uint32_t myMacroBit = macroBit;
-                if ((c0 & 16383u) == 0) {
-                    myMacroBit = carryBits;
-                    macroBit = carryBits;
-                    if (lane == 0) {
-                        macro[2 * (c0 >> 14)] = blockIdxIncl - 1;
-                        macro[2 * (c0 >> 14) + 1] = bitOff;
-                    }
+            c[0] = a.x;
+            c[1] = a.y;
+            c[2] = b.x;
+            c[3] = b.y;
+        }
+        const uint64_t up = shfl_up64(c[3]);
+        uint64_t before = lane == 0 ? prev : up;
+        uint32_t starts = 0, nb = 0, str = 0;  // starts: bit q; str: the lane's weight bits, MSB first
+        uint32_t off[4], w[4];
+#pragma unroll
+        for (uint32_t q = 0; q < 4; ++q) {
+            w[q] = q < nv ? (uint32_t)(c[q] >> 40) & 0xFFu : 0u;
+            off[q] = nb;
+            nb += w[q];
+            if (kWrite) str = (str << w[q]) | ((uint32_t)(c[q] >> 32) & ((1u << w[q]) - 1u));
+            const bool st = q < nv && (((before ^ c[q]) & kColorKey) != 0 || (macroStart && q == 0 && j + lane == 0));
+            starts |= (uint32_t)st << q;
+            before = c[q];
+        }
+        prev = shfl64(c[3], 63);  // read again only if this group is full
+        j += 4;
+        const uint32_t ns = (uint32_t)__popc(starts);
+        if constexpr (!kWrite) {
+            laneStarts += ns;
+            laneBits += nb;
+        } else {
+            // block starts in the low half, weight bits (at most 1024 a group) in the high half
+            const uint32_t incl = wave_incl_scan(ns | (nb << 16), lane);
+            const uint32_t tot = __shfl(incl, 63, 64);
+            uint32_t bi = nBlocks + (incl & 0xFFFFu) - ns;
+            const uint32_t bit = nBits + (incl >> 16) - nb;
+#pragma unroll
+            for (uint32_t q = 0; q < 4; ++q)
+                if ((starts >> q) & 1u) {
+                    const uint32_t li = (i0 + q) & 16383u, rel = bit + off[q] - O.macroBit;
+                    const uint32_t hdr = w[q] == 0 ? ((0xFFFFu << 16) | li) : ((rel << 16) | ((w[q] - 1) << 14) | li);
+                    O.blocks[bi++] = ((uint64_t)(uint32_t)c[q] << 32) | hdr;
                 }
-                if (i < cnt && start) {
-                    const uint32_t rel = bitOff - myMacroBit;
-                    const uint32_t hdr = bpw == 0 ? ((0xFFFFu << 16) | (i & 16383u))
-                                                  : ((rel << 16) | ((bpw - 1) << 14) | (i & 16383u));
-                    blocks[blockIdxIncl - 1] = ((uint64_t)(uint32_t)c << 32) | hdr;
-                }
-                // weight bits of the chunk: [B0, B1), words w0 .. ; MSB-first stream bit k ->
-                // stored word k / 32, byte (k % 32) / 8, bit 7 - k % 8
-                const uint32_t B0 = carryBits, B1 = carryBits + __shfl(sB, 63, 64);
-                const uint32_t w0 = B0 >> 5;
-                if (lane < 12) buf[lane] = lane == 0 ? carryWord : 0u;
-                wave_sync();
-                if (bpw) {
-                    const uint32_t wvv = (uint32_t)(c >> 32) & 0xFFu;
-                    for (uint32_t b = 0; b < bpw; ++b) {
-                        if (!((wvv >> (bpw - 1 - b)) & 1u)) continue;
-                        const uint32_t k = bitOff + b;
-                        atomicOr(&buf[(k >> 5) - w0], 1u << (((k & 31u) >> 3) * 8u + (7u - (k & 7u))));
-                    }
-                }
-                wave_sync();
-                const uint32_t full = (B1 >> 5) - w0;  // complete words of the chunk
-                if (lane < full) weights[w0 + lane] = buf[lane];
-                carryWord = (B1 & 31u) ? buf[full] : 0u;
-                wave_sync();
-                carryBlocks = __shfl(blockIdxIncl, 63, 64);
-                carryBits = B1;
+            // weight bits of the group, [nBits, B1): stream bit k is in word k / 32, byte
+            // (k % 32) / 8, bit 7 - k % 8, so a word is the byte-swapped MSB-first string
+            const uint32_t B1 = nBits + (tot >> 16), w0 = nBits >> 5;
+            if (lane < kEncBuf) O.buf[lane] = lane == 0 ? carryWord : 0u;
+            wave_sync();
+            if (nb) {
+                const uint32_t p = bit & 31u;
+                const uint64_t v = (uint64_t)str << (64u - p - nb);
+                atomicOr(&O.buf[(bit >> 5) - w0], __builtin_bswap32((uint32_t)(v >> 32)));
+                if (p + nb > 32u) atomicOr(&O.buf[(bit >> 5) - w0 + 1], __builtin_bswap32((uint32_t)v));
             }
+            wave_sync();
+            const uint32_t full = (B1 >> 5) - w0;  // complete words of the group
+            if (lane < full) {
+                if (w0 + lane == O.bit0 >> 5 && (O.bit0 & 31u)) atomicOr(&O.weights[w0 + lane], O.buf[lane]);
+                else O.weights[w0 + lane] = O.buf[lane];
+            }
+            carryWord = (B1 & 31u) ? O.buf[full] : 0u;
+            wave_sync();
+            nBlocks += tot & 0xFFFFu;
+            nBits = B1;
         }
     }
-    outBlocks = carryBlocks;
     if constexpr (kWrite) {
-        outBits = carryBits;
-        if (lane == 0 && (carryBits & 31u)) weights[carryBits >> 5] = carryWord;
+        if (lane == 0 && (nBits & 31u) && nBits != O.bit0) atomicOr(&O.weights[nBits >> 5], carryWord);
     } else {
+        outBlocks = nBlocks + wave_sum(laneStarts);
         outBits = wave_sum(laneBits);
     }
 }
 
-// One wavefront per task: encode its colour array into a new unique leaf in the arena. The grid
-// holds a wavefront per task (up to a cap, then a stride), so the hardware hands out tasks to
-// free wavefronts as they finish: task sizes vary by orders of magnitude, and a fixed share of
-// tasks per wavefront would leave the kernel's time to the wavefront with the largest share.
-// Each task reserves its arena words with one atomic once its blocks and weight bits are
-// counted.
-__device__ __forceinline__ void d_encode(const EditPass& P, VGrid G) {
-    const uint32_t ctl = P.ctl;
-    const uint32_t n = min(P.count[ctl], P.cap[ctl]);
+// one wavefront per segment: its blocks and weight bits. T.hash[t] (free after the finds) is the
+// first entry of task t's segments in seg_task / seg_out.
+__device__ __forceinline__ void d_enc_count(const EditPass& P, VGrid G) {
     if (*P.errors) return;
-    const Items T = P.items[ctl];
-    __shared__ uint32_t sBits[kEncWaves][12];
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
-    uint32_t* buf = sBits[wv];
+    const uint32_t nSeg = min(*P.seg_top, P.seg_cap);
+    const Items T = P.items[P.ctl];
+    const uint32_t lane = threadIdx.x & 63u;
     uint64_t stagedBytes = 0;  // chunk markers and explicit colours (measurement)
-    for (uint32_t t = G.block * kEncWaves + wv; t < n; t += G.nblocks * kEncWaves) {
-        const uint32_t cnt = T.ncount[t];
-        if (cnt == 0) continue;
-        if ((cnt + 16383u) / 16384u > 160) {  // more than 160 * 16384 colours in one subtree
-            if (lane == 0) set_error(P.errors, ERR_LEAF_SIZE);
-            continue;
-        }
+    for (uint32_t sg = wave_index(G); sg < nSeg; sg += wave_count(G)) {
+        const uint32_t t = P.seg_task[sg], cnt = T.ncount[t], s0 = (sg - T.hash[t]) * kSegColors;
         const uint64_t cb = T.cbase[t];
         if (P.abytes) {
             // each marker and explicit colour (8 B) is written once by the staging kernels and
             // read twice here (the counting walk, then the writing walk)
-            const uint32_t nCh = (cnt + 63u) / 64u;
-            for (uint32_t c = lane; c < nCh; c += 64) {
+            const uint32_t c = s0 / 64u + lane;
+            if (c < (cnt + 63u) / 64u) {
                 const bool uniform = (P.cmarks[cb / 64 + c] & kUniformChunk) != 0;
                 stagedBytes += 24u * (1u + (uniform ? 0u : min(64u, cnt - c * 64u)));
             }
         }
         uint32_t nBlocks, nBits;
-        encode_colors<false>(P.colors + cb, P.cmarks + cb / 64, cnt, lane, buf, nullptr, nullptr, nullptr, nBlocks,
-                             nBits);
+        encode_segment<false>(P.colors + cb, P.cmarks + cb / 64, cnt, s0, lane, EncOut{}, nBlocks, nBits);
+        if (lane == 0) P.seg_out[sg] = make_uint2(nBlocks, nBits);
+    }
+    if (P.abytes) wave_add64(P.abytes + 2, stagedBytes);
+}
+__global__ __launch_bounds__(kEncBlock) void k_enc_count(EditPass P) { d_enc_count(P, VGrid{blockIdx.x, gridDim.x}); }
+
+// A task's segment counts become offsets, its arena words are reserved, and its leaf descriptor
+// and macro records are written, and zeros into the weight words where a segment ends inside a
+// word. A lane per task, and the whole wavefront for a task of many segments; one atomic on the
+// arena's top per wavefront (one per task held a pass of 700,000 tasks for 6.1 ms: one address
+// takes about 155 M atomics a second).
+constexpr uint32_t kLaneSegs = 8;  // segments a lane walks on its own
+__device__ __forceinline__ void enc_scan_marks(uint64_t* macro, uint32_t* weights, uint32_t k, uint2 v) {
+    constexpr uint32_t kPerMacro = 16384u / kSegColors;
+    if (k % kPerMacro == 0) {
+        macro[2 * (k / kPerMacro)] = v.x;
+        macro[2 * (k / kPerMacro) + 1] = v.y;
+    }
+    if (v.y & 31u) weights[v.y >> 5] = 0u;
+}
+__device__ __forceinline__ void d_enc_scan(const EditPass& P, VGrid G) {
+    if (*P.errors) return;
+    const uint32_t ctl = P.ctl;
+    const uint32_t n = min(P.count[ctl], P.cap[ctl]);
+    const Items T = P.items[ctl];
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint32_t t0 = G.block * blockDim.x + (threadIdx.x & ~63u); t0 < n; t0 += G.nblocks * blockDim.x) {
+        const uint32_t t = t0 + lane;
+        uint32_t cnt = t < n ? T.ncount[t] : 0u;
         const uint32_t nMacro = (cnt + 16383u) / 16384u;
-        const uint32_t nWeights = (nBits + 31) / 32;
-        const uint64_t words = (uint64_t)nBlocks + 2ull * nMacro + (nWeights + 1) / 2 + 1;
-        unsigned long long base = 0;
-        if (lane == 0) base = atomicAdd(P.arena_top, (unsigned long long)words);
-        base = shfl64(base, 0);
-        if (base + words > P.arena_cap) {
-            if (lane == 0) set_error(P.errors, ERR_COLOR_ARENA);
-            continue;
+        if (nMacro > 160) {  // more than 160 * 16384 colours in one subtree
+            set_error(P.errors, ERR_LEAF_SIZE);
+            cnt = 0;
         }
-        uint64_t* blocks = P.arena + base;
-        uint64_t* macro = blocks + nBlocks;
+        const uint32_t nSeg = (cnt + kSegColors - 1u) / kSegColors, seg0 = cnt ? T.hash[t] : 0u;
+        uint32_t nBlocks = 0, nBits = 0;
+        const uint64_t big = __ballot(nSeg > kLaneSegs);
+        if (nSeg <= kLaneSegs)
+            for (uint32_t k = 0; k < nSeg; ++k) {
+                const uint2 v = P.seg_out[seg0 + k];
+                P.seg_out[seg0 + k] = make_uint2(nBlocks, nBits);
+                nBlocks += v.x;
+                nBits += v.y;
+            }
+        for (uint64_t m = big; m; m &= m - 1) {  // wave-uniform
+            const uint32_t src = (uint32_t)__ffsll((long long)m) - 1u;
+            const uint32_t sn = __shfl(nSeg, src, 64);
+            uint2* so = P.seg_out + __shfl(seg0, src, 64);
+            uint32_t bTot = 0, wTot = 0;
+            for (uint32_t k0 = 0; k0 < sn; k0 += 64) {
+                const uint32_t k = k0 + lane;
+                const uint2 v = k < sn ? so[k] : make_uint2(0u, 0u);
+                const uint32_t sb = wave_incl_scan(v.x, lane), sw = wave_incl_scan(v.y, lane);
+                if (k < sn) so[k] = make_uint2(bTot + sb - v.x, wTot + sw - v.y);
+                bTot += __shfl(sb, 63, 64);
+                wTot += __shfl(sw, 63, 64);
+            }
+            if (lane == src) {
+                nBlocks = bTot;
+                nBits = wTot;
+            }
+        }
+        const uint32_t nWeights = (nBits + 31) / 32;
+        const uint64_t words = cnt ? (uint64_t)nBlocks + 2ull * nMacro + (nWeights + 1) / 2 + 1 : 0ull;
+        const uint64_t base = wave_alloc64(P.arena_top, words);
+        const bool ok = cnt && base + words <= P.arena_cap;
+        if (cnt && !ok) set_error(P.errors, ERR_COLOR_ARENA);
+        uint64_t* macro = P.arena + base + nBlocks;
         uint32_t* weights = reinterpret_cast<uint32_t*>(macro + 2 * nMacro);
-        uint32_t wb, wbits;
-        encode_colors<true>(P.colors + cb, P.cmarks + cb / 64, cnt, lane, buf, blocks, macro, weights, wb, wbits);
-        if (lane < 2) weights[nWeights + lane] = 0u;  // padding read by the 16-bit window
-        if (lane == 0) {
+        if (ok) {
+            if (nSeg <= kLaneSegs)
+                for (uint32_t k = 0; k < nSeg; ++k) enc_scan_marks(macro, weights, k, P.seg_out[seg0 + k]);
+            if (nBits & 31u) weights[nBits >> 5] = 0u;
+            weights[nWeights] = 0u;  // padding read by the 16-bit window
+            weights[nWeights + 1] = 0u;
             LeafDesc d;
             d.blocks = base;
             d.n_blocks = nBlocks;
@@ -2135,12 +2217,42 @@ __device__ __forceinline__ void d_encode(const EditPass& P, VGrid G) {
             d.pad = 0;
             P.leaves[T.newhandle[t] & 0x7FFFFFFFu] = d;
         }
+        for (uint64_t m = big & __ballot(ok); m; m &= m - 1) {
+            const uint32_t src = (uint32_t)__ffsll((long long)m) - 1u;
+            const uint32_t sn = __shfl(nSeg, src, 64), sm = __shfl(nMacro, src, 64);
+            const uint2* so = P.seg_out + __shfl(seg0, src, 64);  // lane k wrote entries k, k + 64, ..
+            uint64_t* bm = P.arena + shfl64(base, src) + __shfl(nBlocks, src, 64);
+            uint32_t* bw = reinterpret_cast<uint32_t*>(bm + 2 * sm);
+            for (uint32_t k = lane; k < sn; k += 64) enc_scan_marks(bm, bw, k, so[k]);
+        }
     }
-    if (P.abytes) wave_add64(P.abytes + 2, stagedBytes);
 }
-__global__ __launch_bounds__(kEncBlock) void k_encode(EditPass P) {
-    d_encode(P, VGrid{blockIdx.x, gridDim.x});
+__global__ __launch_bounds__(kEncBlock) void k_enc_scan(EditPass P) { d_enc_scan(P, VGrid{blockIdx.x, gridDim.x}); }
+
+// one wavefront per segment: its blocks and weight words
+__device__ __forceinline__ void d_enc_write(const EditPass& P, VGrid G) {
+    __shared__ uint32_t sBits[kEncWaves][kEncBuf];
+    if (*P.errors) return;
+    const uint32_t nSeg = min(*P.seg_top, P.seg_cap);
+    const Items T = P.items[P.ctl];
+    const uint32_t lane = threadIdx.x & 63u;
+    for (uint32_t sg = wave_index(G); sg < nSeg; sg += wave_count(G)) {
+        const uint32_t t = P.seg_task[sg], cnt = T.ncount[t], k = sg - T.hash[t];
+        const uint64_t cb = T.cbase[t];
+        const LeafDesc d = P.leaves[T.newhandle[t] & 0x7FFFFFFFu];
+        const uint2 at = P.seg_out[sg];
+        EncOut O;
+        O.blocks = P.arena + d.blocks;
+        O.weights = reinterpret_cast<uint32_t*>(P.arena) + d.weights32;
+        O.block0 = at.x;
+        O.bit0 = at.y;
+        O.macroBit = P.seg_out[sg - k % (16384u / kSegColors)].y;
+        O.buf = sBits[threadIdx.x >> 6];
+        uint32_t nb, nw;
+        encode_segment<true>(P.colors + cb, P.cmarks + cb / 64, cnt, k * kSegColors, lane, O, nb, nw);
+    }
 }
+__global__ __launch_bounds__(kEncBlock) void k_enc_write(EditPass P) { d_enc_write(P, VGrid{blockIdx.x, gridDim.x}); }
 
 // ---- fill editor preparation (BufferEditor / FillEditorBase, hash_dag_editors.h:144-209, 629-671) ----
 // value of every buffer voxel: DAGUtils::get_value at get_world_path (min + float(x), ...)
@@ -2266,6 +2378,7 @@ __global__ void k_init_pass(EditPass P, uint32_t root, uint32_t first, uint32_t 
         I.cmode[0] = 0;
         I.cmodeval[0] = 0;
         *P.color_top = 0;
+        *P.seg_top = 0;
     }
 }
 
@@ -2295,6 +2408,8 @@ static void scratch_free(hd_ctx* ctx) {
     hipFree(S.hset);
     hipFree(S.colors);
     hipFree(S.cmarks);
+    hipFree(S.seg_task);
+    hipFree(S.seg_out);
     for (void*& p : S.level_mem) {
         hipFree(p);
         p = nullptr;
@@ -2424,6 +2539,20 @@ hd_status edit_reserve(hd_ctx* ctx, const uint32_t* items, const uint32_t* elist
         if (err != hipSuccess) return hip_fail(ctx, err, "edit scratch (colours)");
         S.color_cap = colors;
     }
+    // the encoder's segments: one per kSegColors staged colours and one more per task
+    const uint64_t segs = encode_segments(S.color_cap, S.item_cap[std::min(ctx->g.color_tree_levels, L)]);
+    if (segs > S.seg_cap) {
+        sync_once();
+        hipFree(S.seg_task);
+        hipFree(S.seg_out);
+        S.seg_task = nullptr;
+        S.seg_out = nullptr;
+        S.seg_cap = 0;
+        hipError_t err = segs > 0xFFFFFFFFull ? hipErrorOutOfMemory : hipMalloc(&S.seg_task, segs * 4);
+        if (err == hipSuccess) err = hipMalloc(&S.seg_out, segs * 8);
+        if (err != hipSuccess) return hip_fail(ctx, err, "edit scratch (segments)");
+        S.seg_cap = (uint32_t)segs;
+    }
     return HD_OK;
 }
 
@@ -2511,7 +2640,7 @@ namespace {
 // steps, and the commit. Every launch form runs this sequence.
 enum PassStep : uint32_t {
     ST_EXPAND, ST_LEAF, ST_BUILD, ST_HCLEAR, ST_DEDUP, ST_FIND, ST_ADD, ST_RESOLVE, ST_CSTARTS, ST_CALLOC,
-    ST_CTREE, ST_CCOPY, ST_CCOPY_LEAVES, ST_CLEAF, ST_ENCODE, ST_FINISH
+    ST_CTREE, ST_CCOPY, ST_CCOPY_LEAVES, ST_CLEAF, ST_ENC_COUNT, ST_ENC_SCAN, ST_ENC_WRITE, ST_FINISH
 };
 constexpr uint32_t kMaxSteps = 8 * kMaxEditLevels + 8;
 struct StepList {
@@ -2539,7 +2668,9 @@ static StepList pass_step_list(uint32_t levels, uint32_t ctl, bool colors) {
         add(ST_CTREE, ctl);
         for (uint32_t l = ctl; l < L; ++l) add(l + 1 == L ? ST_CCOPY_LEAVES : ST_CCOPY, l);
         add(ST_CLEAF, L);
-        add(ST_ENCODE, ctl);
+        add(ST_ENC_COUNT, ctl);
+        add(ST_ENC_SCAN, ctl);
+        add(ST_ENC_WRITE, ctl);
     }
     add(ST_FINISH, 0);
     return sl;
@@ -2569,7 +2700,9 @@ __device__ __forceinline__ void run_step(const EditPass& P, uint32_t code, uint3
             if constexpr (kSpecial) d_color_leaf(P, G);
             else d_color_leaf_items(P, G);
             break;
-        case ST_ENCODE: d_encode(P, G); break;
+        case ST_ENC_COUNT: d_enc_count(P, G); break;
+        case ST_ENC_SCAN: d_enc_scan(P, G); break;
+        case ST_ENC_WRITE: d_enc_write(P, G); break;
         default: d_finish(P, root_out, G); break;
     }
 }
@@ -2654,6 +2787,10 @@ static void fill_pass(hd_ctx* ctx, EditPass& P, const EditScratch& S) {
     P.colors = S.colors;
     P.cmarks = S.cmarks;
     P.color_cap = S.color_cap;
+    P.seg_task = S.seg_task;
+    P.seg_out = S.seg_out;
+    P.seg_cap = S.seg_cap;
+    P.seg_top = reinterpret_cast<uint32_t*>(S.dstats + 5);
     P.cnodes = ctx->cnodes;
     P.cnodes_cap = ctx->cfg.color_nodes_cap;
     P.offsets = ctx->coffsets;
@@ -2745,8 +2882,11 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
     const auto wideGrid = [](uint64_t blocks) {
         return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(blocks, 1u), 1u << 16);
     };
-    const uint32_t encBlocks =
-        (uint32_t)std::min<uint64_t>(std::max<uint64_t>((bound[P.ctl] + kEncWaves - 1) / kEncWaves, 1u), 1u << 16);
+    // encoder: a wavefront per segment of the staged colours. Their number is on the device (at
+    // most what the tasks can hold): twice the wavefronts the chip keeps resident, then a stride
+    const uint64_t maxSegs = bound[P.ctl] * (((1ull << (3 * (D - P.ctl))) + kSegColors - 1) / kSegColors);
+    const uint32_t segBlocks =
+        (uint32_t)std::min<uint64_t>(std::max<uint64_t>((maxSegs + kEncWaves - 1) / kEncWaves, 1u), 4096u);
     for (uint32_t i = 0; i < sl.n;) {
         if (small(sl.step[i])) {
             uint32_t j = i + 1;
@@ -2791,7 +2931,9 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
                 if (special) k_color_leaf<<<gl, 256, 0, s>>>(P);
                 else k_color_leaf_items<<<units(b, 256), 256, 0, s>>>(P);
                 break;
-            case ST_ENCODE: k_encode<<<encBlocks, kEncBlock, 0, s>>>(P); break;
+            case ST_ENC_COUNT: k_enc_count<<<segBlocks, kEncBlock, 0, s>>>(P); break;
+            case ST_ENC_SCAN: k_enc_scan<<<units(b, 256), kEncBlock, 0, s>>>(P); break;  // a thread per task
+            case ST_ENC_WRITE: k_enc_write<<<segBlocks, kEncBlock, 0, s>>>(P); break;
             default: k_finish<<<1, 64, 0, s>>>(P, ctx->d_root); break;
         }
         ++i;

@@ -701,6 +701,9 @@ uint64_t static_layout(EditScratch& S, uint32_t levels, char* base) {
     S.colors = reinterpret_cast<uint64_t*>(take(kStaticColors * 8));
     S.cmarks = reinterpret_cast<uint64_t*>(take(kStaticColors / 64 * 8));
     S.color_cap = kStaticColors;
+    S.seg_cap = (uint32_t)encode_segments(kStaticColors, kStaticItems);
+    S.seg_task = reinterpret_cast<uint32_t*>(take((uint64_t)S.seg_cap * 4));
+    S.seg_out = reinterpret_cast<uint2*>(take((uint64_t)S.seg_cap * 8));
     const uint32_t L = levels - 2;
     for (uint32_t l = 0; l <= L; ++l) {
         const uint64_t c = l < 4 ? std::min<uint64_t>(1ull << (3 * l), kStaticItems) : kStaticItems;

@@ -1,0 +1,25 @@
+"""The segmented colour encoder at the sizes where it changes path: colour arrays that end at,
+just before and just after a segment (4096 colours) and arrays of more segments than a lane
+walks on its own (8). Checked against the oracle, word by word."""
+import pytest
+
+from tests.test_edit_gpu import BOX_ADD, SPHERE_PAINT, assert_same, make
+
+pytestmark = pytest.mark.gpu
+
+
+# a box of integer centre and radius r holds (2 r)^3 voxels: 4096 at r = 8, 32768 (8 segments) at 16
+@pytest.mark.parametrize("r", [7.5, 8.0, 8.5, 16.0, 16.5, 25.0])
+@pytest.mark.parametrize("where", ["air", "ground"])
+def test_segment_edges_match_oracle(r, where):
+    from hashdag_amd import terrain_height
+    p, sc, g, dag, od, oc = make("d10w")
+    shift = 0.5 if r != int(r) else 0.0  # whole voxels either way
+    x, z = 192.0, 192.0  # inside one 128^3 colour subtree
+    y = 960.0 if where == "air" else float(terrain_height(p, 192, 192))
+    c = (x + shift, y + shift, z + shift)
+    edits = [(BOX_ADD, c, r), (SPHERE_PAINT, (x + r, y + r, z + r), r)]  # one colour, then a corner of many
+    st = dag.edit_batch(edits, fused=True)
+    total = sum(od.edit(kind, cc, rr, oc)[1] for kind, cc, rr in edits)
+    assert st.num_voxels == total
+    assert_same(dag, sc, od, oc, f"box of radius {r} in the {where}")
