@@ -1,9 +1,11 @@
-"""The segmented colour encoder at the sizes where it changes path: colour arrays that end at,
-just before and just after a segment (4096 colours) and arrays of more segments than a lane
-walks on its own (8). Checked against the oracle, word by word."""
+"""The segmented colour encoder and the edited-voxel count at the sizes where they change path:
+colour arrays that end at, just before and just after a segment (4096 colours), arrays of more
+segments than a lane walks on its own (8), and editors that leave the scene or fall between
+voxels. Checked against the oracle, word by word."""
+import numpy as np
 import pytest
 
-from tests.test_edit_gpu import BOX_ADD, SPHERE_PAINT, assert_same, make
+from tests.test_edit_gpu import BOX_ADD, BOX_CARVE, SPHERE_ADD, SPHERE_CARVE, SPHERE_PAINT, assert_same, make
 
 pytestmark = pytest.mark.gpu
 
@@ -23,3 +25,20 @@ def test_segment_edges_match_oracle(r, where):
     total = sum(od.edit(kind, cc, rr, oc)[1] for kind, cc, rr in edits)
     assert st.num_voxels == total
     assert_same(dag, sc, od, oc, f"box of radius {r} in the {where}")
+
+
+@pytest.mark.parametrize("seed", range(3))
+def test_voxel_counts_of_odd_editors(seed):
+    p, sc, g, dag, od, oc = make("d8")
+    rng = np.random.default_rng(seed)
+    edits = []
+    for kind in (SPHERE_ADD, SPHERE_CARVE, SPHERE_PAINT, BOX_ADD, BOX_CARVE):
+        for r in (0.25, 0.5, 1.0, 1.7, 19.3, 40.0):
+            c = rng.uniform(-8.0, 264.0, size=3)  # past the scene's ends too
+            if r in (0.5, 40.0):
+                c = np.round(c)
+            edits.append((kind, tuple(float(np.float32(v)) for v in c), r))
+    edits.append((SPHERE_ADD, (300.0, 128.0, 128.0), 20.0))  # touches nothing
+    st = dag.edit_batch(edits, fused=True)
+    assert st.num_voxels == sum(od.edit(kind, c, r, oc)[1] for kind, c, r in edits)
+    assert_same(dag, sc, od, oc, "odd editors")
