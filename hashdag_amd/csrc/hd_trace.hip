@@ -6,7 +6,7 @@
 // Mapping: one lane per pixel; a 64-lane wavefront covers a tile_w x tile_h pixel tile
 // (8 x 8 by default) so neighbouring rays share their upper-level nodes; a 256-thread block
 // holds 2 x 2 wave tiles. The DFS stack (node index, child mask, visit mask per level) lives
-// in LDS, laid out [level][thread] so a wavefront's accesses are bank-conflict free. Node
+// in LDS, laid out [height][thread] so a wavefront's accesses are bank-conflict free. Node
 // words are read straight from the virtual-address pool (no page-table indirection).
 #include <hip/hip_runtime.h>
 
@@ -32,17 +32,15 @@ __device__ __forceinline__ uint32_t child_off(uint32_t mask, uint32_t child) {
     return __popc(mask & ((1u << child) - 1u)) + 1u;
 }
 
-// base_dag.h:16-58: bit i of the mask = byte i of the leaf is non-zero (the bytes' bits are
-// folded onto their bit 0, then the four bit-0s of each word gathered)
-__device__ __forceinline__ uint32_t byte_nonzero4(uint32_t w) {
-    w |= w >> 4;
-    w |= w >> 2;
-    w |= w >> 1;
-    w &= 0x01010101u;
-    return (w | (w >> 7) | (w >> 14) | (w >> 21)) & 0xFu;
+// base_dag.h:16-58: bit i of the mask = byte i of the leaf is non-zero. A byte's top bit is set
+// where adding 0x7F to its low bits carries or it was set before; a dot product with the weights
+// 1, 2, 4 .. 128 gathers the eight top bits.
+__device__ __forceinline__ uint32_t byte_top_bits(uint32_t w) {
+    return (((w & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | w) & 0x80808080u;
 }
 __device__ __forceinline__ uint32_t leaf_first_mask(uint64_t leaf) {
-    return byte_nonzero4((uint32_t)leaf) | (byte_nonzero4((uint32_t)(leaf >> 32)) << 4);
+    const uint32_t lo = __builtin_amdgcn_udot4(byte_top_bits((uint32_t)leaf), 0x08040201u, 0u, false);
+    return __builtin_amdgcn_udot4(byte_top_bits((uint32_t)(leaf >> 32)), 0x80402010u, lo, false) >> 7;
 }
 __device__ __forceinline__ uint32_t leaf_second_mask(uint64_t leaf, uint32_t c) {
     const uint32_t w = (c & 4) ? (uint32_t)(leaf >> 32) : (uint32_t)leaf;
@@ -58,10 +56,6 @@ __device__ __forceinline__ uint32_t permute_order(uint32_t order, uint32_t mask)
     if (order & 1) m = ((m & 0x55u) << 1) | ((m & 0xAAu) >> 1);
     return m;
 }
-__device__ __forceinline__ uint32_t next_child(uint32_t order, uint32_t mask) {
-    return (uint32_t)__builtin_ctz(permute_order(order, mask)) ^ order;
-}
-
 __device__ __forceinline__ float tmax3(float x, float y, float z) {
     const float m = y > z ? y : z;
     return x > m ? x : m;
@@ -126,6 +120,7 @@ __device__ __forceinline__ uint32_t intersection_mask(uint32_t levels, uint32_t 
 //                  node is safe
 constexpr int kFetchPointer = 0, kFetchNode = 1;
 
+typedef uint32_t u32x2_a4 __attribute__((ext_vector_type(2), aligned(4)));
 typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
 
 __device__ __forceinline__ void load_node(const uint32_t* __restrict__ vpool, uint32_t index, uint32_t nd[9]) {
@@ -154,40 +149,161 @@ __device__ __forceinline__ uint32_t pick(const uint32_t nd[9], uint32_t k) {
     return k <= 4u ? ab : cd;
 }
 
-// LDS stack of one block: node index per level 1 .. leafLevel-1 (level 0 is the root; at the
-// two leaf levels the 64-bit leaf stays in registers), then (child mask | visit << 8) per level.
+// The walk keeps a node's height s = levels - level (a child's side is 2^(s-1) voxels; s = 2 at
+// the leaves, 0 at a voxel) and its lowest voxel (x, y, z). Child masks to visit are kept in the
+// ray's order: bit k stands for child k ^ order, so the next child is the lowest set bit. The
+// intersection mask is built in that order from per-ray constants (Halves); a node's child mask
+// is brought into it by a table in LDS.
+//
+// kAxis0: order is 0 for every ray (the sun's direction is positive on all axes).
+// kTame: every ray of the wavefront has |1/d| and |origin| at most 2^40, so no term of the
+// intersection mask is infinite or NaN and three-way minima and maxima may be taken in any order.
+struct Halves {
+    uint32_t xu, xl, yu, yl, zu, zl;  // children in the upper / lower half of each axis
+};
+template <bool kAxis0>
+__device__ __forceinline__ Halves halves_of(uint32_t order) {
+    if (kAxis0) return Halves{0xF0u, 0x0Fu, 0xCCu, 0x33u, 0xAAu, 0x55u};
+    const uint32_t x = (order & 4) ? 0x0Fu : 0xF0u, y = (order & 2) ? 0x33u : 0xCCu, z = (order & 1) ? 0x55u : 0xAAu;
+    return Halves{x, x ^ 0xFFu, y, y ^ 0xFFu, z, z ^ 0xFFu};
+}
+
+__device__ __forceinline__ bool tame_ray(F3 o, F3 inv) {
+    const float m = 1099511627776.0f;  // 2^40; false for NaN
+    return fabsf(o.x) <= m && fabsf(o.y) <= m && fabsf(o.z) <= m && fabsf(inv.x) <= m && fabsf(inv.y) <= m &&
+           fabsf(inv.z) <= m;
+}
+
+// intersection_mask of the node at height s with lowest voxel (x, y, z), in the ray's order: the
+// same IEEE operations (the centre is an integer below 2^24, so converting it is exact), in two
+// parts between which the walk issues a load: the slab terms, then the children.
+struct Slab {
+    float rx, ry, rz, tx, ty, tz, tmin, tmax;
+};
+template <bool kTame>
+__device__ __forceinline__ Slab walk_slab(uint32_t s, uint32_t x, uint32_t y, uint32_t z, F3 o, F3 inv) {
+    const uint32_t half = 1u << (s - 1);
+    const float radius = (float)half;
+    Slab b;
+    b.rx = (float)(x | half) - o.x;
+    b.ry = (float)(y | half) - o.y;
+    b.rz = (float)(z | half) - o.z;
+    b.tx = b.rx * inv.x;
+    b.ty = b.ry * inv.y;
+    b.tz = b.rz * inv.z;
+    const float sx = radius * fabsf(inv.x), sy = radius * fabsf(inv.y), sz = radius * fabsf(inv.z);
+    if (kTame) {
+        b.tmin = fmaxf(fmaxf(fmaxf(b.tx - sx, b.ty - sy), b.tz - sz), 0.0f);
+        b.tmax = fminf(fminf(b.tx + sx, b.ty + sy), b.tz + sz);
+    } else {
+        b.tmin = fmaxf(tmax3(b.tx - sx, b.ty - sy, b.tz - sz), 0.0f);
+        b.tmax = tmin3(b.tx + sx, b.ty + sy, b.tz + sz);
+    }
+    return b;
+}
+template <bool kTame>
+__device__ __forceinline__ uint32_t slab_children(const Slab& b, F3 d, const Halves& hv) {
+    const float eps = 1e-4f;
+    const float xm = b.rx - eps, xp = b.rx + eps, ym = b.ry - eps, yp = b.ry + eps, zm = b.rz - eps, zp = b.rz + eps;
+    const float xqy = b.tx * d.y, xqz = b.tx * d.z, yqx = b.ty * d.x, yqz = b.ty * d.z, zqx = b.tz * d.x, zqy = b.tz * d.y;
+    const bool inx = b.tmin <= b.tx && b.tx <= b.tmax, iny = b.tmin <= b.ty && b.ty <= b.tmax,
+               inz = b.tmin <= b.tz && b.tz <= b.tmax;
+    // the children on the upper / lower side within eps; a finite q is on one of the two
+    const auto side = [](float q, float m, float p, uint32_t up, uint32_t low) {
+        if (kTame) return q >= m ? (q <= p ? 0xFFu : up) : low;
+        return (q >= m ? up : 0u) | (q <= p ? low : 0u);
+    };
+    // the child at the middle of the slab's span: (0.5 (tmin + tmax)) d, the half moved to d (exact)
+    const float h = b.tmin + b.tmax;
+    uint32_t mask = (h * (0.5f * d.x) >= b.rx ? hv.xu : hv.xl) & (h * (0.5f * d.y) >= b.ry ? hv.yu : hv.yl) &
+                    (h * (0.5f * d.z) >= b.rz ? hv.zu : hv.zl);
+    if (!kTame) {
+        const float hh = 0.5f * (b.tmin + b.tmax);
+        mask = (hh * d.x >= b.rx ? hv.xu : hv.xl) & (hh * d.y >= b.ry ? hv.yu : hv.yl) &
+               (hh * d.z >= b.rz ? hv.zu : hv.zl);
+    }
+    // the three face terms are evaluated unconditionally and kept by predicate, as above
+    mask |= (inx ? side(xqy, ym, yp, hv.yu, hv.yl) : 0u) & side(xqz, zm, zp, hv.zu, hv.zl);
+    mask |= (iny ? side(yqx, xm, xp, hv.xu, hv.xl) : 0u) & side(yqz, zm, zp, hv.zu, hv.zl);
+    mask |= (inz ? side(zqx, xm, xp, hv.xu, hv.xl) : 0u) & side(zqy, ym, yp, hv.yu, hv.yl);
+    return mask;
+}
+// keeps a value's computation where it stands (before the waits for the loads in flight)
+__device__ __forceinline__ void pin(uint32_t& v) { asm volatile("" : "+v"(v)); }
+__device__ __forceinline__ void pin(float& v) { asm volatile("" : "+v"(v)); }
+
+// LDS of one block: per height 3 .. levels the node's index (the two leaf heights keep the 64-bit
+// leaf in registers), per height 1 .. levels (child mask | children left << 8), and the child
+// masks' order table (order * 256 + mask).
 struct Stack {
     uint32_t* idx;
     uint16_t* mask;
-    __device__ __forceinline__ uint32_t& at_idx(uint32_t level) { return idx[(level - 1) * kBlock + threadIdx.x]; }
-    __device__ __forceinline__ uint16_t& at_mask(uint32_t level) { return mask[level * kBlock + threadIdx.x]; }
+    uint8_t* perm;
+    __device__ __forceinline__ uint32_t& at_idx(uint32_t s) { return idx[(max(s, 3u) - 3u) * kBlock + threadIdx.x]; }
+    __device__ __forceinline__ uint16_t& at_mask(uint32_t s) { return mask[(s - 1u) * kBlock + threadIdx.x]; }
 };
 
+constexpr uint32_t kPermBytes = 8 * 256;
 __host__ __device__ __forceinline__ uint32_t stack_bytes(uint32_t levels) {
-    return ((levels - 3) * 4u + levels * 2u) * kBlock;
+    return ((levels - 2u) * 4u + levels * 2u) * kBlock + kPermBytes;
 }
 
+// Every thread of the block calls it (the order table is filled, then a block barrier).
+template <bool kAxis0>
 __device__ __forceinline__ Stack stack_of(uint32_t levels) {
     extern __shared__ uint32_t sStack[];
     Stack st;
     st.idx = sStack;
-    st.mask = reinterpret_cast<uint16_t*>(sStack + (levels - 3) * kBlock);
+    st.mask = reinterpret_cast<uint16_t*>(sStack + (levels - 2) * kBlock);
+    st.perm = reinterpret_cast<uint8_t*>(st.mask + levels * kBlock);
+    if (!kAxis0) {
+        for (uint32_t k = threadIdx.x; k < kPermBytes / 4; k += blockDim.x) {
+            uint32_t w = 0;
+            for (uint32_t q = 0; q < 4; ++q) w |= permute_order(k >> 6, (k * 4u + q) & 0xFFu) << (8u * q);
+            reinterpret_cast<uint32_t*>(st.perm)[k] = w;
+        }
+        __syncthreads();
+    }
     return st;
 }
 
-// DFS state of one ray: the current node, its child mask and the children left to visit,
-// the voxel path, and (bit l of alive) which stack levels still hold children to visit.
+// DFS state of one ray: the current node, its child mask, the children left to visit (in the
+// ray's order), its lowest voxel, and (bit s of alive) which heights still hold children to visit.
 struct Walk {
-    uint32_t level, px, py, pz, index, childMask, visit, alive;
+    uint32_t s, px, py, pz, index, childMask, visit, alive;
     uint64_t leaf;
     uint32_t nd[9];  // the current node's words (kFetchNode)
 };
 
+// What a walk needs of its ray.
+struct Ray {
+    F3 o, d, inv;
+    uint32_t order;
+    Halves hv;
+};
+template <bool kAxis0>
+__device__ __forceinline__ Ray make_ray(F3 o, F3 d, F3 inv, uint32_t order) {
+    return Ray{o, d, inv, kAxis0 ? 0u : order, halves_of<kAxis0>(order)};
+}
+
 constexpr uint32_t kWalkOn = 0, kWalkHit = 1, kWalkMiss = 2;
 
-template <bool kCount, int kFetch>
-__device__ __forceinline__ void walk_begin(const DevDag& dag, Walk& w, F3 o, F3 d, F3 inv, uint64_t& bytes) {
-    w.level = 0;
+template <bool kAxis0>
+__device__ __forceinline__ uint32_t in_order(const Stack& st, uint32_t order, uint32_t mask) {
+    return kAxis0 ? mask : (uint32_t)st.perm[order * 256u + mask];
+}
+
+// A walk without anything left: nothing was hit.
+constexpr uint32_t kNothingLeft = 1u;  // in `alive`: height 0 is never on the stack
+__device__ __forceinline__ void walk_miss(Walk& w) {
+    w.px = w.py = w.pz = 0;
+    w.alive = kNothingLeft;
+    w.s = 0;
+}
+
+template <bool kCount, int kFetch, bool kAxis0>
+__device__ __forceinline__ void walk_begin(const DevDag& dag, Walk& w, const Ray& r, Stack st, uint64_t& bytes) {
+    w.s = dag.levels;
     w.px = w.py = w.pz = 0;
     w.index = dag.root;
     w.leaf = 0;
@@ -199,112 +315,108 @@ __device__ __forceinline__ void walk_begin(const DevDag& dag, Walk& w, F3 o, F3 
         w.childMask = dag.vpool[w.index] & 0xFFu;
     }
     if (kCount) bytes += 4;
-    w.visit = w.childMask & intersection_mask<true>(dag.levels, 0, 0, 0, 0, o, d, inv);
+    w.visit = in_order<kAxis0>(st, r.order,
+                               w.childMask & intersection_mask<true>(dag.levels, 0, 0, 0, 0, r.o, r.d, r.inv));
+    if (!w.visit) walk_miss(w);
 }
 
 // One step of the DFS over the DAG (tracer.cu:166-249 ordered first hit; tracer.cu:458-542
-// any hit): back up if the current node has nothing left to visit, then descend into the
-// next child. Returns kWalkHit with the voxel path in (px, py, pz), kWalkMiss with (0, 0, 0),
-// or kWalkOn.
-template <bool kCount, int kFetch>
-__device__ __forceinline__ uint32_t walk_step(const DevDag& dag, Walk& w, F3 o, F3 d, F3 inv, uint32_t order, Stack st,
-                                              uint64_t& bytes) {
+// any hit): descend into the next child, then, if it has nothing to visit, back up to the lowest
+// height with children left. The walk has ended when w.s is 0: at a voxel, its path in (px, py,
+// pz), or with kNothingLeft in w.alive and (0, 0, 0).
+//
+// Bound by VALU issue (SQ_ACTIVE_INST_VALU fills the launch's SIMD cycles at 1080p) and, where few
+// wavefronts are in flight, by the latency of a step. Loads go through one straight path for
+// every lane (lanes inside a leaf read some word of their parent), so the child's pointer and
+// then its words are in flight while the child's intersection mask, which needs neither, is
+// computed; a node's own load per step, and the masks kept in the ray's order, take about 120
+// instructions a step where a load per branch and a permutation per child took about 175.
+// 1920x1080 over a 2^15 terrain 16384 wide, capped at 128 steps: paths 0.42 -> 0.28 ms, shadows
+// 0.59 -> 0.39 ms; 640x360 uncapped: 0.21 -> 0.08 and 0.22 -> 0.16 ms.
+template <bool kCount, int kFetch, bool kAxis0, bool kTame>
+__device__ __forceinline__ void walk_step(const DevDag& dag, Walk& w, const Ray& r, Stack st, uint64_t& bytes) {
     const uint32_t* __restrict__ vpool = dag.vpool;
-    const uint32_t levels = dag.levels, leafLevel = dag.leaf_level;
-    if (!w.visit) {
-        // back up to the deepest level with children left (the DFS backtrack)
-        const uint32_t below = w.alive & ((1u << w.level) - 1u);
-        if (!below) {
-            w.px = w.py = w.pz = 0;
-            return kWalkMiss;
-        }
-        const uint32_t newLevel = 31u - (uint32_t)__builtin_clz(below);
-        const uint32_t m = st.at_mask(newLevel);
-        w.childMask = m & 0xFFu;
-        w.visit = m >> 8;
-        const uint32_t up = w.level - newLevel;
-        w.px >>= up;
-        w.py >>= up;
-        w.pz >>= up;
-        w.level = newLevel;
-        if (w.level < leafLevel) {
-            w.index = w.level == 0 ? dag.root : st.at_idx(w.level);
-            if (kFetch == kFetchNode) load_node(vpool, w.index, w.nd);
-        }
-    }
     // children front to back along the ray, also for the any-hit walk: its result does not
     // depend on the order (tracer.cu:493 takes the highest bit first), and front to back
     // reaches the nearest occluder of a shadowed ray first
-    const uint32_t next = next_child(order, w.visit);
-    w.visit &= ~(1u << next);
-    w.px = (w.px << 1) | ((next >> 2) & 1u);
-    w.py = (w.py << 1) | ((next >> 1) & 1u);
-    w.pz = (w.pz << 1) | (next & 1u);
-    // only entries with children left are ever read back
-    if (w.visit) {
-        if (w.level > 0 && w.level < leafLevel) st.at_idx(w.level) = w.index;
-        st.at_mask(w.level) = (uint16_t)(w.childMask | (w.visit << 8));
-        w.alive |= 1u << w.level;
+    const uint32_t next = (uint32_t)__builtin_ctz(w.visit) ^ r.order;
+    w.visit &= w.visit - 1u;
+    // written whether or not children are left: only heights in `alive` are read back
+    st.at_idx(w.s) = w.index;
+    st.at_mask(w.s) = (uint16_t)(w.childMask | (w.visit << 8));
+    w.alive = (w.alive & ~(1u << w.s)) | (w.visit ? 1u << w.s : 0u);
+    const bool inner = w.s > 2;  // the child is a node or a leaf of its own
+    w.s--;
+    w.px |= ((next >> 2) & 1u) << w.s;
+    w.py |= ((next >> 1) & 1u) << w.s;
+    w.pz |= (next & 1u) << w.s;
+    if (w.s == 0) return;
+    uint32_t addr, w0, w1, im;
+    if (kFetch == kFetchNode) {
+        addr = inner ? pick(w.nd, child_off(w.childMask, next)) : w.index;
+        if (w.s > 2) load_node(vpool, addr, w.nd);
+        w0 = w.s > 2 ? w.nd[0] : vpool[addr];
+        w1 = vpool[addr + 1];
+        im = slab_children<kTame>(walk_slab<kTame>(w.s, w.px, w.py, w.pz, r.o, r.inv), r.d, r.hv);
     } else {
-        w.alive &= ~(1u << w.level);
+        addr = vpool[w.index + child_off(w.childMask, next)];  // inside a leaf: some word of its parent
+        Slab b = walk_slab<kTame>(w.s, w.px, w.py, w.pz, r.o, r.inv);
+        pin(b.tmin);
+        pin(b.tmax);
+        addr = inner ? addr : w.index;
+        const u32x2_a4 v = *reinterpret_cast<const u32x2_a4*>(vpool + addr);
+        im = slab_children<kTame>(b, r.d, r.hv);
+        pin(im);
+        w0 = v.x;
+        w1 = v.y;
     }
-    w.level++;
-    if (w.level == levels) return kWalkHit;
-    if (w.level < leafLevel) {
-        if (kFetch == kFetchNode) {
-            w.index = pick(w.nd, child_off(w.childMask, next));
-            load_node(vpool, w.index, w.nd);
-            w.childMask = w.nd[0] & 0xFFu;
+    uint32_t cm = w0 & 0xFFu;
+    if (w.s <= 2) {
+        if (w.s == 2) w.leaf = (uint64_t)w0 | ((uint64_t)w1 << 32);
+        cm = w.s == 2 ? leaf_first_mask(w.leaf) : leaf_second_mask(w.leaf, next);
+        addr = w.index;  // a leaf keeps its parent's index
+    }
+    w.index = addr;
+    if (kCount) bytes += w.s > 2 ? 8 : (w.s == 2 ? 12 : 0);
+    w.childMask = cm;
+    w.visit = in_order<kAxis0>(st, r.order, cm) & im;
+    if (!w.visit) {
+        if (!w.alive) {
+            walk_miss(w);
         } else {
-            w.index = vpool[w.index + child_off(w.childMask, next)];
-            w.childMask = vpool[w.index] & 0xFFu;
+            w.s = (uint32_t)__builtin_ctz(w.alive);
+            const uint32_t m = st.at_mask(w.s);
+            w.index = st.at_idx(w.s);  // inside a leaf: the leaf's parent, as it is
+            w.childMask = m & 0xFFu;
+            w.visit = m >> 8;
+            const uint32_t keep = ~0u << w.s;
+            w.px &= keep;
+            w.py &= keep;
+            w.pz &= keep;
+            if (kFetch == kFetchNode && w.s > 2) load_node(vpool, w.index, w.nd);
         }
-        if (kCount) bytes += 8;
-    } else if (w.level == leafLevel) {
-        const uint32_t addr = kFetch == kFetchNode ? pick(w.nd, child_off(w.childMask, next))
-                                                   : vpool[w.index + child_off(w.childMask, next)];
-        w.leaf = *reinterpret_cast<const uint64_t*>(vpool + addr);
-        w.childMask = leaf_first_mask(w.leaf);
-        if (kCount) bytes += 12;
-    } else {
-        w.childMask = leaf_second_mask(w.leaf, next);
     }
-    w.visit = w.childMask & intersection_mask<false>(levels, w.level, w.px, w.py, w.pz, o, d, inv);
-    return kWalkOn;
+}
+__device__ __forceinline__ uint32_t walk_result(const Walk& w) {
+    return w.s != 0 ? kWalkOn : (w.alive == kNothingLeft ? kWalkMiss : kWalkHit);
 }
 
-// The whole walk of one ray. Returns true on a hit; (px, py, pz) is the voxel path on a hit,
-// (0,0,0) on a miss.
-template <bool kCount, int kFetch>
-__device__ __forceinline__ bool descend(const DevDag& dag, F3 o, F3 d, F3 inv, uint32_t order, uint32_t& px,
-                                        uint32_t& py, uint32_t& pz, Stack st, uint64_t& bytes) {
-    Walk w;
-    walk_begin<kCount, kFetch>(dag, w, o, d, inv, bytes);
-    uint32_t r;
-    do {
-        r = walk_step<kCount, kFetch>(dag, w, o, d, inv, order, st, bytes);
-    } while (r == kWalkOn);
-    px = w.px;
-    py = w.py;
-    pz = w.pz;
-    return r == kWalkHit;
+// The walk of one ray for at most `cap` steps (~0u: to its end): kWalkHit with the voxel path in
+// w.px, w.py, w.pz, kWalkMiss with (0, 0, 0), kWalkOn when it was stopped at the cap (the ray is
+// then traced by the wavefront-per-ray search).
+template <bool kCount, int kFetch, bool kAxis0, bool kTame>
+__device__ __forceinline__ uint32_t walk_run(const DevDag& dag, Walk& w, const Ray& ray, Stack st, uint32_t cap,
+                                             uint64_t& bytes) {
+    for (uint32_t steps = 0; w.s != 0 && steps < cap; ++steps)
+        walk_step<kCount, kFetch, kAxis0, kTame>(dag, w, ray, st, bytes);
+    return walk_result(w);
 }
-
-// descend() for at most `cap` steps: kWalkHit / kWalkMiss as descend, kWalkOn when the walk
-// was stopped at the cap (the ray is then traced by the wavefront-per-ray search).
-template <int kFetch>
-__device__ __forceinline__ uint32_t descend_capped(const DevDag& dag, F3 o, F3 d, F3 inv, uint32_t order, uint32_t& px,
-                                                   uint32_t& py, uint32_t& pz, Stack st, uint32_t cap, Walk& w) {
-    uint64_t unused = 0;
-    walk_begin<false, kFetch>(dag, w, o, d, inv, unused);
-    uint32_t r, steps = 0;
-    do {
-        r = walk_step<false, kFetch>(dag, w, o, d, inv, order, st, unused);
-    } while (r == kWalkOn && ++steps < cap);
-    px = w.px;
-    py = w.py;
-    pz = w.pz;
-    return r;
+template <bool kCount, int kFetch, bool kAxis0>
+__device__ __forceinline__ uint32_t descend(const DevDag& dag, const Ray& ray, Stack st, uint32_t cap, Walk& w,
+                                            uint64_t& bytes) {
+    walk_begin<kCount, kFetch, kAxis0>(dag, w, ray, st, bytes);
+    if (!__ballot(!tame_ray(ray.o, ray.inv))) return walk_run<kCount, kFetch, kAxis0, true>(dag, w, ray, st, cap, bytes);
+    return walk_run<kCount, kFetch, kAxis0, false>(dag, w, ray, st, cap, bytes);
 }
 
 // Rays whose walk stopped at the cap: appended as pixel indices, one atomic per wavefront.
@@ -331,14 +443,15 @@ __device__ __forceinline__ void long_append(bool give, uint32_t pix, const LongR
 }
 
 // A walk stopped at the cap, saved so another launch continues it (pointer fetch): the walk's
-// registers, then the LDS stack's node indices (levels 1 .. leafLevel - 1) and child masks
-// (two levels per word). Only levels below the walk's level with children left are read back.
+// registers, then the LDS stack's node indices (heights 3 .. levels - 1; the top one is the root)
+// and child masks (two heights per word). Only heights above the walk's own with children left
+// are read back.
 constexpr uint32_t kWalkWords = 10;
 constexpr uint32_t kStateWords = kWalkWords + (kMaxLevels - 3) + (kMaxLevels + 1) / 2;
-__device__ __forceinline__ void save_walk(const Walk& w, Stack st, uint32_t levels, uint32_t leafLevel,
-                                          uint32_t* __restrict__ state, uint32_t stride, uint32_t slot) {
+__device__ __forceinline__ void save_walk(const Walk& w, Stack st, uint32_t levels, uint32_t* __restrict__ state,
+                                          uint32_t stride, uint32_t slot) {
     uint32_t* q = state + slot;
-    q[0 * (uint64_t)stride] = w.level;
+    q[0 * (uint64_t)stride] = w.s;
     q[1 * (uint64_t)stride] = w.px;
     q[2 * (uint64_t)stride] = w.py;
     q[3 * (uint64_t)stride] = w.pz;
@@ -348,17 +461,17 @@ __device__ __forceinline__ void save_walk(const Walk& w, Stack st, uint32_t leve
     q[7 * (uint64_t)stride] = w.alive;
     q[8 * (uint64_t)stride] = (uint32_t)w.leaf;
     q[9 * (uint64_t)stride] = (uint32_t)(w.leaf >> 32);
-    for (uint32_t l = 1; l < leafLevel && l < w.level; ++l) q[(uint64_t)(kWalkWords + l - 1) * stride] = st.at_idx(l);
+    for (uint32_t h = 3; h < levels; ++h) q[(uint64_t)(kWalkWords + h - 3) * stride] = st.at_idx(h);
     const uint32_t m0 = kWalkWords + (kMaxLevels - 3);
-    for (uint32_t l = 0; l < levels && l < w.level; l += 2) {
-        const uint32_t hi = l + 1 < levels ? st.at_mask(l + 1) : 0u;
-        q[(uint64_t)(m0 + l / 2) * stride] = st.at_mask(l) | (hi << 16);
+    for (uint32_t h = 1; h <= levels; h += 2) {
+        const uint32_t hi = h + 1 <= levels ? st.at_mask(h + 1) : 0u;
+        q[(uint64_t)(m0 + h / 2) * stride] = st.at_mask(h) | (hi << 16);
     }
 }
-__device__ __forceinline__ void restore_walk(Walk& w, Stack st, uint32_t levels, uint32_t leafLevel,
+__device__ __forceinline__ void restore_walk(Walk& w, Stack st, uint32_t levels, uint32_t root,
                                              const uint32_t* __restrict__ state, uint32_t stride, uint32_t slot) {
     const uint32_t* q = state + slot;
-    w.level = q[0 * (uint64_t)stride];
+    w.s = q[0 * (uint64_t)stride];
     w.px = q[1 * (uint64_t)stride];
     w.py = q[2 * (uint64_t)stride];
     w.pz = q[3 * (uint64_t)stride];
@@ -367,12 +480,13 @@ __device__ __forceinline__ void restore_walk(Walk& w, Stack st, uint32_t levels,
     w.visit = q[6 * (uint64_t)stride];
     w.alive = q[7 * (uint64_t)stride];
     w.leaf = (uint64_t)q[8 * (uint64_t)stride] | ((uint64_t)q[9 * (uint64_t)stride] << 32);
-    for (uint32_t l = 1; l < leafLevel && l < w.level; ++l) st.at_idx(l) = q[(uint64_t)(kWalkWords + l - 1) * stride];
+    for (uint32_t h = 3; h < levels; ++h) st.at_idx(h) = q[(uint64_t)(kWalkWords + h - 3) * stride];
+    st.at_idx(levels) = root;
     const uint32_t m0 = kWalkWords + (kMaxLevels - 3);
-    for (uint32_t l = 0; l < levels && l < w.level; l += 2) {
-        const uint32_t v = q[(uint64_t)(m0 + l / 2) * stride];
-        st.at_mask(l) = (uint16_t)v;
-        if (l + 1 < levels) st.at_mask(l + 1) = (uint16_t)(v >> 16);
+    for (uint32_t h = 1; h <= levels; h += 2) {
+        const uint32_t v = q[(uint64_t)(m0 + h / 2) * stride];
+        st.at_mask(h) = (uint16_t)v;
+        if (h + 1 <= levels) st.at_mask(h + 1) = (uint16_t)(v >> 16);
     }
 }
 
@@ -419,7 +533,7 @@ template <bool kCount, int kFetch>
 __global__ __launch_bounds__(kBlock) void k_trace_paths(DevDag dag, RayP p, const RayP* __restrict__ pmem, uint32_t W, uint32_t H,
                                                         uint4* __restrict__ out, uint32_t tileW, uint32_t tileH,
                                                         unsigned long long* counter, LongRays L) {
-    const Stack st = stack_of(dag.levels);
+    const Stack st = stack_of<false>(dag.levels);
     if (pmem) p = *pmem;
     if (dag.root_ptr) dag.root = *dag.root_ptr;
     uint32_t x, y;
@@ -431,20 +545,15 @@ __global__ __launch_bounds__(kBlock) void k_trace_paths(DevDag dag, RayP p, cons
         F3 o, d, inv;
         uint32_t order;
         primary_ray(p, x, y, o, d, inv, order);
-        uint32_t vx, vy, vz;
-        if (kCount || L.cap == ~0u) {
-            descend<kCount, kFetch>(dag, o, d, inv, order, vx, vy, vz, st, bytes);
-        } else {
-            give = descend_capped<kFetch>(dag, o, d, inv, order, vx, vy, vz, st, L.cap, w) == kWalkOn;
-        }
-        if (!give) out[(uint64_t)(H - 1 - y) * W + x] = make_uint4(vx, vy, vz, 0u);
+        give = descend<kCount, kFetch, false>(dag, make_ray<false>(o, d, inv, order), st, L.cap, w, bytes) == kWalkOn;
+        if (!give) out[(uint64_t)(H - 1 - y) * W + x] = make_uint4(w.px, w.py, w.pz, 0u);
         if (kCount) bytes += 16;
     }
     if (!kCount && L.cap != ~0u) {
         const uint32_t slot = long_slot(give, L);
         if (give) {
             L.items[slot] = y * W + x;
-            if (L.state) save_walk(w, st, dag.levels, dag.leaf_level, L.state, L.stride, slot);
+            if (L.state) save_walk(w, st, dag.levels, L.state, L.stride, slot);
         }
     }
     flush_count<kCount>(bytes, counter);
@@ -735,7 +844,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_shadows(DevDag dag, RayP p, co
                                                           const uint4* __restrict__ paths, uint32_t* __restrict__ colors,
                                                           float bias, float fog, uint32_t tileW, uint32_t tileH,
                                                           unsigned long long* counter, LongRays L) {
-    const Stack st = stack_of(dag.levels);
+    const Stack st = stack_of<true>(dag.levels);
     if (pmem) p = *pmem;
     if (dag.root_ptr) dag.root = *dag.root_ptr;
     uint32_t x, y;
@@ -766,16 +875,9 @@ __global__ __launch_bounds__(kBlock) void k_trace_shadows(DevDag dag, RayP p, co
             camera_dir(p, x, H - 1 - y, cx, cy, cz);
             const F3 o = shadow_origin(p, pp, cx, cy, cz, bias, sun);
             const F3 inv{(float)(1.0 / (double)sun.x), (float)(1.0 / (double)sun.y), (float)(1.0 / (double)sun.z)};
-            const uint32_t order = (sun.x < 0.f ? 4u : 0u) + (sun.y < 0.f ? 2u : 0u) + (sun.z < 0.f ? 1u : 0u);
-            uint32_t vx, vy, vz;
-            bool shadowed;
-            if (kCount || L.cap == ~0u) {
-                shadowed = descend<kCount, kFetch>(dag, o, sun, inv, order, vx, vy, vz, st, bytes);
-            } else {
-                const uint32_t r = descend_capped<kFetch>(dag, o, sun, inv, order, vx, vy, vz, st, L.cap, w);
-                give = r == kWalkOn;
-                shadowed = r == kWalkHit;
-            }
+            const uint32_t r = descend<kCount, kFetch, true>(dag, make_ray<true>(o, sun, inv, 0), st, L.cap, w, bytes);
+            give = r == kWalkOn;
+            const bool shadowed = r == kWalkHit;
             if (give) {
             } else if (noFog) {
                 colors[pix] = shade_clear(colorIn, shadowed ? 0.f : 1.f);
@@ -790,7 +892,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_shadows(DevDag dag, RayP p, co
         const uint32_t slot = long_slot(give, L);
         if (give) {
             L.items[slot] = y * W + x;
-            if (L.state) save_walk(w, st, dag.levels, dag.leaf_level, L.state, L.stride, slot);
+            if (L.state) save_walk(w, st, dag.levels, L.state, L.stride, slot);
         }
     }
     flush_count<kCount>(bytes, counter);
@@ -923,7 +1025,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_persist(DevDag dag, RayP p, co
                                                           const uint2* __restrict__ shades,
                                                           const uint32_t* __restrict__ cnt, uint32_t tileW,
                                                           uint32_t tileH, TileQ Q, uint32_t refillAt) {
-    const Stack st = stack_of(dag.levels);
+    const Stack st = stack_of<kShadow>(dag.levels);
     if (!kShadow && pmem) p = *pmem;
     if (dag.root_ptr) dag.root = *dag.root_ptr;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
@@ -941,10 +1043,10 @@ __global__ __launch_bounds__(kBlock) void k_trace_persist(DevDag dag, RayP p, co
     Walk w;
     F3 o{}, d{}, inv{};
     uint32_t order = 0;
+    Ray ray{};
     if (kShadow) {
         sun_direction(d.x, d.y, d.z);
         inv = F3{(float)(1.0 / (double)d.x), (float)(1.0 / (double)d.y), (float)(1.0 / (double)d.z)};
-        order = (d.x < 0.f ? 4u : 0u) + (d.y < 0.f ? 2u : 0u) + (d.z < 0.f ? 1u : 0u);
     }
     uint64_t unused = 0;
     for (;;) {
@@ -991,7 +1093,8 @@ __global__ __launch_bounds__(kBlock) void k_trace_persist(DevDag dag, RayP p, co
                         pix = work;
                         primary_ray(p, pix % W, pix / W, o, d, inv, order);
                     }
-                    walk_begin<false, kFetch>(dag, w, o, d, inv, unused);
+                    ray = make_ray<kShadow>(o, d, inv, order);
+                    walk_begin<false, kFetch, kShadow>(dag, w, ray, st, unused);
                     active = true;
                 }
             }
@@ -1001,7 +1104,8 @@ __global__ __launch_bounds__(kBlock) void k_trace_persist(DevDag dag, RayP p, co
             continue;
         }
         if (active) {
-            const uint32_t r = walk_step<false, kFetch>(dag, w, o, d, inv, order, st, unused);
+            if (w.s != 0) walk_step<false, kFetch, kShadow, false>(dag, w, ray, st, unused);
+            const uint32_t r = walk_result(w);
             if (r != kWalkOn) {
                 active = false;
                 if (kShadow) {
@@ -1225,14 +1329,14 @@ __global__ __launch_bounds__(kBlock) void k_trace_rest(DevDag dag, RayP p, const
                                                        uint32_t H, uint4* __restrict__ paths,
                                                        uint32_t* __restrict__ colors, float bias, float fog,
                                                        LongRays rest) {
-    const Stack st = stack_of(dag.levels);
+    const Stack st = stack_of<kShadow>(dag.levels);
     if (pmem) p = *pmem;
     if (dag.root_ptr) dag.root = *dag.root_ptr;
     const uint32_t n = *rest.count;
     uint64_t unused = 0;
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const uint32_t pix = rest.items[i], x = pix % W, y = pix / W;
-        uint32_t vx, vy, vz;
+        Walk w;
         if (kShadow) {
             F3 sun;
             sun_direction(sun.x, sun.y, sun.z);
@@ -1241,8 +1345,8 @@ __global__ __launch_bounds__(kBlock) void k_trace_rest(DevDag dag, RayP p, const
             camera_dir(p, x, H - 1 - y, cx, cy, cz);
             const F3 o = shadow_origin(p, pp, cx, cy, cz, bias, sun);
             const F3 inv{(float)(1.0 / (double)sun.x), (float)(1.0 / (double)sun.y), (float)(1.0 / (double)sun.z)};
-            const uint32_t order = (sun.x < 0.f ? 4u : 0u) + (sun.y < 0.f ? 2u : 0u) + (sun.z < 0.f ? 1u : 0u);
-            const bool shadowed = descend<false, kFetch>(dag, o, sun, inv, order, vx, vy, vz, st, unused);
+            const bool shadowed =
+                descend<false, kFetch, true>(dag, make_ray<true>(o, sun, inv, 0), st, ~0u, w, unused) == kWalkHit;
             const uint32_t colorIn = colors[pix];
             if (fog == 0.f) {
                 colors[pix] = shade_clear(colorIn, shadowed ? 0.f : 1.f);
@@ -1255,8 +1359,8 @@ __global__ __launch_bounds__(kBlock) void k_trace_rest(DevDag dag, RayP p, const
             F3 o, d, inv;
             uint32_t order;
             primary_ray(p, x, y, o, d, inv, order);
-            descend<false, kFetch>(dag, o, d, inv, order, vx, vy, vz, st, unused);
-            paths[(uint64_t)(H - 1 - y) * W + x] = make_uint4(vx, vy, vz, 0u);
+            descend<false, kFetch, false>(dag, make_ray<false>(o, d, inv, order), st, ~0u, w, unused);
+            paths[(uint64_t)(H - 1 - y) * W + x] = make_uint4(w.px, w.py, w.pz, 0u);
         }
     }
 }
@@ -1270,7 +1374,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_resume(DevDag dag, RayP p, con
                                                          uint32_t H, uint4* __restrict__ paths,
                                                          uint32_t* __restrict__ colors, float bias, float fog,
                                                          LongRays R, LongRays B, uint32_t steps) {
-    const Stack st = stack_of(dag.levels);
+    const Stack st = stack_of<kShadow>(dag.levels);
     if (pmem) p = *pmem;
     if (dag.root_ptr) dag.root = *dag.root_ptr;
     const uint32_t n = *R.count;
@@ -1285,7 +1389,7 @@ __global__ __launch_bounds__(kBlock) void k_trace_resume(DevDag dag, RayP p, con
             pix = R.items[i];
             const uint32_t x = pix % W, y = pix / W;
             F3 o, d, inv;
-            uint32_t order;
+            uint32_t order = 0;
             uint4 pp{};
             if (kShadow) {
                 sun_direction(d.x, d.y, d.z);
@@ -1294,14 +1398,13 @@ __global__ __launch_bounds__(kBlock) void k_trace_resume(DevDag dag, RayP p, con
                 camera_dir(p, x, H - 1 - y, cx, cy, cz);
                 o = shadow_origin(p, pp, cx, cy, cz, bias, d);
                 inv = F3{(float)(1.0 / (double)d.x), (float)(1.0 / (double)d.y), (float)(1.0 / (double)d.z)};
-                order = (d.x < 0.f ? 4u : 0u) + (d.y < 0.f ? 2u : 0u) + (d.z < 0.f ? 1u : 0u);
             } else {
                 primary_ray(p, x, y, o, d, inv, order);
             }
+            const Ray ray = make_ray<kShadow>(o, d, inv, order);
             Walk w;
-            restore_walk(w, st, dag.levels, dag.leaf_level, R.state, R.stride, i);
-            uint32_t r = kWalkOn, k = 0;
-            while (r == kWalkOn && k++ < steps) r = walk_step<false, kFetchPointer>(dag, w, o, d, inv, order, st, unused);
+            restore_walk(w, st, dag.levels, dag.root, R.state, R.stride, i);
+            const uint32_t r = walk_run<false, kFetchPointer, kShadow, false>(dag, w, ray, st, steps, unused);
             give = r == kWalkOn;
             if (!give) {
                 if (kShadow) {

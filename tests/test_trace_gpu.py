@@ -69,6 +69,56 @@ def test_trace_parity(name, W, H, ncam):
         assert np.array_equal(gshad, oshad), f"shadows differ at {np.argwhere(gshad != oshad)[:5]}"
 
 
+@pytest.mark.parametrize("schedule", [(0, 0), (1, 16), (2, 5), (3, 4 | (16 << 16))])
+@pytest.mark.parametrize("fetch", [0, 1])
+def test_rays_of_every_order_and_along_axes(schedule, fetch):
+    """Rays of all eight sign patterns, and rays with components that are exactly zero (their
+    inverse is infinite and the intersection terms hold NaN), from inside and outside the scene,
+    through every walk."""
+    import torch
+    from hashdag_amd import DAGTracer
+    from hashdag_amd._lib import hd_ray_params, lib
+    from oracle import Oracle
+
+    p, sc, g, dag, od, oc = _setup("d8")
+    W = H = 64
+    tracer = DAGTracer(W, H)
+    lib.hd_set_trace_schedule(dag.handle, *schedule)
+    tracer.set_fetch(dag, fetch)
+    seen = set()
+    hits = 0
+    for axis in range(3):
+        for sign in (1.0, -1.0):
+            for cam in ((128.0, 160.0, 128.0), (140.5, 90.25, 30.75), (128.0, 300.0, -20.0)):
+                u, v = (axis + 1) % 3, (axis + 2) % 3
+                corner, ddx, ddy = list(cam), [0.0] * 3, [0.0] * 3
+                corner[axis] += sign
+                corner[u] -= 0.5
+                corner[v] -= 0.5
+                ddx[u] = ddy[v] = 1.0 / 64.0  # exact: column and row 32 run along the axis planes
+                flat = [*cam, *corner, *ddx, *ddy]
+                prm = hd_ray_params()
+                prm.camera_position[:], prm.ray_min[:], prm.ray_ddx[:], prm.ray_ddy[:] = cam, corner, ddx, ddy
+                oparams = np.array(flat, np.float64)
+                tracer.resolve_paths(None, None, dag, params=prm)
+                tracer.resolve_colors(dag)
+                tracer.resolve_shadows(None, None, dag, 1.0, 0.0, params=prm)
+                torch.cuda.synchronize()
+                opaths = Oracle.trace_paths(od, oparams, W, H)
+                gpaths = tracer.paths.cpu().numpy().view(np.uint32)
+                assert np.array_equal(gpaths, opaths), (axis, sign, cam, np.argwhere((gpaths != opaths).any(-1))[:5])
+                ocols = Oracle.trace_colors(od, oc, opaths, W, H)
+                oshad = Oracle.trace_shadows(od, oparams, opaths, ocols, W, H, 1.0, 0.0)
+                gshad = tracer.colors.cpu().numpy().view(np.uint32)
+                assert np.array_equal(gshad, oshad), (axis, sign, cam, np.argwhere(gshad != oshad)[:5])
+                hits += int((opaths[..., :3] != 0).any(-1).sum())
+                d = np.array(corner) - np.array(cam)
+                for k in range(4):
+                    e = d + np.array(ddx) * (63 * (k & 1)) + np.array(ddy) * (63 * (k >> 1))
+                    seen.add(tuple(e < 0))
+    assert len(seen) == 8 and hits > 1000
+
+
 def test_byte_counters_match_oracle():
     import torch
     from hashdag_amd import DAGInfo, DAGTracer, ray_params
