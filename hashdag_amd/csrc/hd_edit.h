@@ -116,7 +116,7 @@ struct Items {
     uint8_t* ckind;             // per child slot: keep / empty / full / item
     uint32_t *cval, *corig, *cold, *cnew, *ccolor, *cstart, *costart;
     uint32_t *nidx, *ncount;    // result: new node index and voxel count
-    uint32_t *cont, *clen, *hash, *rep, *state;  // pending node content (9 words) for the table
+    uint32_t *cont, *clen, *hash, *state;  // pending node content (9 words) for the table
     uint32_t *nstart, *ostart;  // colour starts relative to the task
     uint64_t* cbase;            // tasks: base of the task's colour array
 };
@@ -127,6 +127,7 @@ struct EditPass {
     uint32_t* vpool;
     uint32_t* page_table;
     uint32_t* bucket_sizes;
+    const uint32_t* bucket_snap;  // the sizes before the pass
     const uint32_t* full_nodes;
     uint32_t* pool_top;
     uint32_t* errors;

@@ -43,6 +43,7 @@ namespace {
 
 constexpr uint32_t KIND_KEEP = 0, KIND_EMPTY = 1, KIND_FULL = 2, KIND_ITEM = 3;
 constexpr uint32_t kGrid = 2048;  // blocks of grid-stride kernels
+constexpr uint32_t kTopBlock = 1024;  // threads of the workgroup that runs a pass's small levels (k_top)
 
 // Wave-strided loops (one work item per wavefront): the index is made wave-uniform so the
 // compiler keeps it in a scalar register and loads the item's fields through the scalar cache.
@@ -632,7 +633,7 @@ __device__ __forceinline__ void slot_child_item(const EditPass& P, const Items& 
 // expand: items of level l -> child classification and items of level l+1
 // ---------------------------------------------------------------------------------------------
 __device__ __forceinline__ void d_expand(const EditPass& P, uint32_t l, VGrid G) {
-    __shared__ uint32_t sAlloc[2 * (256 / 64 + 1)];
+    __shared__ uint32_t sAlloc[2 * (kTopBlock / 64 + 1)];
     __shared__ uint32_t sErr;
     const uint32_t n = min(P.count[l], P.cap[l]);
     if (threadIdx.x == 0) sErr = *P.errors;
@@ -880,12 +881,29 @@ __device__ __forceinline__ uint64_t leaf_touch_mask(const E& e, uint32_t bx, uin
     return tm;
 }
 
+// Slots of the dedup hash set a level uses: the power of two at or above twice its item
+// count (load factor at most 1/2), at most the whole set.
+__device__ __forceinline__ uint32_t hset_slots(const EditPass& P, uint32_t l) {
+    const uint32_t n = min(P.count[l], P.cap[l]);
+    uint32_t m = 64;
+    while (m < P.hcap && m < 2u * n) m <<= 1;
+    return min(m, P.hcap);
+}
+
+// clears the slots of the dedup hash set that level l will use (the step before its k_nodes /
+// k_dedup does; the level below is done with them)
+__device__ __forceinline__ void d_hset_clear(const EditPass& P, uint32_t l, VGrid G) {
+    const uint32_t m = hset_slots(P, l);
+    for (uint32_t i = G.block * blockDim.x + threadIdx.x; i < m; i += G.nblocks * blockDim.x) P.hset[i] = 0u;
+}
+
 // kSpecial: the pass may hold copy / fill editors (their code is built in only then)
 template <bool kSpecial>
 __device__ __forceinline__ void d_leaf(const EditPass& P, VGrid G) {
     const uint32_t L = P.levels - 2;
     const uint32_t n = min(P.count[L], P.cap[L]);
     if (*P.errors) return;
+    d_hset_clear(P, L, G);
     const Items I = P.items[L];
     uint64_t leafBytes = 0;  // old and original leaves read (measurement)
     for (uint32_t t0 = G.block * blockDim.x + (threadIdx.x & ~63u); t0 < n; t0 += G.nblocks * blockDim.x) {
@@ -982,9 +1000,18 @@ __global__ __launch_bounds__(256) void k_leaf(EditPass P) {
 // ---------------------------------------------------------------------------------------------
 // build interior items of level l from their children's results
 // ---------------------------------------------------------------------------------------------
+// States of an item: its node is known (0, 2), its content waits for the table (1), or it shares
+// the content of the item that nidx names (3, set by dedup).
+constexpr uint32_t kStateKnown = 0, kStatePending = 1, kStateFound = 2, kStateDuplicate = 3;
+// the node a finished item resolved to
+__device__ __forceinline__ uint32_t item_node(const Items& I, uint32_t i) {
+    const uint32_t v = I.nidx[i];
+    return I.state[i] == kStateDuplicate ? I.nidx[v] : v;
+}
 __device__ __forceinline__ void d_build(const EditPass& P, uint32_t l, VGrid G) {
     const uint32_t n = min(P.count[l], P.cap[l]);
     if (*P.errors) return;
+    d_hset_clear(P, l, G);
     const Items I = P.items[l];
     const Items C = P.items[l + 1];
     const uint32_t D = P.levels, ctl = P.ctl;
@@ -999,7 +1026,7 @@ __device__ __forceinline__ void d_build(const EditPass& P, uint32_t l, VGrid G) 
             uint32_t idx, cnt;
             if (kind == KIND_ITEM) {
                 const uint32_t ci = I.cval[slot];
-                idx = C.nidx[ci];
+                idx = item_node(C, ci);
                 cnt = C.ncount[ci];
                 I.cnew[slot] = cnt;
             } else {
@@ -1038,28 +1065,10 @@ __global__ __launch_bounds__(256) void k_build(EditPass P, uint32_t l) {
 }
 
 // ---------------------------------------------------------------------------------------------
-// dedup / find / add / resolve for the pending items of one level
+// dedup / find / add for the pending items of one level
 // ---------------------------------------------------------------------------------------------
 __global__ void k_fill(uint32_t* p, uint64_t n, uint32_t v) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) p[i] = v;
-}
-
-// Slots of the dedup hash set a level uses: the power of two at or above twice its item
-// count (load factor at most 1/2), at most the whole set.
-__device__ __forceinline__ uint32_t hset_slots(const EditPass& P, uint32_t l) {
-    const uint32_t n = min(P.count[l], P.cap[l]);
-    uint32_t m = 64;
-    while (m < P.hcap && m < 2u * n) m <<= 1;
-    return min(m, P.hcap);
-}
-
-// clears the slots of the dedup hash set that level l will use
-__device__ __forceinline__ void d_hset_clear(const EditPass& P, uint32_t l, VGrid G) {
-    const uint32_t m = hset_slots(P, l);
-    for (uint32_t i = G.block * blockDim.x + threadIdx.x; i < m; i += G.nblocks * blockDim.x) P.hset[i] = 0u;
-}
-__global__ void k_hset_clear(EditPass P, uint32_t l) {
-    d_hset_clear(P, l, VGrid{blockIdx.x, gridDim.x});
 }
 
 __device__ __forceinline__ bool same_content(const Items& I, uint32_t a, uint32_t b) {
@@ -1070,8 +1079,30 @@ __device__ __forceinline__ bool same_content(const Items& I, uint32_t a, uint32_
     return true;
 }
 
-// Representatives (the first item of each distinct content) are listed for k_find, in the
-// level's nstart words (free until the colour phase), with one atomic per block.
+// Enters pending item i into the level's hash set: true for the first item of its content (its
+// representative), else the item becomes a duplicate of the one that is there.
+__device__ __forceinline__ bool dedup_item(const EditPass& P, const Items& I, uint32_t i, uint32_t hmask) {
+    uint32_t s = I.hash[i] & hmask;
+    for (;;) {
+        // read first: many items can share one content (and so one slot), and a CAS per
+        // item on one address would serialise them all
+        uint32_t cur = __atomic_load_n(&P.hset[s], __ATOMIC_RELAXED);
+        if (cur == 0) {
+            cur = atomicCAS(&P.hset[s], 0u, i + 1);
+            if (cur == 0) return true;
+        }
+        const uint32_t j = cur - 1;
+        if (I.hash[j] == I.hash[i] && same_content(I, i, j)) {
+            I.nidx[i] = j;
+            I.state[i] = kStateDuplicate;
+            return false;
+        }
+        s = (s + 1) & hmask;
+    }
+}
+
+// Representatives are listed for k_find, in the level's nstart words (free until the colour
+// phase), with one atomic per block.
 __device__ __forceinline__ void d_dedup(const EditPass& P, uint32_t l, VGrid G) {
     __shared__ uint32_t sAlloc[256 / 64 + 1];
     __shared__ uint32_t sErr;
@@ -1083,29 +1114,7 @@ __device__ __forceinline__ void d_dedup(const EditPass& P, uint32_t l, VGrid G) 
     const uint32_t hmask = hset_slots(P, l) - 1;
     for (uint32_t b0 = G.block * blockDim.x; b0 < n; b0 += G.nblocks * blockDim.x) {
         const uint32_t i = b0 + threadIdx.x;
-        bool isRep = false;
-        if (i < n && I.state[i] == 1) {
-            uint32_t s = I.hash[i] & hmask;
-            for (;;) {
-                // read first: many items can share one content (and so one slot), and a CAS per
-                // item on one address would serialise them all
-                uint32_t cur = __atomic_load_n(&P.hset[s], __ATOMIC_RELAXED);
-                if (cur == 0) {
-                    cur = atomicCAS(&P.hset[s], 0u, i + 1);
-                    if (cur == 0) {
-                        I.rep[i] = i;
-                        isRep = true;
-                        break;
-                    }
-                }
-                const uint32_t j = cur - 1;
-                if (I.hash[j] == I.hash[i] && same_content(I, i, j)) {
-                    I.rep[i] = j;
-                    break;
-                }
-                s = (s + 1) & hmask;
-            }
-        }
+        const bool isRep = i < n && I.state[i] == kStatePending && dedup_item(P, I, i, hmask);
         const uint32_t at = block_alloc32(sAlloc, &P.find_count[l], isRep ? 1u : 0u);
         if (isRep) I.nstart[at] = i;
     }
@@ -1114,99 +1123,84 @@ __global__ __launch_bounds__(256) void k_dedup(EditPass P, uint32_t l) {
     d_dedup(P, l, VGrid{blockIdx.x, gridDim.x});
 }
 
-// One wavefront per representative: scan the bucket for an identical node (any word
-// position inside the bucket's used size whose words equal the node and that does not
-// cross a page boundary holds the same node content).
-__device__ __forceinline__ void d_find(const EditPass& P, uint32_t l, VGrid G) {
-    const uint32_t n = min(P.count[l], P.cap[l]);
-    if (*P.errors) return;
-    const Items I = P.items[l];
-    const Geom g = P.g;
+// The wavefront scans the bucket of item i for an identical node (any word position inside the
+// bucket's used size whose words equal the node and that does not cross a page boundary holds
+// the same node content); its position in the bucket, or ~0. The size is the bucket's before the
+// pass: what the pass appends to a level are contents that no other item of the level has, so
+// they need not be seen, and other wavefronts may be writing them.
+__device__ __forceinline__ uint32_t find_node(const EditPass& P, const Items& I, uint32_t l, uint32_t i,
+                                              uint64_t& scanBytes) {
+    const Geom& g = P.g;
     const uint32_t lane = threadIdx.x & 63u;
     const bool leafLevel = l == g.leaf_level();
-    // the representatives listed by k_dedup
-    const uint32_t nReps = min(P.find_count[l], n);
-    uint64_t scanBytes = 0;  // bucket bytes this lane read (measurement)
-    for (uint32_t r = wave_index(G); r < nReps; r += wave_count(G)) {
-        const uint32_t i = I.nstart[r];
-        const uint32_t bucket = g.bucket_from_hash(l, I.hash[i]);
-        const uint32_t base = g.make_ptr(l, bucket, 0);
-        const uint32_t bs = P.bucket_sizes[g.bucket_global(l, bucket)];
-        const uint32_t nw = I.clen[i];
-        uint32_t found = ~0u;
-        if (leafLevel && P.leaf_tags) {
-            // slots (2 words each) whose tag byte matches, lowest first, confirmed on the leaf;
-            // 4 tags per lane, 256 slots per wavefront step
-            const uint64_t key = (uint64_t)I.cont[i * 9] | ((uint64_t)I.cont[i * 9 + 1] << 32);
-            const uint32_t want = I.hash[i] >> 24, nslots = bs / 2;
-            const uint8_t* tags = P.leaf_tags + (uint64_t)bucket * (g.bucket_size(l) / 2);
-            for (uint32_t s0 = 0; s0 < nslots && found == ~0u; s0 += 256) {
-                const uint32_t sl = s0 + 4 * lane;
-                uint32_t hitSlot = ~0u;
-                if (sl < nslots) {
-                    const uint32_t four = *reinterpret_cast<const uint32_t*>(tags + sl);
-                    scanBytes += min(4u, nslots - sl);
-                    for (uint32_t k = 0; k < 4 && hitSlot == ~0u; ++k)
-                        if (sl + k < nslots && ((four >> (8 * k)) & 0xFFu) == want) {
-                            scanBytes += 8;
-                            if (*reinterpret_cast<const uint64_t*>(P.vpool + base + 2 * (sl + k)) == key) hitSlot = sl + k;
-                        }
-                }
-                const uint64_t b = __ballot(hitSlot != ~0u);
-                if (b) found = 2u * (uint32_t)__shfl((int)hitSlot, __ffsll((long long)b) - 1, 64);
-            }
-        } else if (leafLevel) {
-            const uint64_t key = (uint64_t)I.cont[i * 9] | ((uint64_t)I.cont[i * 9 + 1] << 32);
-            for (uint32_t p0 = 0; p0 < bs && found == ~0u; p0 += 128) {
-                const uint32_t pos = p0 + 2 * lane;
-                if (pos + 2 <= bs) scanBytes += 8;
-                const bool hit = pos + 2 <= bs && *reinterpret_cast<const uint64_t*>(P.vpool + base + pos) == key;
-                const uint64_t b = __ballot(hit);
-                if (b) found = p0 + 2 * (uint32_t)__ffsll((long long)b) - 2;
-            }
-        } else {
-            // The reference walks node by node from each page start and compares only nodes
-            // with start + n < min(bucketSize, pageEnd). The wave compares all positions at
-            // once, then confirms the first candidate lies on that walk.
-            const uint32_t h0 = I.cont[i * 9];
-            const uint32_t ps = g.page_size;
-            for (uint32_t p0 = 0; p0 + nw < bs && found == ~0u; p0 += 64) {
-                const uint32_t pos = p0 + lane;
-                const uint32_t pageEnd = min(bs, pos - pos % ps + ps);
-                if (pos < bs) scanBytes += 4;
-                bool hit = pos + nw < pageEnd && P.vpool[base + pos] == h0;
-                if (hit)
-                    for (uint32_t k = 1; k < nw; ++k) {
-                        scanBytes += 4;
-                        if (P.vpool[base + pos + k] != I.cont[i * 9 + k]) {
-                            hit = false;
-                            break;
-                        }
+    const uint32_t bucket = g.bucket_from_hash(l, I.hash[i]);
+    const uint32_t base = g.make_ptr(l, bucket, 0);
+    const uint32_t bs = P.bucket_snap[g.bucket_global(l, bucket)];
+    const uint32_t nw = I.clen[i];
+    uint32_t found = ~0u;
+    if (leafLevel && P.leaf_tags) {
+        // slots (2 words each) whose tag byte matches, lowest first, confirmed on the leaf;
+        // 4 tags per lane, 256 slots per wavefront step
+        const uint64_t key = (uint64_t)I.cont[i * 9] | ((uint64_t)I.cont[i * 9 + 1] << 32);
+        const uint32_t want = I.hash[i] >> 24, nslots = bs / 2;
+        const uint8_t* tags = P.leaf_tags + (uint64_t)bucket * (g.bucket_size(l) / 2);
+        for (uint32_t s0 = 0; s0 < nslots && found == ~0u; s0 += 256) {
+            const uint32_t sl = s0 + 4 * lane;
+            uint32_t hitSlot = ~0u;
+            if (sl < nslots) {
+                const uint32_t four = *reinterpret_cast<const uint32_t*>(tags + sl);
+                scanBytes += min(4u, nslots - sl);
+                for (uint32_t k = 0; k < 4 && hitSlot == ~0u; ++k)
+                    if (sl + k < nslots && ((four >> (8 * k)) & 0xFFu) == want) {
+                        scanBytes += 8;
+                        if (*reinterpret_cast<const uint64_t*>(P.vpool + base + 2 * (sl + k)) == key) hitSlot = sl + k;
                     }
-                uint64_t b = __ballot(hit);
-                while (b) {
-                    const uint32_t c = p0 + (uint32_t)__ffsll((long long)b) - 1;  // wave-uniform
-                    uint32_t w = c - c % ps;
-                    while (w < c) w += 1u + __popc(P.vpool[base + w] & 0xFFu);  // advances >= 1 word
-                    if (w == c) {
-                        found = c;
+            }
+            const uint64_t b = __ballot(hitSlot != ~0u);
+            if (b) found = 2u * (uint32_t)__shfl((int)hitSlot, __ffsll((long long)b) - 1, 64);
+        }
+    } else if (leafLevel) {
+        const uint64_t key = (uint64_t)I.cont[i * 9] | ((uint64_t)I.cont[i * 9 + 1] << 32);
+        for (uint32_t p0 = 0; p0 < bs && found == ~0u; p0 += 128) {
+            const uint32_t pos = p0 + 2 * lane;
+            if (pos + 2 <= bs) scanBytes += 8;
+            const bool hit = pos + 2 <= bs && *reinterpret_cast<const uint64_t*>(P.vpool + base + pos) == key;
+            const uint64_t b = __ballot(hit);
+            if (b) found = p0 + 2 * (uint32_t)__ffsll((long long)b) - 2;
+        }
+    } else {
+        // The reference walks node by node from each page start and compares only nodes
+        // with start + n < min(bucketSize, pageEnd). The wave compares all positions at
+        // once, then confirms the first candidate lies on that walk.
+        const uint32_t h0 = I.cont[i * 9];
+        const uint32_t ps = g.page_size;
+        for (uint32_t p0 = 0; p0 + nw < bs && found == ~0u; p0 += 64) {
+            const uint32_t pos = p0 + lane;
+            const uint32_t pageEnd = min(bs, pos - pos % ps + ps);
+            if (pos < bs) scanBytes += 4;
+            bool hit = pos + nw < pageEnd && P.vpool[base + pos] == h0;
+            if (hit)
+                for (uint32_t k = 1; k < nw; ++k) {
+                    scanBytes += 4;
+                    if (P.vpool[base + pos + k] != I.cont[i * 9 + k]) {
+                        hit = false;
                         break;
                     }
-                    b &= b - 1;
                 }
-            }
-        }
-        if (lane == 0) {
-            if (found != ~0u) {
-                I.nidx[i] = base + found;
-                I.state[i] = 2;  // resolved by find
+            uint64_t b = __ballot(hit);
+            while (b) {
+                const uint32_t c = p0 + (uint32_t)__ffsll((long long)b) - 1;  // wave-uniform
+                uint32_t w = c - c % ps;
+                while (w < c) w += 1u + __popc(P.vpool[base + w] & 0xFFu);  // advances >= 1 word
+                if (w == c) {
+                    found = c;
+                    break;
+                }
+                b &= b - 1;
             }
         }
     }
-    if (P.abytes) wave_add64(P.abytes + 1, scanBytes);
-}
-__global__ __launch_bounds__(256) void k_find(EditPass P, uint32_t l) {
-    d_find(P, l, VGrid{blockIdx.x, gridDim.x});
+    return found == ~0u ? ~0u : base + found;
 }
 
 __device__ bool alloc_page(const EditPass& P, uint32_t page) {
@@ -1221,46 +1215,86 @@ __device__ bool alloc_page(const EditPass& P, uint32_t page) {
     return true;
 }
 
-__device__ __forceinline__ void d_add(const EditPass& P, uint32_t l, VGrid G) {
-    const uint32_t n = min(P.count[l], P.cap[l]);
+// Appends item i to its bucket (one lane): space by a CAS on the bucket size, with the page
+// padding rule; the words added.
+__device__ __forceinline__ uint32_t append_node(const EditPass& P, const Items& I, uint32_t l, uint32_t i) {
+    const Geom& g = P.g;
+    const uint32_t ps = g.page_size;
+    const uint32_t nw = I.clen[i];
+    const uint32_t bucket = g.bucket_from_hash(l, I.hash[i]);
+    uint32_t* bsPtr = &P.bucket_sizes[g.bucket_global(l, bucket)];
+    const uint32_t cap = g.bucket_size(l);
+    uint32_t start;
+    uint32_t cur = *reinterpret_cast<volatile uint32_t*>(bsPtr);
+    for (;;) {
+        const uint32_t left = ps - cur % ps;
+        start = (left == ps || left < nw) ? (left == ps ? cur : cur + left) : cur;
+        if (start + nw > cap) {
+            set_error(P.errors, ERR_BUCKET);
+            return 0;
+        }
+        const uint32_t prev = atomicCAS(bsPtr, cur, start + nw);
+        if (prev == cur) break;
+        cur = prev;
+    }
+    const uint32_t va = g.make_ptr(l, bucket, start);
+    if (start % ps == 0 && !alloc_page(P, va / ps)) return 0;
+    for (uint32_t k = 0; k < nw; ++k) P.vpool[va + k] = I.cont[i * 9 + k];
+    if (P.leaf_tags && l == g.leaf_level())
+        P.leaf_tags[(uint64_t)bucket * (cap / 2) + start / 2] = (uint8_t)(I.hash[i] >> 24);
+    I.nidx[i] = va;
+    return nw;
+}
+
+// One representative by a wavefront: found in the table, or appended to it. The words added
+// (in lane 0).
+__device__ __forceinline__ uint32_t find_or_add(const EditPass& P, const Items& I, uint32_t l, uint32_t i,
+                                                uint64_t& scanBytes) {
+    const uint32_t va = find_node(P, I, l, i, scanBytes);
+    uint32_t added = 0;
+    if ((threadIdx.x & 63u) == 0) {
+        if (va != ~0u) {
+            I.nidx[i] = va;
+            I.state[i] = kStateFound;
+        } else {
+            added = append_node(P, I, l, i);
+        }
+    }
+    return added;
+}
+
+// a wavefront per representative listed by k_dedup: found in the table, or left pending
+__device__ __forceinline__ void d_find(const EditPass& P, uint32_t l, VGrid G) {
     if (*P.errors) return;
     const Items I = P.items[l];
-    const Geom g = P.g;
-    const uint32_t ps = g.page_size;
-    for (uint32_t t0 = G.block * blockDim.x + (threadIdx.x & ~63u); t0 < n; t0 += G.nblocks * blockDim.x) {
-        const uint32_t i = t0 + (threadIdx.x & 63u);
+    const uint32_t nReps = min(P.find_count[l], min(P.count[l], P.cap[l]));
+    uint64_t scanBytes = 0;  // bucket bytes this lane read (measurement)
+    for (uint32_t r = wave_index(G); r < nReps; r += wave_count(G)) {
+        const uint32_t i = I.nstart[r];
+        const uint32_t va = find_node(P, I, l, i, scanBytes);
+        if ((threadIdx.x & 63u) == 0 && va != ~0u) {
+            I.nidx[i] = va;
+            I.state[i] = kStateFound;
+        }
+    }
+    if (P.abytes) wave_add64(P.abytes + 1, scanBytes);
+}
+__global__ __launch_bounds__(256) void k_find(EditPass P, uint32_t l) {
+    d_find(P, l, VGrid{blockIdx.x, gridDim.x});
+}
+
+// a thread per representative: those k_find left pending are appended (one lane of k_find's
+// wavefronts doing so held a first pass of 4096 editors, which adds 17 M words, for 35 ms)
+__device__ __forceinline__ void d_add(const EditPass& P, uint32_t l, VGrid G) {
+    if (*P.errors) return;
+    const Items I = P.items[l];
+    const uint32_t nReps = min(P.find_count[l], min(P.count[l], P.cap[l]));
+    for (uint32_t t0 = G.block * blockDim.x + (threadIdx.x & ~63u); t0 < nReps; t0 += G.nblocks * blockDim.x) {
+        const uint32_t r = t0 + (threadIdx.x & 63u);
         uint32_t added = 0;
-        if (i < n && I.state[i] == 1 && I.rep[i] == i) {
-            const uint32_t nw = I.clen[i];
-            const uint32_t bucket = g.bucket_from_hash(l, I.hash[i]);
-            uint32_t* bsPtr = &P.bucket_sizes[g.bucket_global(l, bucket)];
-            const uint32_t cap = g.bucket_size(l);
-            uint32_t start;
-            bool ok = true;
-            uint32_t cur = *reinterpret_cast<volatile uint32_t*>(bsPtr);
-            for (;;) {
-                const uint32_t left = ps - cur % ps;
-                start = (left == ps || left < nw) ? (left == ps ? cur : cur + left) : cur;
-                if (start + nw > cap) {
-                    ok = false;
-                    break;
-                }
-                const uint32_t prev = atomicCAS(bsPtr, cur, start + nw);
-                if (prev == cur) break;
-                cur = prev;
-            }
-            if (!ok) {
-                set_error(P.errors, ERR_BUCKET);
-            } else {
-                const uint32_t va = g.make_ptr(l, bucket, start);
-                if (start % ps != 0 || alloc_page(P, va / ps)) {
-                    for (uint32_t k = 0; k < nw; ++k) P.vpool[va + k] = I.cont[i * 9 + k];
-                    if (P.leaf_tags && l == g.leaf_level())
-                        P.leaf_tags[(uint64_t)bucket * (cap / 2) + start / 2] = (uint8_t)(I.hash[i] >> 24);
-                    I.nidx[i] = va;
-                    added = nw;
-                }
-            }
+        if (r < nReps) {
+            const uint32_t i = I.nstart[r];
+            if (I.state[i] == kStatePending) added = append_node(P, I, l, i);
         }
         wave_add64(P.stat_new_words, added);
     }
@@ -1269,15 +1303,32 @@ __global__ __launch_bounds__(256) void k_add(EditPass P, uint32_t l) {
     d_add(P, l, VGrid{blockIdx.x, gridDim.x});
 }
 
-__device__ __forceinline__ void d_resolve(const EditPass& P, uint32_t l, VGrid G) {
+// Dedup, find and add of a level in one step: a wavefront takes a run of items (one where the
+// level has no more items than there are wavefronts), a lane each enters them into the hash set,
+// then the whole wavefront finds or adds the representatives among them one after another. One
+// launch where dedup, find and add need three (a launch costs a small level more than its work:
+// 2-5 us of each were the time of a level of a few items); on levels of many items the runs
+// would queue behind each other, so those keep the three.
+__device__ __forceinline__ void d_nodes(const EditPass& P, uint32_t l, VGrid G) {
     const uint32_t n = min(P.count[l], P.cap[l]);
     if (*P.errors) return;
     const Items I = P.items[l];
-    for (uint32_t i = G.block * blockDim.x + threadIdx.x; i < n; i += G.nblocks * blockDim.x)
-        if (I.state[i] == 1 && I.rep[i] != i) I.nidx[i] = I.nidx[I.rep[i]];
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t hmask = hset_slots(P, l) - 1;
+    const uint32_t waves = wave_count(G), run = min(64u, (n + waves - 1) / waves);
+    uint64_t scanBytes = 0;
+    uint32_t added = 0;
+    for (uint32_t i0 = wave_index(G) * run; i0 < n; i0 += waves * run) {
+        const uint32_t i = i0 + lane;
+        const bool isRep = lane < run && i < n && I.state[i] == kStatePending && dedup_item(P, I, i, hmask);
+        for (uint64_t m = __ballot(isRep); m; m &= m - 1)
+            added += find_or_add(P, I, l, i0 + (uint32_t)__ffsll((long long)m) - 1u, scanBytes);
+    }
+    wave_add64(P.stat_new_words, added);
+    if (P.abytes) wave_add64(P.abytes + 1, scanBytes);
 }
-__global__ __launch_bounds__(256) void k_resolve(EditPass P, uint32_t l) {
-    d_resolve(P, l, VGrid{blockIdx.x, gridDim.x});
+__global__ __launch_bounds__(256) void k_nodes(EditPass P, uint32_t l) {
+    d_nodes(P, l, VGrid{blockIdx.x, gridDim.x});
 }
 
 // ---------------------------------------------------------------------------------------------
@@ -1606,7 +1657,7 @@ __device__ __forceinline__ void d_color_leaf_items(const EditPass& P, VGrid G) {
         const uint32_t old = I.old_[i];
         const uint64_t oldMask = old != kInvalidNode ? *reinterpret_cast<const uint64_t*>(P.vpool + old) : 0ull;
         // the voxels k_leaf set: the leaf node the item resolved to
-        const uint32_t leaf = I.nidx[i];
+        const uint32_t leaf = item_node(I, i);
         const uint64_t v = leaf != kInvalidNode ? *reinterpret_cast<const uint64_t*>(P.vpool + leaf) : 0ull;
         bool paint = false;
         for (uint32_t k = 0; k < ec; ++k) {
@@ -2448,7 +2499,7 @@ uint64_t carve_level(Items& I, uint32_t*& elist, bool leafLevel, uint64_t c, uin
         {(void**)&I.cnew, c8 * 4},    {(void**)&I.ccolor, c8 * 4}, {(void**)&I.cstart, c8 * 4},
         {(void**)&I.costart, c8 * 4}, {(void**)&I.nidx, c * 4},    {(void**)&I.ncount, c * 4},
         {(void**)&I.cont, c * 36},    {(void**)&I.clen, c * 4},    {(void**)&I.hash, c * 4},
-        {(void**)&I.rep, c * 4},      {(void**)&I.state, c * 4},   {(void**)&I.nstart, c * 4},
+        {(void**)&I.state, c * 4},    {(void**)&I.nstart, c * 4},
         {(void**)&I.ostart, c * 4},   {(void**)&I.cbase, c * 8},   {(void**)&elist, e * 4},
     };
     auto up = [](uint64_t v) { return (v + 255) & ~255ull; };
@@ -2631,15 +2682,14 @@ hd_status leaf_tags_rebuild(hd_ctx* ctx, hipStream_t s) {
 namespace {
 // A whole pass in one launch: the pass kernels' bodies in the order the level-synchronous form
 // launches them, each over the same per-level item queues (the items k_expand appends for the
-// next level, the representatives k_dedup lists for k_find), with a grid-wide barrier between
-// steps. Launched cooperatively, so every block is resident and every barrier is reached by
+// next level), with a grid-wide barrier between steps. Launched cooperatively, so every block is resident and every barrier is reached by
 // every block: the step sequence depends only on the kernel's arguments, and a body that finds
 // an error flag set returns to the sequence, not out of the kernel.
 // The steps of a pass, in order, as (step << 8 | level): expand per level top-down, the
-// leaves, then per level bottom-up build / clear / dedup / find / add / resolve, the colour
-// steps, and the commit. Every launch form runs this sequence.
+// leaves, then per level bottom-up build and nodes (dedup, find, add), the colour steps, and the
+// commit. Every launch form runs this sequence.
 enum PassStep : uint32_t {
-    ST_EXPAND, ST_LEAF, ST_BUILD, ST_HCLEAR, ST_DEDUP, ST_FIND, ST_ADD, ST_RESOLVE, ST_CSTARTS, ST_CALLOC,
+    ST_EXPAND, ST_LEAF, ST_BUILD, ST_NODES, ST_CSTARTS, ST_CALLOC,
     ST_CTREE, ST_CCOPY, ST_CCOPY_LEAVES, ST_CLEAF, ST_ENC_COUNT, ST_ENC_SCAN, ST_ENC_WRITE, ST_FINISH
 };
 constexpr uint32_t kMaxSteps = 8 * kMaxEditLevels + 8;
@@ -2656,11 +2706,7 @@ static StepList pass_step_list(uint32_t levels, uint32_t ctl, bool colors) {
     add(ST_LEAF, L);
     for (int l = (int)L; l >= 0; --l) {
         if (l < (int)L) add(ST_BUILD, (uint32_t)l);
-        add(ST_HCLEAR, (uint32_t)l);
-        add(ST_DEDUP, (uint32_t)l);
-        add(ST_FIND, (uint32_t)l);
-        add(ST_ADD, (uint32_t)l);
-        add(ST_RESOLVE, (uint32_t)l);
+        add(ST_NODES, (uint32_t)l);
     }
     if (colors) {
         for (uint32_t l = ctl; l < L; ++l) add(ST_CSTARTS, l);
@@ -2686,11 +2732,7 @@ __device__ __forceinline__ void run_step(const EditPass& P, uint32_t code, uint3
             break;
         case ST_LEAF: d_leaf<kSpecial>(P, G); break;
         case ST_BUILD: d_build(P, l, G); break;
-        case ST_HCLEAR: d_hset_clear(P, l, G); break;
-        case ST_DEDUP: d_dedup(P, l, G); break;
-        case ST_FIND: d_find(P, l, G); break;
-        case ST_ADD: d_add(P, l, G); break;
-        case ST_RESOLVE: d_resolve(P, l, G); break;
+        case ST_NODES: d_nodes(P, l, G); break;
         case ST_CSTARTS: d_color_starts(P, l, G); break;
         case ST_CALLOC: d_color_alloc(P, G); break;
         case ST_CTREE: d_color_tree(P, G); break;
@@ -2732,6 +2774,21 @@ __global__ __launch_bounds__(256) void k_pass_block(EditPass P, StepList sl, uin
     }
 }
 
+// Consecutive expand, build and node steps of levels with few items in one workgroup: such a
+// level's launch is shorter than the gap to the next one (13 levels of a brush stroke took 9 us
+// each to expand and 15-20 us each to build and enter).
+__global__ __launch_bounds__(kTopBlock) void k_top(EditPass P, StepList sl, uint32_t first, uint32_t last) {
+    for (uint32_t i = first; i < last; ++i) {
+        const uint32_t l = sl.step[i] & 0xFFu;
+        switch (sl.step[i] >> 8) {
+            case ST_EXPAND: d_expand(P, l, VGrid{0, 1}); break;
+            case ST_BUILD: d_build(P, l, VGrid{0, 1}); break;
+            default: d_nodes(P, l, VGrid{0, 1}); break;
+        }
+        if (i + 1 < last) __syncthreads();
+    }
+}
+
 template <bool kSpecial>
 hd_status launch_persistent(hd_ctx* ctx, EditPass& P, StepList& sl, hipStream_t s) {
     auto* fn = k_pass_persistent<kSpecial>;
@@ -2756,6 +2813,7 @@ static void fill_pass(hd_ctx* ctx, EditPass& P, const EditScratch& S) {
     P.vpool = ctx->vpool;
     P.page_table = ctx->page_table;
     P.bucket_sizes = ctx->bucket_sizes;
+    P.bucket_snap = ctx->bucket_snapshot;
     P.full_nodes = ctx->full_nodes;
     P.pool_top = ctx->counters + 0;
     P.errors = ctx->counters + 1;
@@ -2835,6 +2893,7 @@ static void level_bounds(const EditPass& P, const DevEdit* e, uint32_t n, uint64
 }
 
 constexpr uint32_t kWideEdits = 64, kWideItems = 512;
+constexpr uint32_t kTopItems = 128, kTopNodes = 32, kNodesItems = 1u << 15;
 
 hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hipStream_t s, const uint32_t* dN,
                        bool special, const EditScratch* scratch, const DevEdit* hostEdits) {
@@ -2879,6 +2938,17 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
     const auto small = [&](uint32_t) { return smallPass; };
     // a wavefront per task slot (the task count is on the device), at most 2^18 of them
     const bool bounded = hostEdits && !dN;  // bound[] from the editors' boxes
+    // steps of k_top: a thread per child slot of a level with at most kTopItems items, 16
+    // wavefronts for the nodes of one with at most kTopNodes
+    const auto top_step = [&](uint16_t code) {
+        const uint32_t l = code & 0xFFu;
+        switch (code >> 8) {
+            case ST_EXPAND: return bound[l] <= kTopItems && !((P.wide_levels >> l) & 1u);
+            case ST_BUILD: return bound[l] <= kTopNodes;
+            case ST_NODES: return l < L && bound[l] <= kTopNodes;
+            default: return false;
+        }
+    };
     const auto wideGrid = [](uint64_t blocks) {
         return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(blocks, 1u), 1u << 16);
     };
@@ -2896,6 +2966,16 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
             i = j;
             continue;
         }
+        const uint32_t st = sl.step[i] >> 8;
+        if (bounded) {  // the small levels around the root, together
+            uint32_t j = i;
+            while (j < sl.n && top_step(sl.step[j])) ++j;
+            if (j > i + 1) {
+                k_top<<<1, kTopBlock, 0, s>>>(P, sl, i, j);
+                i = j;
+                continue;
+            }
+        }
         const uint32_t l = sl.step[i] & 0xFFu, gl = grid[l];
         // Grids from the level's item bound by each kernel's unit of work (a thread, or a
         // wavefront, per item or per child slot), up to 2^16 blocks: free wavefronts then take
@@ -2906,7 +2986,7 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
             return bounded ? wideGrid((n + perBlock - 1) / perBlock) : gl;
         };
         const uint64_t b = bound[l];
-        switch (sl.step[i] >> 8) {
+        switch (st) {
             case ST_EXPAND:  // wide: a wavefront per child slot; otherwise a thread per slot
                 if ((P.wide_levels >> l) & 1u) k_expand_wide<<<gl, 256, 0, s>>>(P, l);
                 else k_expand<<<units(8 * b, 256), 256, 0, s>>>(P, l);
@@ -2916,11 +2996,15 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
                 else k_leaf<false><<<units(b, 256), 256, 0, s>>>(P);
                 break;
             case ST_BUILD: k_build<<<units(b, 256), 256, 0, s>>>(P, l); break;  // a thread per item
-            case ST_HCLEAR: k_hset_clear<<<std::min<uint32_t>(gl, 256), 256, 0, s>>>(P, l); break;
-            case ST_DEDUP: k_dedup<<<units(b, 256), 256, 0, s>>>(P, l); break;  // a thread per item
-            case ST_FIND: k_find<<<units(b, 4), 256, 0, s>>>(P, l); break;      // a wavefront per representative
-            case ST_ADD: k_add<<<units(b, 256), 256, 0, s>>>(P, l); break;      // a thread per item
-            case ST_RESOLVE: k_resolve<<<gl, 256, 0, s>>>(P, l); break;
+            case ST_NODES:
+                if (b <= kNodesItems || !bounded) {  // a wavefront per item
+                    k_nodes<<<units(b, 4), 256, 0, s>>>(P, l);
+                } else {
+                    k_dedup<<<units(b, 256), 256, 0, s>>>(P, l);  // a thread per item
+                    k_find<<<units(b, 4), 256, 0, s>>>(P, l);     // a wavefront per representative
+                    k_add<<<units(b, 256), 256, 0, s>>>(P, l);    // a thread per representative
+                }
+                break;
             case ST_CSTARTS: k_color_starts<<<units(8 * b, 256), 256, 0, s>>>(P, l); break;  // a thread per slot
             case ST_CALLOC: k_color_alloc<<<gl, 256, 0, s>>>(P); break;
             case ST_CTREE: k_color_tree<<<gridMax, 256, 0, s>>>(P); break;
