@@ -1114,7 +1114,31 @@ __device__ __forceinline__ void d_dedup(const EditPass& P, uint32_t l, VGrid G) 
     const uint32_t hmask = hset_slots(P, l) - 1;
     for (uint32_t b0 = G.block * blockDim.x; b0 < n; b0 += G.nblocks * blockDim.x) {
         const uint32_t i = b0 + threadIdx.x;
-        const bool isRep = i < n && I.state[i] == kStatePending && dedup_item(P, I, i, hmask);
+        bool pending = i < n && I.state[i] == kStatePending;
+        // Items of one wavefront that share a content (neighbours often do: full leaves, planes)
+        // enter the set once, through the first of them: thousands of threads that see one slot
+        // still empty would queue their CAS on it (196 us for a level of a pass of 48 editors).
+        const uint32_t h = pending ? I.hash[i] : 0u;
+        bool isRep = false;
+        for (uint32_t round = 0; round < 4; ++round) {
+            const uint64_t m = __ballot(pending);
+            if (!m) break;
+            const uint32_t first = (uint32_t)__ffsll((long long)m) - 1u;
+            const uint32_t lead = __shfl(i, first, 64), lh = __shfl(h, first, 64);
+            const bool same = pending && i != lead && h == lh && same_content(I, i, lead);
+            uint32_t rep = 0;
+            if (pending && i == lead) {
+                isRep = dedup_item(P, I, i, hmask);
+                rep = isRep ? i : I.nidx[i];
+            }
+            rep = __shfl(rep, first, 64);
+            if (same) {
+                I.nidx[i] = rep;
+                I.state[i] = kStateDuplicate;
+            }
+            pending = pending && i != lead && !same;
+        }
+        if (pending) isRep = dedup_item(P, I, i, hmask);
         const uint32_t at = block_alloc32(sAlloc, &P.find_count[l], isRep ? 1u : 0u);
         if (isRep) I.nstart[at] = i;
     }
@@ -1477,16 +1501,20 @@ __device__ __forceinline__ uint64_t old_color(const EditPass& P, uint32_t mode, 
 constexpr uint64_t kUniformChunk = 1ull << 63;
 constexpr uint64_t kColorKey = 0x0000FF00FFFFFFFFull;
 
-// keep / full slots of interior items at levels >= ctl: one wavefront per slot. Whole chunks
-// of one colour become markers; the partial chunks at either end are written as colours.
-__device__ __forceinline__ void d_color_copy(const EditPass& P, uint32_t l, VGrid G) {
+// keep / full slots of interior items at levels >= ctl: 2^lp wavefronts per slot, each a run
+// of whole chunks (a launch with few slots lasted as long as its largest: one wavefront copies
+// 64 colours a step, 109 us for a slot of a 32^3 subtree). Whole chunks of one colour become
+// markers; the partial chunks at either end are written as colours.
+constexpr uint32_t kPieceChunks = 4;  // fewer chunks than this stay in one piece
+__device__ __forceinline__ void d_color_copy(const EditPass& P, uint32_t l, uint32_t lp, VGrid G) {
     const uint32_t n = min(P.count[l], P.cap[l]);
     if (*P.errors) return;
     const Items I = P.items[l];
     const Items T = P.items[P.ctl];
     const uint32_t lane = threadIdx.x & 63u;
-    for (uint32_t w = wave_index(G); w < n * 8; w += wave_count(G)) {
-        const uint32_t i = w >> 3, slot = w;
+    const uint32_t pieces = 1u << lp;
+    for (uint64_t w = wave_index(G); w < ((uint64_t)n * 8) << lp; w += wave_count(G)) {
+        const uint32_t slot = (uint32_t)(w >> lp), piece = (uint32_t)w & (pieces - 1u), i = slot >> 3;
         const uint32_t kind = I.ckind[slot];
         if (kind != KIND_KEEP && kind != KIND_FULL) continue;
         const uint32_t cnt = I.cnew[slot];
@@ -1497,6 +1525,7 @@ __device__ __forceinline__ void d_color_copy(const EditPass& P, uint32_t l, VGri
         uint64_t* marks = P.cmarks + cb / 64;
         const uint32_t cs = I.cstart[slot], ce = cs + cnt;
         if (kind == KIND_FULL) {
+            if (piece) continue;  // a marker per chunk, 64 at a time
             const uint64_t col = pack_color(I.ccolor[slot], 0, 0);
             const uint32_t a = min((cs + 63u) & ~63u, ce), b = max(ce & ~63u, a);
             for (uint32_t k = cs + lane; k < a; k += 64) out[k] = col;
@@ -1507,7 +1536,10 @@ __device__ __forceinline__ void d_color_copy(const EditPass& P, uint32_t l, VGri
             const uint32_t mode = I.cmode[i], mv = I.cmodeval[i];
             const uint64_t os = (uint64_t)I.costart[slot] - cs;
             uint32_t pos = ~0u;  // block of the colour before the chunk (decoded runs)
-            for (uint32_t k0 = cs & ~63u; k0 < ce; k0 += 64) {
+            const uint32_t ch0 = cs / 64u, chunks = (ce + 63u) / 64u - ch0;
+            const uint32_t per = max((chunks + pieces - 1) >> lp, kPieceChunks);
+            const uint32_t kEnd = (ch0 + min((piece + 1) * per, chunks)) * 64u;
+            for (uint32_t k0 = (ch0 + piece * per) * 64u; k0 < kEnd; k0 += 64) {
                 const uint32_t k = k0 + lane;
                 const bool in = k >= cs && k < ce;
                 uint64_t col;
@@ -1529,8 +1561,8 @@ __device__ __forceinline__ void d_color_copy(const EditPass& P, uint32_t l, VGri
         }
     }
 }
-__global__ __launch_bounds__(256) void k_color_copy(EditPass P, uint32_t l) {
-    d_color_copy(P, l, VGrid{blockIdx.x, gridDim.x});
+__global__ __launch_bounds__(256) void k_color_copy(EditPass P, uint32_t l, uint32_t lp) {
+    d_color_copy(P, l, lp, VGrid{blockIdx.x, gridDim.x});
 }
 
 // keep / full slots of the items at level L - 1 (their children are leaves: at most 64 colours
@@ -2192,8 +2224,10 @@ __global__ __launch_bounds__(kEncBlock) void k_enc_count(EditPass P) { d_enc_cou
 // and macro records are written, and zeros into the weight words where a segment ends inside a
 // word. A lane per task, and the whole wavefront for a task of many segments; one atomic on the
 // arena's top per wavefront (one per task held a pass of 700,000 tasks for 6.1 ms: one address
-// takes about 155 M atomics a second).
+// takes about 155 M atomics a second). A wavefront takes as many tasks as there are per wavefront;
+// with few, every task is the whole wavefront's (46 -> 11 us in a pass of 48 editors).
 constexpr uint32_t kLaneSegs = 8;  // segments a lane walks on its own
+constexpr uint32_t kScanBlocks = 256;
 __device__ __forceinline__ void enc_scan_marks(uint64_t* macro, uint32_t* weights, uint32_t k, uint2 v) {
     constexpr uint32_t kPerMacro = 16384u / kSegColors;
     if (k % kPerMacro == 0) {
@@ -2208,9 +2242,11 @@ __device__ __forceinline__ void d_enc_scan(const EditPass& P, VGrid G) {
     const uint32_t n = min(P.count[ctl], P.cap[ctl]);
     const Items T = P.items[ctl];
     const uint32_t lane = threadIdx.x & 63u;
-    for (uint32_t t0 = G.block * blockDim.x + (threadIdx.x & ~63u); t0 < n; t0 += G.nblocks * blockDim.x) {
+    const uint32_t waves = wave_count(G), run = min(64u, (n + waves - 1) / waves);
+    const uint32_t laneSegs = run > 8 ? kLaneSegs : 0u;
+    for (uint32_t t0 = wave_index(G) * run; t0 < n; t0 += waves * run) {
         const uint32_t t = t0 + lane;
-        uint32_t cnt = t < n ? T.ncount[t] : 0u;
+        uint32_t cnt = lane < run && t < n ? T.ncount[t] : 0u;
         const uint32_t nMacro = (cnt + 16383u) / 16384u;
         if (nMacro > 160) {  // more than 160 * 16384 colours in one subtree
             set_error(P.errors, ERR_LEAF_SIZE);
@@ -2218,8 +2254,8 @@ __device__ __forceinline__ void d_enc_scan(const EditPass& P, VGrid G) {
         }
         const uint32_t nSeg = (cnt + kSegColors - 1u) / kSegColors, seg0 = cnt ? T.hash[t] : 0u;
         uint32_t nBlocks = 0, nBits = 0;
-        const uint64_t big = __ballot(nSeg > kLaneSegs);
-        if (nSeg <= kLaneSegs)
+        const uint64_t big = __ballot(nSeg > laneSegs);
+        if (nSeg <= laneSegs)
             for (uint32_t k = 0; k < nSeg; ++k) {
                 const uint2 v = P.seg_out[seg0 + k];
                 P.seg_out[seg0 + k] = make_uint2(nBlocks, nBits);
@@ -2252,7 +2288,7 @@ __device__ __forceinline__ void d_enc_scan(const EditPass& P, VGrid G) {
         uint64_t* macro = P.arena + base + nBlocks;
         uint32_t* weights = reinterpret_cast<uint32_t*>(macro + 2 * nMacro);
         if (ok) {
-            if (nSeg <= kLaneSegs)
+            if (nSeg <= laneSegs)
                 for (uint32_t k = 0; k < nSeg; ++k) enc_scan_marks(macro, weights, k, P.seg_out[seg0 + k]);
             if (nBits & 31u) weights[nBits >> 5] = 0u;
             weights[nWeights] = 0u;  // padding read by the 16-bit window
@@ -2736,7 +2772,7 @@ __device__ __forceinline__ void run_step(const EditPass& P, uint32_t code, uint3
         case ST_CSTARTS: d_color_starts(P, l, G); break;
         case ST_CALLOC: d_color_alloc(P, G); break;
         case ST_CTREE: d_color_tree(P, G); break;
-        case ST_CCOPY: d_color_copy(P, l, G); break;
+        case ST_CCOPY: d_color_copy(P, l, 0, G); break;
         case ST_CCOPY_LEAVES: d_color_copy_leaves(P, G); break;
         case ST_CLEAF:
             if constexpr (kSpecial) d_color_leaf(P, G);
@@ -2892,7 +2928,7 @@ static void level_bounds(const EditPass& P, const DevEdit* e, uint32_t n, uint64
     }
 }
 
-constexpr uint32_t kWideEdits = 64, kWideItems = 512;
+constexpr uint32_t kWideEdits = 8, kWideItems = 512;
 constexpr uint32_t kTopItems = 128, kTopNodes = 32, kNodesItems = 1u << 15;
 
 hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hipStream_t s, const uint32_t* dN,
@@ -3009,14 +3045,18 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
             case ST_CALLOC: k_color_alloc<<<gl, 256, 0, s>>>(P); break;
             case ST_CTREE: k_color_tree<<<gridMax, 256, 0, s>>>(P); break;
             // colour copies: a wavefront per slot (per item at the leaf parents)
-            case ST_CCOPY: k_color_copy<<<units(8 * b, 4), 256, 0, s>>>(P, l); break;
+            case ST_CCOPY: {
+                const uint32_t lp = bounded && b <= 4096 ? 3u : 0u;
+                k_color_copy<<<units((8 * b) << lp, 4), 256, 0, s>>>(P, l, lp);
+                break;
+            }
             case ST_CCOPY_LEAVES: k_color_copy_leaves<<<units(b, 4), 256, 0, s>>>(P); break;
             case ST_CLEAF:  // special: a wavefront per item; otherwise a thread per item
                 if (special) k_color_leaf<<<gl, 256, 0, s>>>(P);
                 else k_color_leaf_items<<<units(b, 256), 256, 0, s>>>(P);
                 break;
             case ST_ENC_COUNT: k_enc_count<<<segBlocks, kEncBlock, 0, s>>>(P); break;
-            case ST_ENC_SCAN: k_enc_scan<<<units(b, 256), kEncBlock, 0, s>>>(P); break;  // a thread per task
+            case ST_ENC_SCAN: k_enc_scan<<<std::min<uint32_t>(units(b, 4), kScanBlocks), kEncBlock, 0, s>>>(P); break;
             case ST_ENC_WRITE: k_enc_write<<<segBlocks, kEncBlock, 0, s>>>(P); break;
             default: k_finish<<<1, 64, 0, s>>>(P, ctx->d_root); break;
         }
