@@ -1147,6 +1147,30 @@ __global__ __launch_bounds__(256) void k_dedup(EditPass P, uint32_t l) {
     d_dedup(P, l, VGrid{blockIdx.x, gridDim.x});
 }
 
+// Does the walk node by node from word w of a bucket (a page start) come to word c? Called by
+// the whole wavefront with the same arguments. The words up to c are loaded 256 at a time and
+// the walk reads the nodes' lengths out of the lanes: one load latency where following the
+// headers in memory took one per node (up to 60 a page).
+__device__ __forceinline__ bool on_page_walk(const uint32_t* __restrict__ words, uint32_t w, uint32_t c) {
+    const uint32_t lane = threadIdx.x & 63u;
+    w = __builtin_amdgcn_readfirstlane(w);
+    c = __builtin_amdgcn_readfirstlane(c);
+    for (uint32_t q = w; q < c; q += 256) {
+        uint32_t len[4];
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t pos = q + 64 * k + lane;
+            len[k] = 1u + (uint32_t)__popc(pos < c ? words[pos] & 0xFFu : 0u);
+        }
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t q0 = q + 64 * k, end = min(q0 + 64u, c);
+            while (w < end) w += (uint32_t)__builtin_amdgcn_readlane((int)len[k], (int)(w - q0));
+        }
+    }
+    return w == c;
+}
+
 // The wavefront scans the bucket of item i for an identical node (any word position inside the
 // bucket's used size whose words equal the node and that does not cross a page boundary holds
 // the same node content); its position in the bucket, or ~0. The size is the bucket's before the
@@ -1214,9 +1238,7 @@ __device__ __forceinline__ uint32_t find_node(const EditPass& P, const Items& I,
             uint64_t b = __ballot(hit);
             while (b) {
                 const uint32_t c = p0 + (uint32_t)__ffsll((long long)b) - 1;  // wave-uniform
-                uint32_t w = c - c % ps;
-                while (w < c) w += 1u + __popc(P.vpool[base + w] & 0xFFu);  // advances >= 1 word
-                if (w == c) {
+                if (on_page_walk(P.vpool + base, c - c % ps, c)) {
                     found = c;
                     break;
                 }
