@@ -43,7 +43,7 @@ namespace {
 
 constexpr uint32_t KIND_KEEP = 0, KIND_EMPTY = 1, KIND_FULL = 2, KIND_ITEM = 3;
 constexpr uint32_t kGrid = 2048;  // blocks of grid-stride kernels
-constexpr uint32_t kTopBlock = 1024;  // threads of the workgroup that runs a pass's small levels (k_top)
+constexpr uint32_t kTopBlock = 1024;  // threads of the workgroup that runs a pass's small levels
 
 // Wave-strided loops (one work item per wavefront): the index is made wave-uniform so the
 // compiler keeps it in a scalar register and loads the item's fields through the scalar cache.
@@ -546,25 +546,22 @@ __device__ __forceinline__ SlotRefs slot_refs(const EditPass& P, const Items& I,
     return r;
 }
 
+// old voxel count of a slot's effective old child (colour offsets, "keep" counts)
+__device__ __forceinline__ uint32_t slot_old_count(const EditPass& P, uint32_t l, const SlotRefs& r) {
+    if (l + 1 < P.ctl || r.childOld == kInvalidNode) return 0;
+    if (l + 1 == P.levels - 2) return __popcll(*reinterpret_cast<const uint64_t*>(P.vpool + r.childOld));
+    return P.vpool[r.childOld] >> 8;
+}
+
 // Classifies a child slot from its filtered edits (m edits touch it; the last full / empty
 // cover among them is the lastCover-th, ~0 for none): keep, full, empty or a child item.
 // Writes the slot's corig / cold / cval / cnew / ccolor; coveredVoxels is the voxel count of a
 // full / empty early exit.
 __device__ __forceinline__ uint32_t slot_classify(const EditPass& P, const Items& I, uint32_t l, uint32_t slot,
-                                                  uint32_t depth, const SlotRefs& r, uint32_t m, uint32_t lastCover,
-                                                  uint32_t coverKind, uint32_t coverColor,
+                                                  uint32_t depth, const SlotRefs& r, uint32_t oldCount, uint32_t m,
+                                                  uint32_t lastCover, uint32_t coverKind, uint32_t coverColor,
                                                   unsigned long long& coveredVoxels) {
-    const uint32_t L = P.levels - 2, ctl = P.ctl;
-    // old voxel count of the effective old child (colour offsets, "keep" counts)
-    uint32_t oldCount = 0;
-    if (l + 1 >= ctl && r.childOld != kInvalidNode) {
-        if (l + 1 == L) {
-            const uint64_t lf = *reinterpret_cast<const uint64_t*>(P.vpool + r.childOld);
-            oldCount = __popcll(lf);
-        } else {
-            oldCount = P.vpool[r.childOld] >> 8;
-        }
-    }
+    const uint32_t ctl = P.ctl;
     I.corig[slot] = r.childOrig;
     I.cold[slot] = oldCount;
     const bool covered = lastCover != ~0u;
@@ -592,11 +589,19 @@ __device__ __forceinline__ uint32_t slot_classify(const EditPass& P, const Items
     return kind;
 }
 
-// child item ci of a slot, all but its edit list (rest words from eo)
+// What a child item takes from its parent: the colour mode of its old colours, the colour node or
+// task (aux), and, for a covered child, the covering editor's colour.
+struct ParentRefs {
+    uint32_t cmode, cmodeval, aux;
+};
+
+// child item ci of a slot, all but its edit list (rest words from eo); its old node, colour mode
+// and aux come back for a caller that goes on with it
 __device__ __forceinline__ void slot_child_item(const EditPass& P, const Items& I, const Items& C, uint32_t l,
                                                 uint32_t i, uint32_t c, uint32_t slot, uint32_t ci, uint32_t eo,
                                                 uint32_t rest, const SlotRefs& r, uint32_t lastCover,
-                                                uint32_t coverKind) {
+                                                uint32_t coverKind, uint32_t coverColor, const ParentRefs& par,
+                                                uint32_t& childOld, ParentRefs& child) {
     const uint32_t ctl = P.ctl;
     C.px[ci] = r.cx;
     C.py[ci] = r.cy;
@@ -606,26 +611,25 @@ __device__ __forceinline__ void slot_child_item(const EditPass& P, const Items& 
     C.slot[ci] = (uint8_t)c;
     C.estart[ci] = eo;
     C.ecount[ci] = rest;
+    childOld = r.childOld;
+    child = par;
     if (lastCover != ~0u) {
-        C.old_[ci] = coverKind == 1 ? P.full_nodes[l + 1] : kInvalidNode;
-        C.cmode[ci] = coverKind == 1 ? 1u : 2u;  // old colours: single colour / none
-        C.cmodeval[ci] = I.ccolor[slot];
-    } else {
-        C.old_[ci] = r.childOld;
-        C.cmode[ci] = I.cmode[i];
-        C.cmodeval[ci] = I.cmodeval[i];
+        childOld = coverKind == 1 ? P.full_nodes[l + 1] : kInvalidNode;
+        child.cmode = coverKind == 1 ? 1u : 2u;  // old colours: single colour / none
+        child.cmodeval = coverColor;
     }
+    C.old_[ci] = childOld;
+    C.cmode[ci] = child.cmode;
+    C.cmodeval[ci] = child.cmodeval;
     // colour tree: node of the child (levels < ctl), or the subtree's leaf handle / task
-    const uint32_t cn = I.aux[i];
+    const uint32_t cn = par.aux;
     if (l + 1 < ctl) {
-        C.aux[ci] = (l == 0 || cn > 0) ? P.cnodes[cn + c] : 0u;
+        child.aux = (l == 0 || cn > 0) ? P.cnodes[cn + c] : 0u;
     } else if (l + 1 == ctl) {
-        C.aux[ci] = ci;  // task id = own index at level ctl
-        const uint32_t h = (l == 0 || cn > 0) ? P.cnodes[cn + c] : 0u;
-        C.handle[ci] = h;
-    } else {
-        C.aux[ci] = cn;  // task of the ancestor at level ctl
-    }
+        child.aux = ci;  // task id = own index at level ctl
+        C.handle[ci] = (l == 0 || cn > 0) ? P.cnodes[cn + c] : 0u;
+    }  // below: task of the ancestor at level ctl
+    C.aux[ci] = child.aux;
     I.cval[slot] = ci;
 }
 
@@ -653,6 +657,7 @@ __device__ __forceinline__ void d_expand(const EditPass& P, uint32_t l, VGrid G)
         const uint32_t i = (uint32_t)(t >> 3), c = (uint32_t)(t & 7u);
         const uint32_t slot = i * 8 + c;
         uint32_t kind = KIND_KEEP, m = 0, lastCover = ~0u, coverKind = 0, es = 0, ec = 0;
+        uint32_t coverColor = 0;
         uint64_t touch = 0;
         SlotRefs r{};
         unsigned long long coveredVoxels = 0;
@@ -662,7 +667,6 @@ __device__ __forceinline__ void d_expand(const EditPass& P, uint32_t l, VGrid G)
             ec = I.ecount[i];
             // filter the edit list, two edit heads in flight; remember the last cover at levels
             // >= ctl (and its colour) and which of the first 64 edits touch
-            uint32_t coverColor = 0;
             for (uint32_t k = 0; k < ec; k += 2) {
                 const bool two = k + 1 < ec;
                 const uint32_t e0 = P.elist[l][es + k];
@@ -685,7 +689,8 @@ __device__ __forceinline__ void d_expand(const EditPass& P, uint32_t l, VGrid G)
                     m++;
                 }
             }
-            kind = slot_classify(P, I, l, slot, depth, r, m, lastCover, coverKind, coverColor, coveredVoxels);
+            kind = slot_classify(P, I, l, slot, depth, r, slot_old_count(P, l, r), m, lastCover, coverKind, coverColor,
+                                 coveredVoxels);
         }
         const bool isItem = active && kind == KIND_ITEM;
         const uint32_t rest = isItem ? (lastCover == ~0u ? m : m - lastCover - 1) : 0u;
@@ -709,7 +714,10 @@ __device__ __forceinline__ void d_expand(const EditPass& P, uint32_t l, VGrid G)
                 if (lastCover == ~0u || q > lastCover) P.elist[l + 1][eo + w++] = ei;
                 q++;
             }
-            slot_child_item(P, I, C, l, i, c, slot, ci, eo, rest, r, lastCover, coverKind);
+            uint32_t childOld;
+            ParentRefs child;
+            slot_child_item(P, I, C, l, i, c, slot, ci, eo, rest, r, lastCover, coverKind, coverColor,
+                            ParentRefs{I.cmode[i], I.cmodeval[i], I.aux[i]}, childOld, child);
         }
         I.ckind[slot] = (uint8_t)kind;
     }
@@ -768,7 +776,8 @@ __device__ __forceinline__ void d_expand_wide(const EditPass& P, uint32_t l, VGr
         unsigned long long coveredVoxels = 0;
         uint32_t kind = 0;
         if (lane == 0)
-            kind = slot_classify(P, I, l, (uint32_t)slot, depth, r, m, lastCover, coverKind, coverColor, coveredVoxels);
+            kind = slot_classify(P, I, l, (uint32_t)slot, depth, r, slot_old_count(P, l, r), m, lastCover, coverKind,
+                                 coverColor, coveredVoxels);
         kind = __shfl(kind, 0, 64);
         if (P.single_edit && lane == 0 && coveredVoxels) atomicAdd(P.stat_voxels, coveredVoxels);
         if (kind == KIND_ITEM) {
@@ -804,7 +813,12 @@ __device__ __forceinline__ void d_expand_wide(const EditPass& P, uint32_t l, VGr
                 w += (uint32_t)__popcll(E);
                 q += (uint32_t)__popcll(T);
             }
-            if (lane == 0) slot_child_item(P, I, C, l, i, c, (uint32_t)slot, ci, eo, rest, r, lastCover, coverKind);
+            if (lane == 0) {
+                uint32_t childOld;
+                ParentRefs child;
+                slot_child_item(P, I, C, l, i, c, (uint32_t)slot, ci, eo, rest, r, lastCover, coverKind, coverColor,
+                                ParentRefs{I.cmode[i], I.cmodeval[i], I.aux[i]}, childOld, child);
+            }
         }
         if (lane == 0) I.ckind[slot] = (uint8_t)kind;
     }
@@ -1171,26 +1185,53 @@ __device__ __forceinline__ bool on_page_walk(const uint32_t* __restrict__ words,
     return w == c;
 }
 
-// The wavefront scans the bucket of item i for an identical node (any word position inside the
+// A node's content: its words (wave-uniform where a wavefront works on one node), length and hash.
+struct NodeWords {
+    uint32_t w[9];
+    uint32_t n, hash;
+};
+// hash_words over words held in registers (no indexed access to them)
+__device__ __forceinline__ uint32_t node_hash(const NodeWords& c) {
+    uint32_t h = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < 9; ++i) {
+        if (i >= c.n) break;
+        uint32_t k = c.w[i] * 0xcc9e2d51u;
+        k = (k << 15) | (k >> 17);
+        k *= 0x1b873593u;
+        h ^= k;
+        h = (h << 13) | (h >> 19);
+        h = h * 5u + 0xe6546b64u;
+    }
+    return fmix32(h ^ c.n);
+}
+__device__ __forceinline__ NodeWords item_words(const Items& I, uint32_t i) {
+    NodeWords c;
+#pragma unroll
+    for (uint32_t k = 0; k < 9; ++k) c.w[k] = I.cont[i * 9 + k];  // words past the length are not used
+    c.n = I.clen[i];
+    c.hash = I.hash[i];
+    return c;
+}
+
+// The wavefront scans a node's bucket for an identical node (any word position inside the
 // bucket's used size whose words equal the node and that does not cross a page boundary holds
-// the same node content); its position in the bucket, or ~0. The size is the bucket's before the
-// pass: what the pass appends to a level are contents that no other item of the level has, so
-// they need not be seen, and other wavefronts may be writing them.
-__device__ __forceinline__ uint32_t find_node(const EditPass& P, const Items& I, uint32_t l, uint32_t i,
-                                              uint64_t& scanBytes) {
+// the same node content); its address, or ~0. The size is the bucket's before the pass: what the
+// pass appends to a level are contents that no other item of the level has, so they need not be
+// seen, and other wavefronts may be writing them.
+__device__ __forceinline__ uint32_t find_node(const EditPass& P, uint32_t l, const NodeWords& c, uint64_t& scanBytes) {
     const Geom& g = P.g;
     const uint32_t lane = threadIdx.x & 63u;
     const bool leafLevel = l == g.leaf_level();
-    const uint32_t bucket = g.bucket_from_hash(l, I.hash[i]);
+    const uint32_t bucket = g.bucket_from_hash(l, c.hash);
     const uint32_t base = g.make_ptr(l, bucket, 0);
-    const uint32_t bs = P.bucket_snap[g.bucket_global(l, bucket)];
-    const uint32_t nw = I.clen[i];
     uint32_t found = ~0u;
     if (leafLevel && P.leaf_tags) {
+        const uint32_t bs = P.bucket_snap[g.bucket_global(l, bucket)];
         // slots (2 words each) whose tag byte matches, lowest first, confirmed on the leaf;
         // 4 tags per lane, 256 slots per wavefront step
-        const uint64_t key = (uint64_t)I.cont[i * 9] | ((uint64_t)I.cont[i * 9 + 1] << 32);
-        const uint32_t want = I.hash[i] >> 24, nslots = bs / 2;
+        const uint64_t key = (uint64_t)c.w[0] | ((uint64_t)c.w[1] << 32);
+        const uint32_t want = c.hash >> 24, nslots = bs / 2;
         const uint8_t* tags = P.leaf_tags + (uint64_t)bucket * (g.bucket_size(l) / 2);
         for (uint32_t s0 = 0; s0 < nslots && found == ~0u; s0 += 256) {
             const uint32_t sl = s0 + 4 * lane;
@@ -1208,7 +1249,8 @@ __device__ __forceinline__ uint32_t find_node(const EditPass& P, const Items& I,
             if (b) found = 2u * (uint32_t)__shfl((int)hitSlot, __ffsll((long long)b) - 1, 64);
         }
     } else if (leafLevel) {
-        const uint64_t key = (uint64_t)I.cont[i * 9] | ((uint64_t)I.cont[i * 9 + 1] << 32);
+        const uint32_t bs = P.bucket_snap[g.bucket_global(l, bucket)];
+        const uint64_t key = (uint64_t)c.w[0] | ((uint64_t)c.w[1] << 32);
         for (uint32_t p0 = 0; p0 < bs && found == ~0u; p0 += 128) {
             const uint32_t pos = p0 + 2 * lane;
             if (pos + 2 <= bs) scanBytes += 8;
@@ -1220,26 +1262,28 @@ __device__ __forceinline__ uint32_t find_node(const EditPass& P, const Items& I,
         // The reference walks node by node from each page start and compares only nodes
         // with start + n < min(bucketSize, pageEnd). The wave compares all positions at
         // once, then confirms the first candidate lies on that walk.
-        const uint32_t h0 = I.cont[i * 9];
         const uint32_t ps = g.page_size;
-        for (uint32_t p0 = 0; p0 + nw < bs && found == ~0u; p0 += 64) {
+        uint32_t word = lane < g.bucket_size(l) ? P.vpool[base + lane] : 0u;  // in flight with the size
+        const uint32_t bs = P.bucket_snap[g.bucket_global(l, bucket)];
+        for (uint32_t p0 = 0; p0 + c.n < bs && found == ~0u; p0 += 64) {
             const uint32_t pos = p0 + lane;
             const uint32_t pageEnd = min(bs, pos - pos % ps + ps);
             if (pos < bs) scanBytes += 4;
-            bool hit = pos + nw < pageEnd && P.vpool[base + pos] == h0;
-            if (hit)
-                for (uint32_t k = 1; k < nw; ++k) {
-                    scanBytes += 4;
-                    if (P.vpool[base + pos + k] != I.cont[i * 9 + k]) {
-                        hit = false;
-                        break;
+            if (p0 != 0) word = pos < bs ? P.vpool[base + pos] : 0u;
+            bool hit = pos + c.n < pageEnd && word == c.w[0];
+            if (hit) {
+#pragma unroll
+                for (uint32_t k = 1; k < 9; ++k)
+                    if (k < c.n && hit) {
+                        scanBytes += 4;
+                        hit = P.vpool[base + pos + k] == c.w[k];
                     }
-                }
+            }
             uint64_t b = __ballot(hit);
             while (b) {
-                const uint32_t c = p0 + (uint32_t)__ffsll((long long)b) - 1;  // wave-uniform
-                if (on_page_walk(P.vpool + base, c - c % ps, c)) {
-                    found = c;
+                const uint32_t at = p0 + (uint32_t)__ffsll((long long)b) - 1;  // wave-uniform
+                if (on_page_walk(P.vpool + base, at - at % ps, at)) {
+                    found = at;
                     break;
                 }
                 b &= b - 1;
@@ -1261,50 +1305,51 @@ __device__ bool alloc_page(const EditPass& P, uint32_t page) {
     return true;
 }
 
-// Appends item i to its bucket (one lane): space by a CAS on the bucket size, with the page
-// padding rule; the words added.
-__device__ __forceinline__ uint32_t append_node(const EditPass& P, const Items& I, uint32_t l, uint32_t i) {
+// Appends a node to its bucket (one lane): space by a CAS on the bucket size, with the page
+// padding rule; its address, or ~0 with an error set.
+__device__ __forceinline__ uint32_t append_node(const EditPass& P, uint32_t l, const NodeWords& c) {
     const Geom& g = P.g;
     const uint32_t ps = g.page_size;
-    const uint32_t nw = I.clen[i];
-    const uint32_t bucket = g.bucket_from_hash(l, I.hash[i]);
+    const uint32_t bucket = g.bucket_from_hash(l, c.hash);
     uint32_t* bsPtr = &P.bucket_sizes[g.bucket_global(l, bucket)];
     const uint32_t cap = g.bucket_size(l);
     uint32_t start;
     uint32_t cur = *reinterpret_cast<volatile uint32_t*>(bsPtr);
     for (;;) {
         const uint32_t left = ps - cur % ps;
-        start = (left == ps || left < nw) ? (left == ps ? cur : cur + left) : cur;
-        if (start + nw > cap) {
+        start = (left == ps || left < c.n) ? (left == ps ? cur : cur + left) : cur;
+        if (start + c.n > cap) {
             set_error(P.errors, ERR_BUCKET);
-            return 0;
+            return ~0u;
         }
-        const uint32_t prev = atomicCAS(bsPtr, cur, start + nw);
+        const uint32_t prev = atomicCAS(bsPtr, cur, start + c.n);
         if (prev == cur) break;
         cur = prev;
     }
     const uint32_t va = g.make_ptr(l, bucket, start);
-    if (start % ps == 0 && !alloc_page(P, va / ps)) return 0;
-    for (uint32_t k = 0; k < nw; ++k) P.vpool[va + k] = I.cont[i * 9 + k];
+    if (start % ps == 0 && !alloc_page(P, va / ps)) return ~0u;
+#pragma unroll
+    for (uint32_t k = 0; k < 9; ++k)
+        if (k < c.n) P.vpool[va + k] = c.w[k];
     if (P.leaf_tags && l == g.leaf_level())
-        P.leaf_tags[(uint64_t)bucket * (cap / 2) + start / 2] = (uint8_t)(I.hash[i] >> 24);
-    I.nidx[i] = va;
-    return nw;
+        P.leaf_tags[(uint64_t)bucket * (cap / 2) + start / 2] = (uint8_t)(c.hash >> 24);
+    return va;
 }
 
 // One representative by a wavefront: found in the table, or appended to it. The words added
 // (in lane 0).
 __device__ __forceinline__ uint32_t find_or_add(const EditPass& P, const Items& I, uint32_t l, uint32_t i,
                                                 uint64_t& scanBytes) {
-    const uint32_t va = find_node(P, I, l, i, scanBytes);
-    uint32_t added = 0;
+    const NodeWords c = item_words(I, i);
+    uint32_t va = find_node(P, l, c, scanBytes), added = 0;
     if ((threadIdx.x & 63u) == 0) {
         if (va != ~0u) {
-            I.nidx[i] = va;
             I.state[i] = kStateFound;
         } else {
-            added = append_node(P, I, l, i);
+            va = append_node(P, l, c);
+            added = va != ~0u ? c.n : 0u;
         }
+        if (va != ~0u) I.nidx[i] = va;
     }
     return added;
 }
@@ -1317,7 +1362,7 @@ __device__ __forceinline__ void d_find(const EditPass& P, uint32_t l, VGrid G) {
     uint64_t scanBytes = 0;  // bucket bytes this lane read (measurement)
     for (uint32_t r = wave_index(G); r < nReps; r += wave_count(G)) {
         const uint32_t i = I.nstart[r];
-        const uint32_t va = find_node(P, I, l, i, scanBytes);
+        const uint32_t va = find_node(P, l, item_words(I, i), scanBytes);
         if ((threadIdx.x & 63u) == 0 && va != ~0u) {
             I.nidx[i] = va;
             I.state[i] = kStateFound;
@@ -1340,7 +1385,14 @@ __device__ __forceinline__ void d_add(const EditPass& P, uint32_t l, VGrid G) {
         uint32_t added = 0;
         if (r < nReps) {
             const uint32_t i = I.nstart[r];
-            if (I.state[i] == kStatePending) added = append_node(P, I, l, i);
+            if (I.state[i] == kStatePending) {
+                const NodeWords c = item_words(I, i);
+                const uint32_t va = append_node(P, l, c);
+                if (va != ~0u) {
+                    I.nidx[i] = va;
+                    added = c.n;
+                }
+            }
         }
         wave_add64(P.stat_new_words, added);
     }
@@ -2832,19 +2884,348 @@ __global__ __launch_bounds__(256) void k_pass_block(EditPass P, StepList sl, uin
     }
 }
 
-// Consecutive expand, build and node steps of levels with few items in one workgroup: such a
-// level's launch is shorter than the gap to the next one (13 levels of a brush stroke took 9 us
-// each to expand and 15-20 us each to build and enter).
-__global__ __launch_bounds__(kTopBlock) void k_top(EditPass P, StepList sl, uint32_t first, uint32_t last) {
-    for (uint32_t i = first; i < last; ++i) {
-        const uint32_t l = sl.step[i] & 0xFFu;
-        switch (sl.step[i] >> 8) {
-            case ST_EXPAND: d_expand(P, l, VGrid{0, 1}); break;
-            case ST_BUILD: d_build(P, l, VGrid{0, 1}); break;
-            default: d_nodes(P, l, VGrid{0, 1}); break;
-        }
-        if (i + 1 < last) __syncthreads();
+// ---------------------------------------------------------------------------------------------
+// the small levels around the root, in one workgroup
+// ---------------------------------------------------------------------------------------------
+// A level of few items costs its launch and the latency of what it reads one after another. Here
+// a workgroup goes through consecutive levels with the items in LDS: between two levels only the
+// tree's own words (a child pointer, the child's header) are waited for, not the item arrays,
+// which are written for the later steps on the way. 13 levels of a brush stroke: expand 108 -> 35
+// us, build and nodes 110 -> 50 us (as steps over the item arrays in one workgroup, and 9 and
+// 15-20 us a level as launches).
+constexpr uint32_t kTopCap = 256;    // items of a level held in LDS
+constexpr uint32_t kTopEdits = 64;   // editors of a pass (a bit each)
+constexpr uint32_t kTopFilter = 512;  // child slots of a level whose editors are filtered a wavefront per slot
+constexpr uint32_t kTopNodes = 32;   // items of a level whose nodes k_top_nodes enters
+
+// barrier for LDS alone: stores to global memory stay in flight
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+struct TopItems {
+    uint32_t px[kTopCap], py[kTopCap], pz[kTopCap], old_[kTopCap], orig[kTopCap], hOld[kTopCap], hOrig[kTopCap];
+    uint32_t aux[kTopCap], cmode[kTopCap], cmodeval[kTopCap];
+    uint64_t edits[kTopCap];  // the item's editors, a bit each
+};
+
+// expand of levels [0, last) of a pass over editors [first, first + n), n <= kTopEdits (d_expand,
+// level by level). A level that turns out to hold more than kTopCap items, and the levels after
+// it, run over the item arrays.
+__global__ __launch_bounds__(kTopBlock) void k_top_expand(EditPass P, uint32_t first, uint32_t n, uint32_t last) {
+    __shared__ TopItems sItems[2];
+    __shared__ EditHead sHead[kTopEdits];
+    __shared__ uint64_t sTouch[kTopFilter];
+    __shared__ uint8_t sCover[kTopFilter];
+    __shared__ uint32_t sCount[2], sWords[2], sErr;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, L = P.levels - 2, ctl = P.ctl;
+    const uint64_t below = (1ull << lane) - 1ull;
+    for (uint32_t k = tid; k < n; k += blockDim.x) sHead[k] = load_head(P.edits, first + k);
+    if (tid == 0) {
+        const Items I = P.items[0];
+        TopItems& T = sItems[0];
+        const uint32_t root = I.old_[0];
+        T.px[0] = T.py[0] = T.pz[0] = 0;
+        T.old_[0] = T.orig[0] = root;
+        T.hOld[0] = T.hOrig[0] = root != kInvalidNode ? P.vpool[root] : 0u;
+        T.aux[0] = I.aux[0];
+        T.cmode[0] = I.cmode[0];
+        T.cmodeval[0] = I.cmodeval[0];
+        T.edits[0] = n >= 64 ? ~0ull : (1ull << n) - 1ull;
+        sCount[0] = 1;
+        sErr = *P.errors;
     }
+    lds_barrier();
+    if (sErr) return;
+    uint32_t l = 0;
+    for (; l < last; ++l) {
+        const TopItems& T = sItems[l & 1u];
+        TopItems& N = sItems[(l & 1u) ^ 1u];
+        const uint32_t cur = l & 1u, nxt = cur ^ 1u, count = sCount[cur];  // block-uniform
+        if (count > kTopCap || count > P.cap[l]) break;
+        if (tid == 0) sCount[nxt] = sWords[nxt] = 0;
+        lds_barrier();
+        const Items I = P.items[l];
+        const Items C = P.items[l + 1];
+        const uint32_t depth = P.levels - (l + 1);
+        // position and box of child slot c of item i
+        const auto place = [&](uint32_t i, uint32_t c) {
+            SlotRefs r{};
+            r.cx = (T.px[i] << 1) | ((c >> 2) & 1u);
+            r.cy = (T.py[i] << 1) | ((c >> 1) & 1u);
+            r.cz = (T.pz[i] << 1) | (c & 1u);
+            const float side = (float)(1u << depth);
+            r.x0 = (float)(r.cx << depth);
+            r.y0 = (float)(r.cy << depth);
+            r.z0 = (float)(r.cz << depth);
+            r.x1 = r.x0 + side;
+            r.y1 = r.y0 + side;
+            r.z1 = r.z0 + side;
+            return r;
+        };
+        const auto touches = [&](const SlotRefs& r, uint32_t k) {
+            return expand_touch(P, sHead[k], first + k, l, r.x0, r.y0, r.z0, r.x1, r.y1, r.z1);
+        };
+        const auto covers = [&](const SlotRefs& r, uint32_t k) {
+            return l + 1 >= ctl && e_cover(sHead[k], r.x0, r.y0, r.z0, r.x1, r.y1, r.z1) != 0;
+        };
+        // More than a few editors on few slots: a wavefront per slot tests them a lane each (a
+        // thread per slot takes 0.4 us an editor, 20 us a level at 48).
+        const bool filtered = n > 8 && count * 8 <= kTopFilter;
+        if (filtered) {
+            for (uint32_t slot = tid >> 6; slot < count * 8; slot += blockDim.x >> 6) {
+                const uint32_t i = slot >> 3;
+                const SlotRefs r = place(i, slot & 7u);
+                const bool t = lane < n && ((T.edits[i] >> lane) & 1ull) && touches(r, lane);
+                const uint64_t tm = __ballot(t), cm = __ballot(t && covers(r, lane));
+                if (lane == 0) {
+                    sTouch[slot] = tm;
+                    sCover[slot] = cm ? (uint8_t)(63u - (uint32_t)__builtin_clzll(cm)) : 0xFFu;
+                }
+            }
+            lds_barrier();
+        }
+        unsigned long long covered = 0;
+        for (uint32_t b0 = 0; b0 < count * 8; b0 += blockDim.x) {  // block-uniform
+            const uint32_t slot = b0 + tid, i = slot >> 3, c = slot & 7u;
+            const bool active = slot < count * 8;
+            uint32_t kind = KIND_KEEP, lastCover = ~0u, coverKind = 0, coverColor = 0, h1 = 0;
+            uint64_t rest = 0;
+            SlotRefs r{};
+            if (active) {
+                r = place(i, c);
+                const uint32_t old = T.old_[i], orig = T.orig[i], mo = T.hOld[i] & 0xFFu, mg = T.hOrig[i] & 0xFFu;
+                r.childOld = old != kInvalidNode && (mo >> c) & 1u ? P.vpool[old + child_off(mo, c)] : kInvalidNode;
+                r.childOrig = orig == old ? r.childOld
+                              : orig != kInvalidNode && (mg >> c) & 1u ? P.vpool[orig + child_off(mg, c)]
+                                                                       : kInvalidNode;
+                uint64_t touch = 0;
+                uint32_t cover = 0xFFu;  // the last editor that covers the slot
+                if (filtered) {
+                    touch = sTouch[slot];
+                    cover = sCover[slot];
+                } else {
+                    for (uint64_t q = T.edits[i]; q; q &= q - 1) {
+                        const uint32_t k = (uint32_t)__ffsll((long long)q) - 1u;
+                        if (!touches(r, k)) continue;
+                        touch |= 1ull << k;
+                        if (covers(r, k)) cover = k;
+                    }
+                }
+                rest = touch;
+                if (cover != 0xFFu) {
+                    const EditHead& h = sHead[cover];
+                    lastCover = (uint32_t)__popcll(touch & ((1ull << cover) - 1ull));
+                    coverKind = h.kind == EDIT_SPHERE_ADD || h.kind == EDIT_BOX_ADD ? 1u : 2u;
+                    coverColor = h.single;
+                    rest = touch & ~((2ull << cover) - 1ull);  // the editors after it
+                }
+                uint32_t oldCount = 0;
+                if (l + 1 < L) {
+                    h1 = r.childOld != kInvalidNode ? P.vpool[r.childOld] : 0u;
+                    oldCount = l + 1 >= ctl ? h1 >> 8 : 0u;
+                } else {
+                    oldCount = slot_old_count(P, l, r);
+                }
+                unsigned long long cvx = 0;
+                kind = slot_classify(P, I, l, slot, depth, r, oldCount, (uint32_t)__popcll(touch), lastCover, coverKind,
+                                     coverColor, cvx);
+                covered += cvx;
+                I.ckind[slot] = (uint8_t)kind;
+            }
+            const bool isItem = active && kind == KIND_ITEM;
+            const uint32_t nRest = isItem ? (uint32_t)__popcll(rest) : 0u;
+            const uint64_t im = __ballot(isItem);
+            if (!im) continue;  // wave-uniform
+            const uint32_t incl = wave_scan32(nRest);
+            uint32_t ci = 0, eo = 0;
+            if (lane == 63) {
+                ci = atomicAdd(&sCount[nxt], (uint32_t)__popcll(im));
+                eo = atomicAdd(&sWords[nxt], incl);
+            }
+            ci = __shfl(ci, 63, 64) + (uint32_t)__popcll(im & below);
+            eo = __shfl(eo, 63, 64) + incl - nRest;
+            if (!isItem) continue;
+            if (ci >= P.cap[l + 1] || eo + nRest > P.ecap[l + 1]) {
+                set_error(P.errors, ERR_SCRATCH);
+                sErr = 1;
+                continue;
+            }
+            uint32_t w = 0;
+            for (uint64_t q = rest; q; q &= q - 1)
+                P.elist[l + 1][eo + w++] = first + (uint32_t)__ffsll((long long)q) - 1u;
+            uint32_t childOld;
+            ParentRefs child;
+            slot_child_item(P, I, C, l, i, c, slot, ci, eo, nRest, r, lastCover, coverKind, coverColor,
+                            ParentRefs{T.cmode[i], T.cmodeval[i], T.aux[i]}, childOld, child);
+            if (ci < kTopCap && l + 1 < last) {
+                N.px[ci] = r.cx;
+                N.py[ci] = r.cy;
+                N.pz[ci] = r.cz;
+                N.old_[ci] = childOld;
+                N.orig[ci] = r.childOrig;
+                const uint32_t ho = childOld == r.childOld       ? h1
+                                    : childOld != kInvalidNode ? P.vpool[childOld]
+                                                               : 0u;
+                N.hOld[ci] = ho;
+                N.hOrig[ci] = r.childOrig == childOld        ? ho
+                              : r.childOrig == r.childOld    ? h1
+                              : r.childOrig != kInvalidNode ? P.vpool[r.childOrig]
+                                                            : 0u;
+                N.aux[ci] = child.aux;
+                N.cmode[ci] = child.cmode;
+                N.cmodeval[ci] = child.cmodeval;
+                N.edits[ci] = rest;
+            }
+        }
+        if (P.single_edit) wave_add64(P.stat_voxels, covered);
+        lds_barrier();
+        if (tid == 0) {
+            P.count[l + 1] = sCount[nxt];
+            P.ecount[l + 1] = sWords[nxt];
+        }
+        if (sErr) return;  // block-uniform: sErr was last written before the barrier
+    }
+    for (; l < last; ++l) {
+        __syncthreads();
+        d_expand(P, l, VGrid{0, 1});
+    }
+}
+
+// Build and nodes of levels first .. 0, each of at most kTopNodes items, in one workgroup: eight
+// lanes build an item's node from its children's results, which stay in LDS, and a wavefront
+// enters it into the table. The child slots of all these levels are loaded at once at the start.
+// More items on one of the levels than that (the host's bound is of the editors' boxes, rounded):
+// all levels run over the item arrays.
+constexpr uint32_t kTopSlots = kTopNodes * 8;
+struct TopSlots {
+    uint32_t cval[kTopSlots], corig[kTopSlots], cnew[kTopSlots];
+    uint8_t kind[kTopSlots];
+};
+__global__ __launch_bounds__(kTopBlock) void k_top_nodes(EditPass P, uint32_t first) {
+    __shared__ TopSlots sSlots[kMaxEditLevels];
+    __shared__ uint32_t sIdx[2][kTopNodes], sCnt[2][kTopNodes], sDup[2][kTopNodes];
+    __shared__ uint32_t sWord[kTopNodes][9], sLen[kTopNodes];
+    __shared__ uint32_t sErr;
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, waves = blockDim.x >> 6;
+    if (tid == 0) sErr = *P.errors;
+    lds_barrier();
+    if (sErr) return;
+    bool fits = true;
+    for (uint32_t l = 0; l <= first; ++l) fits &= P.count[l] <= min(kTopNodes, P.cap[l]);
+    if (!fits) {  // block-uniform
+        for (uint32_t l = first + 1; l-- > 0;) {
+            d_build(P, l, VGrid{0, 1});
+            __syncthreads();
+            d_nodes(P, l, VGrid{0, 1});
+            __syncthreads();
+        }
+        return;
+    }
+    for (uint32_t l = wave; l <= first; l += waves) {
+        const Items I = P.items[l];
+        const uint32_t slots = P.count[l] * 8;
+        for (uint32_t t = lane; t < slots; t += 64) {
+            uint32_t kind = I.ckind[t], cval = I.cval[t], cnew = I.cnew[t];
+            if (l == first && kind == KIND_ITEM) {  // the children's nodes are in the item arrays
+                const Items C = P.items[l + 1];
+                const uint32_t ci = cval;
+                cval = item_node(C, ci);
+                cnew = C.ncount[ci];
+                I.cnew[t] = cnew;
+                kind = KIND_KEEP;
+            }
+            sSlots[l].kind[t] = (uint8_t)kind;
+            sSlots[l].cval[t] = cval;
+            sSlots[l].cnew[t] = cnew;
+            sSlots[l].corig[t] = I.corig[t];
+        }
+    }
+    lds_barrier();
+    uint32_t added = 0;
+    uint64_t scanBytes = 0;
+    for (uint32_t l = first + 1; l-- > 0;) {
+        const uint32_t cur = l & 1u, prv = cur ^ 1u, n = P.count[l];
+        const Items I = P.items[l];
+        const TopSlots& S = sSlots[l];
+        if (tid < kTopSlots) {
+            const uint32_t i = tid >> 3, c = tid & 7u;
+            uint32_t idx = kInvalidNode, cnt = 0, corig = kInvalidNode;
+            if (i < n) {
+                corig = S.corig[tid];
+                if (S.kind[tid] == KIND_ITEM) {
+                    const uint32_t ci = S.cval[tid];
+                    idx = sIdx[prv][sDup[prv][ci]];
+                    cnt = sCnt[prv][ci];
+                    I.cnew[tid] = cnt;
+                } else {
+                    idx = S.cval[tid];
+                    cnt = S.cnew[tid];
+                }
+            }
+            const uint32_t valid = (uint32_t)(__ballot(idx != kInvalidNode) >> (lane & ~7u)) & 0xFFu;
+            const uint32_t changed = (uint32_t)(__ballot(idx != corig) >> (lane & ~7u)) & 0xFFu;
+            uint32_t sum = idx != kInvalidNode ? cnt : 0u;
+#pragma unroll
+            for (uint32_t d = 1; d < 8; d <<= 1) sum += __shfl_xor(sum, d, 64);
+            if (i < n) {
+                if (idx != kInvalidNode) sWord[i][1 + __popc(valid & ((1u << c) - 1u))] = idx;
+                if (c == 0) {
+                    if (l >= P.ctl && sum >= (1u << 24)) set_error(P.errors, ERR_HEADER);
+                    const bool pending = changed && valid;
+                    sWord[i][0] = valid | (l >= P.ctl ? sum << 8 : 0u);
+                    sLen[i] = pending ? 1u + (uint32_t)__popc(valid) : 0u;
+                    sDup[cur][i] = i;
+                    sCnt[cur][i] = sum;
+                    sIdx[cur][i] = changed ? kInvalidNode : I.orig[i];
+                    I.ncount[i] = sum;
+                }
+            }
+        }
+        lds_barrier();
+        // two items a wavefront at most
+        for (uint32_t i = wave; i < n; i += waves) {
+            const uint32_t len = sLen[i];
+            uint32_t idx = sIdx[cur][i];
+            if (len) {
+                NodeWords c;
+#pragma unroll
+                for (uint32_t k = 0; k < 9; ++k) c.w[k] = __builtin_amdgcn_readfirstlane(k < len ? sWord[i][k] : 0u);
+                c.n = __builtin_amdgcn_readfirstlane(len);
+                c.hash = node_hash(c);
+                // an earlier item with the same content stands for this one
+                bool same = lane < i && sLen[min(lane, kTopNodes - 1u)] == len;
+                if (same) {
+#pragma unroll
+                    for (uint32_t k = 0; k < 9; ++k) same = same && (k >= len || sWord[lane][k] == c.w[k]);
+                }
+                const uint64_t dup = __ballot(same);
+                if (dup) {
+                    if (lane == 0) sDup[cur][i] = (uint32_t)__ffsll((long long)dup) - 1u;
+                } else {
+                    idx = find_node(P, l, c, scanBytes);
+                    if (lane == 0) {
+                        if (idx == ~0u) {
+                            idx = append_node(P, l, c);
+                            if (idx == ~0u) sErr = 1;
+                            else added += c.n;
+                        }
+                        sIdx[cur][i] = idx;
+                    }
+                }
+            }
+            if (lane == 0 && l == 0) {  // the root, for the commit
+                I.nidx[i] = idx;
+                I.state[i] = kStateKnown;
+            }
+        }
+        lds_barrier();
+        if (sErr) break;  // block-uniform; the error flags are set
+    }
+    wave_add64(P.stat_new_words, added);
+    if (P.abytes) wave_add64(P.abytes + 1, scanBytes);
 }
 
 template <bool kSpecial>
@@ -2951,7 +3332,7 @@ static void level_bounds(const EditPass& P, const DevEdit* e, uint32_t n, uint64
 }
 
 constexpr uint32_t kWideEdits = 8, kWideItems = 512;
-constexpr uint32_t kTopItems = 128, kTopNodes = 32, kNodesItems = 1u << 15;
+constexpr uint32_t kTopItems = 128, kNodesItems = 1u << 12;
 
 hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hipStream_t s, const uint32_t* dN,
                        bool special, const EditScratch* scratch, const DevEdit* hostEdits) {
@@ -2996,17 +3377,14 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
     const auto small = [&](uint32_t) { return smallPass; };
     // a wavefront per task slot (the task count is on the device), at most 2^18 of them
     const bool bounded = hostEdits && !dN;  // bound[] from the editors' boxes
-    // steps of k_top: a thread per child slot of a level with at most kTopItems items, 16
-    // wavefronts for the nodes of one with at most kTopNodes
-    const auto top_step = [&](uint16_t code) {
-        const uint32_t l = code & 0xFFu;
-        switch (code >> 8) {
-            case ST_EXPAND: return bound[l] <= kTopItems && !((P.wide_levels >> l) & 1u);
-            case ST_BUILD: return bound[l] <= kTopNodes;
-            case ST_NODES: return l < L && bound[l] <= kTopNodes;
-            default: return false;
-        }
-    };
+    // levels [0, topExpand) expand in k_top_expand, levels topNodes .. 0 build and enter their
+    // nodes in k_top_nodes (~0: none)
+    uint32_t topExpand = 0, topNodes = ~0u;
+    if (hostEdits && !dN && !P.abytes) {
+        if (n <= kTopEdits)
+            while (topExpand < L && bound[topExpand] <= kTopItems) ++topExpand;
+        while (topNodes + 1 < L && bound[topNodes + 1] <= kTopNodes) ++topNodes;
+    }
     const auto wideGrid = [](uint64_t blocks) {
         return (uint32_t)std::min<uint64_t>(std::max<uint64_t>(blocks, 1u), 1u << 16);
     };
@@ -3025,14 +3403,17 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
             continue;
         }
         const uint32_t st = sl.step[i] >> 8;
-        if (bounded) {  // the small levels around the root, together
-            uint32_t j = i;
-            while (j < sl.n && top_step(sl.step[j])) ++j;
-            if (j > i + 1) {
-                k_top<<<1, kTopBlock, 0, s>>>(P, sl, i, j);
-                i = j;
-                continue;
-            }
+        // the small levels around the root, together (not while bytes are counted: d_expand counts
+        // the descent's)
+        if (i == 0 && topExpand > 1) {
+            k_top_expand<<<1, kTopBlock, 0, s>>>(P, first, n, topExpand);
+            i = topExpand;
+            continue;
+        }
+        if (st == ST_BUILD && (sl.step[i] & 0xFFu) == topNodes) {
+            k_top_nodes<<<1, kTopBlock, 0, s>>>(P, topNodes);
+            i += 2 * (topNodes + 1);  // build and nodes of levels topNodes .. 0
+            continue;
         }
         const uint32_t l = sl.step[i] & 0xFFu, gl = grid[l];
         // Grids from the level's item bound by each kernel's unit of work (a thread, or a
