@@ -165,6 +165,8 @@ hd_status hd_create(const hd_config* cfg, hd_ctx** out) {
     if ((e = hipMalloc(&ctx->byte_counters, 8 * sizeof(unsigned long long))) != hipSuccess)
         return cleanup(hip_fail(nullptr, e, "byte counters"));
     if ((e = hipMalloc(&ctx->d_root, 64)) != hipSuccess) return cleanup(hip_fail(nullptr, e, "root"));
+    if ((e = hipHostMalloc(&ctx->h_readback, sizeof(PassReadback))) != hipSuccess)
+        return cleanup(hip_fail(nullptr, e, "pass report"));
     if ((e = hipMalloc(&ctx->leaf_tags, std::max<uint64_t>(leaf_tag_bytes(g), 4))) != hipSuccess)
         return cleanup(hip_fail(nullptr, e, "leaf tags"));
     if ((e = hipMalloc(&ctx->edit_bytes, 8 * sizeof(unsigned long long))) != hipSuccess)
@@ -188,6 +190,7 @@ hd_status hd_destroy(hd_ctx* ctx) {
     hipDeviceSynchronize();
     edit_free(ctx);
     gc_scratch_free(ctx);
+    hipHostFree(ctx->h_readback);
     hipFree(ctx->d_root);
     hipFree(ctx->vpool);
     hipFree(ctx->page_table);

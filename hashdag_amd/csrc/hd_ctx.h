@@ -3,6 +3,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
+#include <memory>
 #include <mutex>
 #include <string>
 #include <utility>
@@ -33,10 +35,81 @@ struct TraceScratch {
     uint64_t pixels_cap = 0;
 };
 
+// Device memory for the undo history's leaf records: slabs filled from the front, each kept while
+// a frame lives in it, then held for reuse (at most kSpare of them) or freed. A pass of 4096
+// editors re-points 700,000 leaves: as host vectors its frame was 90 MB copied through pageable
+// memory, and half of that back on undo. Beyond kBytes of slabs frames go to the host.
+struct UndoSlab {
+    UndoRecord* mem = nullptr;
+    uint64_t cap = 0, used = 0;
+};
+class UndoPool {
+public:
+    static constexpr uint64_t kBytes = 4ull << 30, kMinRecords = 1u << 16;
+    static constexpr size_t kSpare = 2;
+    // a slab with room for n more records, or null (budget or memory: the caller keeps the frame
+    // on the host)
+    std::shared_ptr<UndoSlab> reserve(uint64_t n) {
+        if (cur_ && cur_.use_count() == 1) cur_->used = 0;  // no frame left in it
+        if (cur_ && cur_->cap - cur_->used >= n) return cur_;
+        cur_.reset();
+        for (size_t k = 0; k < spare_.size(); ++k)
+            if (spare_[k]->cap >= n) {
+                UndoSlab* sl = spare_[k];
+                spare_.erase(spare_.begin() + (long)k);
+                sl->used = 0;
+                return cur_ = own(sl);
+            }
+        const uint64_t want = std::max<uint64_t>(n + n / 4, kMinRecords), bytes = want * sizeof(UndoRecord);
+        if (bytes_ + bytes > kBytes) drop_spares();
+        if (bytes_ + bytes > kBytes) return nullptr;
+        auto* sl = new UndoSlab();
+        if (hipMalloc(&sl->mem, bytes) != hipSuccess) {
+            (void)hipGetLastError();
+            delete sl;
+            return nullptr;
+        }
+        sl->cap = want;
+        bytes_ += bytes;
+        return cur_ = own(sl);
+    }
+    ~UndoPool() {
+        cur_.reset();
+        drop_spares();
+    }
+
+private:
+    std::shared_ptr<UndoSlab> own(UndoSlab* sl) {
+        return std::shared_ptr<UndoSlab>(sl, [this](UndoSlab* x) { give_back(x); });
+    }
+    void give_back(UndoSlab* sl) {
+        spare_.push_back(sl);
+        if (spare_.size() > kSpare) {
+            release(spare_.front());
+            spare_.erase(spare_.begin());
+        }
+    }
+    void release(UndoSlab* sl) {
+        bytes_ -= sl->cap * sizeof(UndoRecord);
+        (void)hipFree(sl->mem);
+        delete sl;
+    }
+    void drop_spares() {
+        for (UndoSlab* sl : spare_) release(sl);
+        spare_.clear();
+    }
+    std::vector<UndoSlab*> spare_;
+    uint64_t bytes_ = 0;
+    std::shared_ptr<UndoSlab> cur_;
+};
+
 // One undo step (HashDAGUndoRedo::Frame, hash_dag.h:29-45): the roots before / after and the
-// colour-leaf descriptors the pass replaced (old leaf data stays in the colour arena).
+// colour-leaf descriptors the pass replaced (old leaf data stays in the colour arena), n of them
+// from record `first` of a slab, or on the host.
 struct UndoFrame {
-    uint32_t prev_root = 0, new_root = 0;
+    uint32_t prev_root = 0, new_root = 0, n = 0;
+    std::shared_ptr<UndoSlab> slab;
+    uint64_t first = 0;
     std::vector<uint32_t> handles;
     std::vector<LeafDesc> prev, next;
 };
@@ -106,6 +179,8 @@ struct hd_ctx {
     // edits
     uint32_t* d_root = nullptr;  // device copy of the root (edit passes chain through it)
     hd::EditScratch edit;
+    hd::PassReadback* h_readback = nullptr;  // pinned: the last pass's report
+    hd::UndoPool undo_pool;                  // outlives the frames below
     std::vector<hd::UndoFrame> undo, redo;
     // GC scratch, kept between collections and grown when a call needs more (freed with the
     // context): slot k holds (buffer, bytes)

@@ -121,6 +121,19 @@ struct Items {
     uint64_t* cbase;            // tasks: base of the task's colour array
 };
 
+// What a pass reports to the host: written into pinned memory by its last kernel.
+struct PassReadback {
+    uint32_t counters[8];
+    uint64_t stats[8];
+    uint32_t root, pad;
+};
+
+// One colour leaf a pass re-pointed: its slot, and the leaf before and after the pass.
+struct UndoRecord {
+    LeafDesc prev, next;
+    uint32_t handle, pad;
+};
+
 struct EditPass {
     Geom g;
     uint32_t levels, ctl;
@@ -175,6 +188,7 @@ struct EditPass {
     uint32_t* undo_handles;
     LeafDesc* undo_descs;
     uint32_t undo_cap;
+    PassReadback* rb;
 };
 
 // Per-pass scratch. Item arrays and edit lists are sized per level (one allocation each) from

@@ -39,6 +39,9 @@
 #include "hd_edit.h"
 
 namespace hd {
+// edited-voxel count of editors into *out (hd_edit_api.hip)
+void launch_count_voxels(const DevEdit* edits, uint32_t n, const uint32_t* dN, uint32_t E, unsigned long long* out,
+                         hipStream_t s);
 namespace {
 
 constexpr uint32_t KIND_KEEP = 0, KIND_EMPTY = 1, KIND_FULL = 2, KIND_ITEM = 3;
@@ -2083,6 +2086,33 @@ __global__ __launch_bounds__(256) void k_scatter_leaves(LeafDesc* leaves, const 
         leaves[handles[k] & 0x7FFFFFFFu] = descs[k];
 }
 
+// The undo frame of a pass: every slot of its undo log with the leaf before and after the pass
+// (at most cap records). Nothing after a failed pass.
+__global__ __launch_bounds__(256) void k_capture_frame(const LeafDesc* __restrict__ leaves,
+                                                       const uint32_t* __restrict__ handles,
+                                                       const LeafDesc* __restrict__ descs,
+                                                       const uint32_t* __restrict__ count,
+                                                       const uint32_t* __restrict__ errors, UndoRecord* rec,
+                                                       uint32_t cap) {
+    if (*errors) return;
+    const uint32_t n = min(*count, cap);
+    for (uint32_t k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) {
+        const uint32_t h = handles[k];
+        rec[k].prev = descs[k];
+        rec[k].next = leaves[h & 0x7FFFFFFFu];
+        rec[k].handle = h;
+    }
+}
+
+// A frame's leaves from before (undo) or after its pass, and the root that goes with them.
+__global__ __launch_bounds__(256) void k_apply_frame(LeafDesc* leaves, const UndoRecord* __restrict__ rec, uint32_t n,
+                                                     bool undo, uint32_t* d_root, uint32_t root) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0) *d_root = root;
+    for (uint32_t k = t; k < n; k += gridDim.x * blockDim.x)
+        leaves[rec[k].handle & 0x7FFFFFFFu] = undo ? rec[k].prev : rec[k].next;
+}
+
 // The leaves a pass wrote, in undo-log order (the redo half of an undo frame).
 __global__ __launch_bounds__(256) void k_gather_leaves(const LeafDesc* leaves, const uint32_t* handles,
                                                        LeafDesc* out, uint32_t n) {
@@ -2515,12 +2545,22 @@ __global__ __launch_bounds__(256) void k_fill_colors(EditPass P, const uint32_t*
         out[i] = source_color(P, root, xyz[3 * i], xyz[3 * i + 1], xyz[3 * i + 2]);
 }
 
-__global__ void k_init_pass(EditPass P, uint32_t root, uint32_t first, uint32_t nEdits, const uint32_t* dN) {
-    // level-0 item = the root, carrying the edits [first, first + nEdits)
+// Start of a pass: its counters, and the level-0 item, the root with the editors [first, first +
+// nEdits). An eager pass brings the root along (and into d_root); a graph replay (dN) starts from
+// the root the last one left in d_root.
+__global__ void k_init_pass(EditPass P, uint32_t* d_root, uint32_t root, uint32_t first, uint32_t nEdits,
+                            const uint32_t* dN) {
     if (dN) nEdits = min(nEdits, *dN);
     const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t < nEdits) P.elist[0][t] = first + t;
     if (t == 0) {
+        if (dN) root = *d_root;
+        else *d_root = root;
+        *P.errors = 0;
+        *P.undo_count = 0;
+        unsigned long long* stats = P.stat_voxels;
+        for (uint32_t i = 0; i < 32; ++i) stats[i] = 0;  // stats, and the per-level find-list counts
+        *P.arena_top = *reinterpret_cast<const unsigned long long*>(P.pool_top + kArenaTopWord);  // committed top
         for (uint32_t l = 0; l < P.levels; ++l) {
             P.count[l] = 0;
             P.ecount[l] = 0;
@@ -2538,22 +2578,34 @@ __global__ void k_init_pass(EditPass P, uint32_t root, uint32_t first, uint32_t 
         I.aux[0] = 0;  // colour node of the root
         I.cmode[0] = 0;
         I.cmodeval[0] = 0;
-        *P.color_top = 0;
-        *P.seg_top = 0;
     }
 }
 
+// End of a pass: the root and the colour arena top are committed unless an error is set, and the
+// pass's report goes to the host.
 __device__ __forceinline__ void d_finish(const EditPass& P, uint32_t* root_out, VGrid G) {
-    if (G.block == 0 && threadIdx.x == 0 && *P.errors == 0) {
-        const uint32_t r = P.items[0].nidx[0];
-        if (r == kInvalidNode) {
-            set_error(P.errors, ERR_EMPTY);
-        } else {
-            *root_out = r;
-            // commit the colour arena top (a failed pass leaves the committed value)
-            *reinterpret_cast<unsigned long long*>(P.pool_top + kArenaTopWord) = *P.arena_top;
+    if (G.block != 0 || threadIdx.x >= 64) return;
+    const uint32_t t = threadIdx.x;
+    const uint32_t* counters = P.pool_top;
+    const unsigned long long* stats = P.stat_voxels;
+    if (t == 0) {
+        uint32_t err = *P.errors;
+        if (err == 0) {
+            const uint32_t r = P.items[0].nidx[0];
+            if (r == kInvalidNode) {
+                err = ERR_EMPTY;
+                set_error(P.errors, ERR_EMPTY);
+            } else {
+                *root_out = r;
+                P.rb->root = r;
+                // commit the colour arena top (a failed pass leaves the committed value)
+                *reinterpret_cast<unsigned long long*>(P.pool_top + kArenaTopWord) = *P.arena_top;
+            }
         }
+        P.rb->counters[1] = err;
     }
+    if (t < 8 && t != 1) P.rb->counters[t] = counters[t];
+    if (t < 8) P.rb->stats[t] = stats[t];
 }
 __global__ void k_finish(EditPass P, uint32_t* root_out) {
     d_finish(P, root_out, VGrid{blockIdx.x, gridDim.x});
@@ -2890,8 +2942,8 @@ __global__ __launch_bounds__(256) void k_pass_block(EditPass P, StepList sl, uin
 // A level of few items costs its launch and the latency of what it reads one after another. Here
 // a workgroup goes through consecutive levels with the items in LDS: between two levels only the
 // tree's own words (a child pointer, the child's header) are waited for, not the item arrays,
-// which are written for the later steps on the way. 13 levels of a brush stroke: expand 108 -> 35
-// us, build and nodes 110 -> 50 us (as steps over the item arrays in one workgroup, and 9 and
+// which are written for the later steps on the way. 13 levels of a brush stroke: expand 108 -> 63
+// us, build and nodes 110 -> 51 us (as steps over the item arrays in one workgroup, and 9 and
 // 15-20 us a level as launches).
 constexpr uint32_t kTopCap = 256;    // items of a level held in LDS
 constexpr uint32_t kTopEdits = 64;   // editors of a pass (a bit each)
@@ -3334,10 +3386,11 @@ static void level_bounds(const EditPass& P, const DevEdit* e, uint32_t n, uint64
 constexpr uint32_t kWideEdits = 8, kWideItems = 512;
 constexpr uint32_t kTopItems = 128, kNodesItems = 1u << 12;
 
-hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hipStream_t s, const uint32_t* dN,
-                       bool special, const EditScratch* scratch, const DevEdit* hostEdits) {
+hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hipStream_t s, PassReadback* rb,
+                       const uint32_t* dN, bool special, const EditScratch* scratch, const DevEdit* hostEdits) {
     EditPass P{};
     fill_pass(ctx, P, scratch ? *scratch : ctx->edit);
+    P.rb = rb;
     // grid per level: two blocks per item the level can hold (a wavefront per child slot is the
     // most any step uses), at most kGrid; kGrid everywhere without the host's copy of the edits
     uint32_t grid[kMaxEditLevels];
@@ -3358,10 +3411,9 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
         for (uint32_t l = 0; l < kMaxEditLevels && l < 32; ++l)
             if (bound[l] <= kWideItems) P.wide_levels |= 1u << l;
     const uint32_t D = P.levels, L = D - 2;
-    k_init_pass<<<(std::max<uint32_t>(n, 1) + 255) / 256, 256, 0, s>>>(P, 0xFFFFFFFFu, first, n, dN);
-    // the root index lives in ctx->d_root (device) so passes chain without a host round trip
-    hipMemcpyAsync(&P.items[0].old_[0], ctx->d_root, 4, hipMemcpyDeviceToDevice, s);
-    hipMemcpyAsync(&P.items[0].orig[0], ctx->d_root, 4, hipMemcpyDeviceToDevice, s);
+    k_init_pass<<<(std::max<uint32_t>(n, 1) + 255) / 256, 256, 0, s>>>(P, ctx->d_root, ctx->root, first, n, dN);
+    // a plain pass counts its edited voxels on the way; the others' are counted from the editors
+    if (n > 1 || dN) launch_count_voxels(P.edits + first, n, dN, 1u << D, P.stat_voxels, s);
     StepList sl = pass_step_list(D, P.ctl, colors);
     // one cooperative launch for passes of at most edit_persist_max edits (not under capture)
     if (!dN && n <= ctx->edit_persist_max)
@@ -3467,6 +3519,32 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
     }
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return hip_fail(ctx, e, "edit pass launch");
+    return HD_OK;
+}
+
+// Upper bound of the colour leaves a pass over these editors re-points (one per task).
+uint64_t pass_task_bound(hd_ctx* ctx, const DevEdit* hostEdits, uint32_t n) {
+    EditPass P{};
+    fill_pass(ctx, P, ctx->edit);
+    uint64_t bound[kMaxEditLevels];
+    for (uint32_t l = 0; l < kMaxEditLevels; ++l) bound[l] = P.cap[l];
+    if (hostEdits) level_bounds(P, hostEdits, n, bound);
+    return std::min<uint64_t>(bound[std::min(P.ctl, kMaxEditLevels - 1)], P.undo_cap);
+}
+
+// The undo log of the pass in flight on s into `rec` (room for cap records).
+void edit_capture_frame(hd_ctx* ctx, UndoRecord* rec, uint32_t cap, hipStream_t s) {
+    const EditScratch& S = ctx->edit;
+    if (cap == 0) return;
+    k_capture_frame<<<std::min<uint32_t>((cap + 255) / 256, 2048), 256, 0, s>>>(
+        ctx->cleaves, S.undo_handles, S.undo_descs, ctx->counters + 4, ctx->counters + 1, rec, cap);
+}
+
+// Undo / redo of a frame kept on the device.
+hd_status edit_apply_frame(hd_ctx* ctx, const UndoRecord* rec, uint32_t n, bool undo, uint32_t root) {
+    k_apply_frame<<<std::min<uint32_t>((n + 255) / 256 + 1, 2048), 256>>>(ctx->cleaves, rec, n, undo, ctx->d_root, root);
+    HD_HIP(ctx, hipGetLastError());
+    HD_HIP(ctx, hipDeviceSynchronize());
     return HD_OK;
 }
 

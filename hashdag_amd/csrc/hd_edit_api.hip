@@ -16,9 +16,12 @@ namespace hd {
 
 hd_status edit_reserve(hd_ctx* ctx, const uint32_t* items, const uint32_t* elist, uint64_t colors);
 void edit_free(hd_ctx* ctx);
-hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hipStream_t s,
+hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hipStream_t s, PassReadback* rb,
                        const uint32_t* dN = nullptr, bool special = true, const EditScratch* scratch = nullptr,
                        const DevEdit* hostEdits = nullptr);
+uint64_t pass_task_bound(hd_ctx* ctx, const DevEdit* hostEdits, uint32_t n);
+void edit_capture_frame(hd_ctx* ctx, UndoRecord* rec, uint32_t cap, hipStream_t s);
+hd_status edit_apply_frame(hd_ctx* ctx, const UndoRecord* rec, uint32_t n, bool undo, uint32_t root);
 hd_status edit_ensure_edits(hd_ctx* ctx, uint32_t n);
 hd_status enqueue_frame_from_device(hd_ctx* ctx, const hd_ray_params* d_params, uint32_t W, uint32_t H,
                                     uint32_t* d_paths, uint32_t* d_colors, float bias, float fog, hipStream_t s);
@@ -106,15 +109,6 @@ __global__ __launch_bounds__(256) void k_count_voxels(const DevEdit* __restrict_
 inline dim3 count_grid(uint32_t n) {
     const uint32_t gx = std::min<uint32_t>(n, 4096);
     return dim3(gx, std::min<uint32_t>(64, std::max<uint32_t>(4, 8192 / gx)));
-}
-
-__global__ void k_reset(uint32_t* counters, uint64_t* stats) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
-        counters[1] = 0;  // errors
-        counters[4] = 0;  // undo log
-        for (int i = 0; i < 32; ++i) stats[i] = 0;  // stats, and the per-level find-list counts
-        stats[3] = *reinterpret_cast<const uint64_t*>(counters + kArenaTopWord);  // committed arena top
-    }
 }
 
 // The copy's transform; all zeros stands for the identity (callers that zero the struct).
@@ -207,14 +201,12 @@ uint64_t fill_voxels(const DevEdit& d, uint32_t E) {
     return n;
 }
 
-struct Readback {
-    uint32_t counters[8];
-    uint64_t stats[8];
-    uint32_t root;
-    uint32_t count_ctl;
-};
-
 }  // namespace
+
+void launch_count_voxels(const DevEdit* edits, uint32_t n, const uint32_t* dN, uint32_t E, unsigned long long* out,
+                         hipStream_t s) {
+    k_count_voxels<<<count_grid(n), 256, 0, s>>>(edits, n, dN, E, out);
+}
 
 static hd_status ensure_color_tree(hd_ctx* ctx) {
     if (ctx->colors_loaded) return HD_OK;
@@ -268,9 +260,11 @@ static hd_status grow_color_tables(hd_ctx* ctx, uint64_t nodes, uint64_t leaves)
     return HD_OK;
 }
 
-// The undo frame of a committed pass: the touched slots with their previous and new leaves.
-static hd_status capture_frame(hd_ctx* ctx, uint32_t nu, UndoFrame& frame, hipStream_t s) {
+// The undo frame of a committed pass on the host: the touched slots with their previous and new
+// leaves.
+static hd_status capture_frame_host(hd_ctx* ctx, uint32_t nu, UndoFrame& frame, hipStream_t s) {
     const EditScratch& S = ctx->edit;
+    frame.n = nu;
     frame.handles.resize(nu);
     frame.prev.resize(nu);
     frame.next.resize(nu);
@@ -280,6 +274,24 @@ static hd_status capture_frame(hd_ctx* ctx, uint32_t nu, UndoFrame& frame, hipSt
         HD_HIP(ctx, edit_gather_next(ctx, nu, frame.next.data(), s));
         HD_HIP(ctx, hipStreamSynchronize(s));
     }
+    return HD_OK;
+}
+
+// Room for a pass's undo frame in device memory (`cap` records from frame.first; none: the frame
+// goes to the host), and the frame's size once the pass is known to have touched nu slots.
+static uint32_t frame_reserve(hd_ctx* ctx, uint64_t cap, UndoFrame& frame) {
+    frame.slab = ctx->undo_pool.reserve(cap);
+    if (!frame.slab) return 0;
+    frame.first = frame.slab->used;
+    return (uint32_t)cap;
+}
+static hd_status frame_commit(hd_ctx* ctx, uint32_t nu, uint32_t cap, UndoFrame& frame, hipStream_t s) {
+    if (nu > cap) {
+        frame.slab.reset();
+        return capture_frame_host(ctx, nu, frame, s);
+    }
+    frame.n = nu;
+    if (frame.slab) frame.slab->used = frame.first + nu;
     return HD_OK;
 }
 
@@ -302,7 +314,7 @@ static hd_status edit_prepare(hd_ctx* ctx) {
 // `special`: the pass holds a copy or a fill editor (leaf kernels built with their code).
 // `fixed`: run in this scratch and grow nothing (the colour arena, tables and undo log
 // included); a pass that needs more fails with the previous state kept.
-static hd_status run_pass(hd_ctx* ctx, uint32_t first, uint32_t n, hipStream_t s, Readback& rb, UndoFrame* frame,
+static hd_status run_pass(hd_ctx* ctx, uint32_t first, uint32_t n, hipStream_t s, PassReadback& rb, UndoFrame* frame,
                           bool special, const EditScratch* fixed = nullptr, const DevEdit* hostEdits = nullptr) {
     const bool colors = ctx->colors_loaded && ctx->g.leaf_level() > ctx->g.color_tree_levels;
     for (int attempt = 0; attempt < 40; ++attempt) {
@@ -312,19 +324,16 @@ static hd_status run_pass(hd_ctx* ctx, uint32_t first, uint32_t n, hipStream_t s
         const EditScratch& S = fixed ? *fixed : ctx->edit;
         const uint64_t bucketBytes = (uint64_t)ctx->g.total_buckets() * 4;
         HD_HIP(ctx, hipMemcpyAsync(ctx->bucket_snapshot, ctx->bucket_sizes, bucketBytes, hipMemcpyDeviceToDevice, s));
-        k_reset<<<1, 1, 0, s>>>(ctx->counters, S.dstats);
-        st = enqueue_pass(ctx, first, n, colors, s, nullptr, special, fixed, hostEdits);
+        st = enqueue_pass(ctx, first, n, colors, s, ctx->h_readback, nullptr, special, fixed, hostEdits);
         if (st != HD_OK) return st;
-        if (n > 1) {
-            k_count_voxels<<<count_grid(n), 256, 0, s>>>(S.edits_dev + first, n, nullptr,
-                                                                      1u << ctx->g.levels,
-                                                                      reinterpret_cast<unsigned long long*>(S.dstats + 0));
+        uint32_t frameCap = 0;
+        if (frame && colors) {
+            frameCap = frame_reserve(ctx, pass_task_bound(ctx, hostEdits, n), *frame);
+            if (frameCap) edit_capture_frame(ctx, frame->slab->mem + frame->first, frameCap, s);
         }
-        HD_HIP(ctx, hipMemcpyAsync(rb.counters, ctx->counters, sizeof(rb.counters), hipMemcpyDeviceToHost, s));
-        HD_HIP(ctx, hipMemcpyAsync(rb.stats, S.dstats, sizeof(rb.stats), hipMemcpyDeviceToHost, s));
-        HD_HIP(ctx, hipMemcpyAsync(&rb.root, ctx->d_root, 4, hipMemcpyDeviceToHost, s));
-        HD_HIP(ctx, hipMemcpyAsync(&rb.count_ctl, S.dcount + ctx->g.color_tree_levels, 4, hipMemcpyDeviceToHost, s));
+        HD_HIP(ctx, hipGetLastError());
         HD_HIP(ctx, hipStreamSynchronize(s));
+        rb = *ctx->h_readback;
         const uint32_t err = rb.counters[1];
         if (err) {
             // The root was not switched. Leaf slots the pass already re-pointed get their
@@ -408,7 +417,7 @@ static hd_status run_pass(hd_ctx* ctx, uint32_t first, uint32_t n, hipStream_t s
         ctx->arena_top = rb.stats[3];
         ctx->n_cnodes = rb.counters[2];
         ctx->n_cleaves = rb.counters[3];
-        if (frame) return capture_frame(ctx, rb.counters[4], *frame, s);
+        if (frame) return frame_commit(ctx, rb.counters[4], frameCap, *frame, s);
         return HD_OK;
     }
     return fail(ctx, HD_ERR_OOM, "edit scratch could not be grown enough");
@@ -453,7 +462,6 @@ hd_status hd_edit_batch(hd_ctx* ctx, const hd_edit* edits, uint32_t n, uint32_t 
     st = edit_ensure_edits(ctx, n);
     if (st != HD_OK) return st;
     if (n) HD_HIP(ctx, hipMemcpyAsync(ctx->edit.edits_dev, dev.data(), (uint64_t)n * sizeof(DevEdit), hipMemcpyHostToDevice, s));
-    HD_HIP(ctx, hipMemcpyAsync(ctx->d_root, &ctx->root, 4, hipMemcpyHostToDevice, s));
     hd_edit_stats out{};
     // a fill's or a noise editor's buffers are built from the DAG as it is when its pass starts
     FillBuffers fb;
@@ -479,7 +487,7 @@ hd_status hd_edit_batch(hd_ctx* ctx, const hd_edit* edits, uint32_t n, uint32_t 
             while (last < n && !is_copy_kind(edits[last].kind) && !is_buffer_kind(edits[last].kind)) ++last;
             UndoFrame frame;
             frame.prev_root = ctx->root;
-            Readback rb{};
+            PassReadback rb{};
             st = prepare_fill(first);
             if (st != HD_OK) return st;
             st = run_pass(ctx, first, last - first, s, rb, &frame,
@@ -503,7 +511,7 @@ hd_status hd_edit_batch(hd_ctx* ctx, const hd_edit* edits, uint32_t n, uint32_t 
         for (uint32_t i = 0; i < n; ++i) {
             UndoFrame frame;
             frame.prev_root = ctx->root;
-            Readback rb{};
+            PassReadback rb{};
             st = prepare_fill(i);
             if (st != HD_OK) return st;
             st = run_pass(ctx, i, 1, s, rb, &frame, is_copy_kind(edits[i].kind) || is_buffer_kind(edits[i].kind),
@@ -526,10 +534,17 @@ hd_status hd_edit_batch(hd_ctx* ctx, const hd_edit* edits, uint32_t n, uint32_t 
 }
 
 static hd_status apply_frame(hd_ctx* ctx, const UndoFrame& f, bool undo) {
+    const uint32_t root = undo ? f.prev_root : f.new_root;
+    if (f.slab || f.n == 0) {
+        const hd_status st = edit_apply_frame(ctx, f.slab ? f.slab->mem + f.first : nullptr, f.n, undo, root);
+        if (st != HD_OK) return st;
+        ctx->root = root;
+        return HD_OK;
+    }
     const hd_status st = edit_scatter_leaves(ctx, f.handles.data(), undo ? f.prev.data() : f.next.data(),
                                              (uint32_t)f.handles.size());
     if (st != HD_OK) return st;
-    ctx->root = undo ? f.prev_root : f.new_root;
+    ctx->root = root;
     HD_HIP(ctx, hipMemcpy(ctx->d_root, &ctx->root, 4, hipMemcpyHostToDevice));
     return HD_OK;
 }
@@ -787,8 +802,7 @@ hd_status hd_edit_batch_static(hd_ctx* ctx, const hd_edit* edits, uint32_t n, hd
         HD_HIP(ctx, hipMemcpyAsync(S.edits_dev + i, dev, (uint64_t)m * sizeof(DevEdit), hipMemcpyHostToDevice, s));
         HD_HIP(ctx, hipStreamSynchronize(s));
     }
-    HD_HIP(ctx, hipMemcpyAsync(ctx->d_root, &ctx->root, 4, hipMemcpyHostToDevice, s));
-    Readback rb{};
+    PassReadback rb{};
     st = run_pass(ctx, 0, n, s, rb, nullptr, false, &S);
     if (st != HD_OK) return st;
     ctx->root = rb.root;
@@ -828,7 +842,7 @@ struct hd_frame_graph {
     DevEdit* h_edits = nullptr;      // pinned staging
     uint32_t* h_n = nullptr;
     hd_ray_params* h_params = nullptr;
-    Readback* h_rb = nullptr;
+    PassReadback* h_rb = nullptr;
     uint32_t* d_n = nullptr;         // device copies read by the replay
     hd_ray_params* d_params = nullptr;
 };
@@ -856,15 +870,9 @@ static hd_status graph_capture(hd_frame_graph* g) {
     hipMemcpyAsync(S.edits_dev, g->h_edits, (uint64_t)g->max_edits * sizeof(DevEdit), hipMemcpyHostToDevice, s);
     if (trace) hipMemcpyAsync(g->d_params, g->h_params, sizeof(hd_ray_params), hipMemcpyHostToDevice, s);
     hipMemcpyAsync(ctx->bucket_snapshot, ctx->bucket_sizes, (uint64_t)ctx->g.total_buckets() * 4, hipMemcpyDeviceToDevice, s);
-    k_reset<<<1, 1, 0, s>>>(ctx->counters, S.dstats);
-    hd_status st = enqueue_pass(ctx, 0, g->max_edits, colors, s, g->d_n, false);  // kinds checked at capture
-    k_count_voxels<<<count_grid(g->max_edits), 256, 0, s>>>(
-        S.edits_dev, g->max_edits, g->d_n, 1u << ctx->g.levels, reinterpret_cast<unsigned long long*>(S.dstats + 0));
+    hd_status st = enqueue_pass(ctx, 0, g->max_edits, colors, s, g->h_rb, g->d_n, false);  // kinds checked at capture
     if (st == HD_OK && trace)
         st = enqueue_frame_from_device(ctx, g->d_params, g->width, g->height, g->paths, g->colors, g->bias, g->fog, s);
-    hipMemcpyAsync(g->h_rb->counters, ctx->counters, sizeof(g->h_rb->counters), hipMemcpyDeviceToHost, s);
-    hipMemcpyAsync(g->h_rb->stats, S.dstats, sizeof(g->h_rb->stats), hipMemcpyDeviceToHost, s);
-    hipMemcpyAsync(&g->h_rb->root, ctx->d_root, 4, hipMemcpyDeviceToHost, s);
     const hipError_t e = hipStreamEndCapture(s, &g->graph);
     if (st != HD_OK) return st;
     if (e != hipSuccess) return hip_fail(ctx, e, "frame graph capture");
@@ -894,7 +902,7 @@ hd_status hd_frame_graph_create(hd_ctx* ctx, uint32_t max_edits, uint32_t width,
     if (e == hipSuccess) e = hipHostMalloc(&g->h_edits, (uint64_t)max_edits * sizeof(DevEdit));
     if (e == hipSuccess) e = hipHostMalloc(&g->h_n, 4);
     if (e == hipSuccess) e = hipHostMalloc(&g->h_params, sizeof(hd_ray_params));
-    if (e == hipSuccess) e = hipHostMalloc(&g->h_rb, sizeof(Readback));
+    if (e == hipSuccess) e = hipHostMalloc(&g->h_rb, sizeof(PassReadback));
     if (e == hipSuccess) e = hipMalloc(&g->d_n, 4);
     if (e == hipSuccess) e = hipMalloc(&g->d_params, sizeof(hd_ray_params));
     if (e != hipSuccess) {
@@ -950,7 +958,7 @@ hd_status hd_frame_graph_launch(hd_frame_graph* g, const hd_edit* edits, uint32_
     if (params) *g->h_params = *params;
     HD_HIP(ctx, hipGraphLaunch(g->exec, g->stream));
     HD_HIP(ctx, hipStreamSynchronize(g->stream));
-    const Readback& rb = *g->h_rb;
+    const PassReadback& rb = *g->h_rb;
     if (rb.counters[1]) {
         // a capacity ran out: drop what the pass appended, roll the leaf slots back and run the
         // frame eagerly (which grows it)
@@ -987,7 +995,12 @@ hd_status hd_frame_graph_launch(hd_frame_graph* g, const hd_edit* edits, uint32_
     ctx->arena_top = rb.stats[3];
     ctx->n_cnodes = rb.counters[2];
     ctx->n_cleaves = rb.counters[3];
-    st = capture_frame(ctx, rb.counters[4], frame, g->stream);
+    const uint32_t nu = rb.counters[4], frameCap = nu ? frame_reserve(ctx, nu, frame) : 0;
+    if (frameCap) {
+        edit_capture_frame(ctx, frame.slab->mem + frame.first, frameCap, g->stream);
+        HD_HIP(ctx, hipStreamSynchronize(g->stream));
+    }
+    st = frame_commit(ctx, nu, frameCap, frame, g->stream);
     if (st != HD_OK) return st;
     ctx->undo.push_back(std::move(frame));
     ctx->redo.clear();
