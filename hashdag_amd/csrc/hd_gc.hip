@@ -3,14 +3,13 @@
 //   mark     level by level from the root: every child pointer of a live node sets its bit in
 //            a bitmap over the virtual address space; the first setter appends the child to
 //            the next level's frontier (the reference's per-level unordered_sets)
-//   rebuild  levels maxLevel .. 0: gather every live node with its children remapped through
-//            the old -> new map of the level below, reset the level's bucket sizes, append the
-//            full node first (ADD_FULL_NODES_FIRST), place every live node in its bucket with
-//            the append rule (in the order of the ranks the nodes draw in their bucket), record
-//            old -> new
+//   rebuild  levels maxLevel .. 0, two launches each: gather every live node with its children
+//            remapped through the old -> new map of the level below and hang it into its
+//            bucket's list; then lay every bucket out anew, the full node first
+//            (ADD_FULL_NODES_FIRST), its list after it by the append rule, record old -> new
 //
 // Pages stay mapped (poolTop never shrinks), as in the reference. The result is canonically
-// identical to the DAG before GC; node order within a bucket is the rank order.
+// identical to the DAG before GC; node order within a bucket is the order of its list.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -22,10 +21,8 @@
 namespace hd {
 namespace {
 
-constexpr uint32_t kGcGrid = 2048;
+constexpr uint32_t kGcGrid = 2048;  // most blocks of a launch over a level's nodes (they stride)
 constexpr uint32_t GC_ERR_CAP = 1, GC_ERR_BUCKET = 2, GC_ERR_POOL = 4, GC_ERR_MAP = 8;
-
-__device__ __forceinline__ uint32_t child_off(uint32_t mask, uint32_t c) { return __popc(mask & ((1u << c) - 1u)) + 1u; }
 
 __global__ void k_gc_fill(uint32_t* p, uint64_t n, uint32_t v) {
     for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) p[i] = v;
@@ -44,21 +41,43 @@ __global__ __launch_bounds__(256) void k_gc_level_used(Geom g, const uint32_t* _
     if ((threadIdx.x & 63u) == 0 && sum) atomicAdd(&used[l], sum);
 }
 
+// the report of a collection: one block of words in device memory, read back once at its end
+// (error flags, bucket of each level's full node, live nodes per level, words used per level, the
+// kept roots)
+constexpr uint32_t kRepFull = 64, kRepCounts = 128, kRepUsed = 192, kRepRoots = 320;
+
 // level 0 frontier = the (distinct) roots kept alive
-__global__ void k_gc_seed(uint32_t* frontier0, uint32_t* counts, const uint32_t* roots, uint32_t n_roots,
-                          uint32_t levels) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) {
-        for (uint32_t l = 0; l <= levels; ++l) counts[l] = 0;
-        counts[0] = n_roots;
+__global__ void k_gc_seed(uint32_t* frontier0, uint32_t* report, uint32_t n_roots) {
+    if (blockIdx.x == 0) {
+        for (uint32_t i = threadIdx.x; i < kRepRoots; i += blockDim.x) report[i] = i == kRepCounts ? n_roots : 0u;
     }
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n_roots; i += gridDim.x * blockDim.x)
-        frontier0[i] = roots[i];
+        frontier0[i] = report[kRepRoots + i];
+}
+
+// A node's 9 words in registers (words past its length belong to its neighbours, or to the pad
+// behind the last bucket): three loads in place of nine.
+typedef uint32_t u32x4_a4 __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void load_node(const uint32_t* __restrict__ vpool, uint32_t va, uint32_t w[9]) {
+    const u32x4_a4 a = *reinterpret_cast<const u32x4_a4*>(vpool + va);
+    const u32x4_a4 b = *reinterpret_cast<const u32x4_a4*>(vpool + va + 4);
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) {
+        w[k] = a[k];
+        w[4 + k] = b[k];
+    }
+    w[8] = vpool[va + 8];
 }
 
 // mark children of the live nodes of `level` (an interior level): one lane per node, its
-// children's pointers, bitmap words and atomics issued together; a wavefront appends the
-// children it marked first with one atomic (in node order, child order within a node)
-__global__ __launch_bounds__(256) void k_gc_mark(const uint32_t* __restrict__ vpool, uint32_t* __restrict__ bitmap,
+// children's pointers, bitmap words and atomics issued together; a block appends the children it
+// marked first with one atomic (in node order, child order within a node). Bound by latency and by
+// the atomics, which leave the XCD. A word is read from the CU's own cache first: a bit seen there
+// is set for good, and the leaves that a terrain's columns share are mostly seen there; the rest
+// is asked for by atomics, all of a node's in flight before the first answer is looked at. The
+// levels of a terrain 8192 wide took 830 us with a read beyond the XCD per child and one atomic
+// at a time, and take 680 us.
+__global__ __launch_bounds__(256) void k_gc_mark(const uint32_t* __restrict__ vpool, uint32_t* bitmap,
                                                  const uint32_t* __restrict__ frontier, uint32_t* __restrict__ next,
                                                  uint32_t* counts, uint32_t level, uint32_t capCur, uint32_t cap,
                                                  uint64_t numVirtual, uint32_t* errors) {
@@ -69,30 +88,32 @@ __global__ __launch_bounds__(256) void k_gc_mark(const uint32_t* __restrict__ vp
     // block-uniform loop: the next frontier is appended with one atomic per block
     for (uint32_t b0 = blockIdx.x * blockDim.x; b0 < n; b0 += stride) {
         const uint32_t i = b0 + threadIdx.x;
-        uint32_t kid[8], nk = 0, firstBits = 0;
+        uint32_t node[9], nk = 0, firstBits = 0;
         if (i < n) {
-            const uint32_t va = frontier[i];
-            nk = __popc(vpool[va] & 0xFFu);
-#pragma unroll
-            for (uint32_t k = 0; k < 8; ++k) kid[k] = k < nk ? vpool[va + 1 + k] : 0u;
-            uint32_t w[8];
-            // shared children are marked by many parents: read first, so only the first few
-            // pay for the atomic on a hot bitmap word
-#pragma unroll
-            for (uint32_t k = 0; k < 8; ++k)
-                w[k] = k < nk && kid[k] < numVirtual
-                           ? __hip_atomic_load(&bitmap[kid[k] >> 5], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)
-                           : ~0u;
+            load_node(vpool, frontier[i], node);
+            nk = __popc(node[0] & 0xFFu);
+            uint32_t ask = 0;  // children whose bit is not seen set
 #pragma unroll
             for (uint32_t k = 0; k < 8; ++k) {
                 if (k >= nk) continue;
-                if (kid[k] >= numVirtual) {  // not an address of this table
-                    atomicOr(errors, GC_ERR_MAP);
-                    continue;
-                }
-                const uint32_t bit = 1u << (kid[k] & 31u);
-                if (!(w[k] & bit) && !(atomicOr(&bitmap[kid[k] >> 5], bit) & bit)) firstBits |= 1u << k;
+                if (node[1 + k] < numVirtual) ask |= 1u << k;
+                else atomicOr(errors, GC_ERR_MAP);  // not an address of this table
             }
+            uint32_t w[8];
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k)
+                w[k] = (ask >> k) & 1u ? __hip_atomic_load(&bitmap[node[1 + k] >> 5], __ATOMIC_RELAXED,
+                                                           __HIP_MEMORY_SCOPE_WORKGROUP)
+                                       : 0u;
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k)
+                if ((w[k] >> (node[1 + k] & 31u)) & 1u) ask &= ~(1u << k);
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k)
+                w[k] = (ask >> k) & 1u ? atomicOr(&bitmap[node[1 + k] >> 5], 1u << (node[1 + k] & 31u)) : ~0u;
+#pragma unroll
+            for (uint32_t k = 0; k < 8; ++k)
+                if (!((w[k] >> (node[1 + k] & 31u)) & 1u)) firstBits |= 1u << k;
         }
         // block scan of the marked counts, one atomic for the block
         const uint32_t cnt = __popc(firstBits);
@@ -120,214 +141,164 @@ __global__ __launch_bounds__(256) void k_gc_mark(const uint32_t* __restrict__ vp
         for (uint32_t k = 0; k < 8; ++k) {
             if (!((firstBits >> k) & 1u)) continue;
             if (base >= cap) atomicOr(errors, GC_ERR_CAP);
-            else next[base] = kid[k];
+            else next[base] = node[1 + k];
             ++base;
         }
     }
 }
 
-// gather live nodes of `level` with their children's new addresses (the forwarding array of
-// the level below) into tmp (9 words per node), and each node's bucket
-__global__ __launch_bounds__(256) void k_gc_gather(Geom g, const uint32_t* __restrict__ vpool,
-                                                   const uint32_t* __restrict__ frontier, const uint32_t* counts,
-                                                   uint32_t level, uint32_t maxLevel, uint32_t cap,
-                                                   const uint32_t* __restrict__ fwd, uint32_t* __restrict__ tmp,
-                                                   uint32_t* __restrict__ tlen, uint32_t* __restrict__ bkt) {
-    const uint32_t n = min(counts[level], cap);
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const uint32_t va = frontier[i];
-        uint32_t* out = tmp + (uint64_t)i * 9;
-        if (level == g.leaf_level()) {
-            const uint32_t w0 = vpool[va], w1 = vpool[va + 1];
-            out[0] = w0;
-            out[1] = w1;
-            tlen[i] = 2;
-            bkt[i] = g.bucket_from_hash(level, hash_leaf((uint64_t)w0 | ((uint64_t)w1 << 32)));
-            continue;
-        }
-        const uint32_t hdr = vpool[va];
-        const uint32_t nk = __popc(hdr & 0xFFu);
-        uint32_t c[8];
+// hash_words over words held in registers (no indexed access to them)
+__device__ __forceinline__ uint32_t hash_node(const uint32_t w[9], uint32_t n) {
+    uint32_t h = 0;
 #pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) c[k] = k < nk ? vpool[va + 1 + k] : 0u;
-        if (level != maxLevel) {
-#pragma unroll
-            for (uint32_t k = 0; k < 8; ++k)
-                if (k < nk) c[k] = fwd[c[k]];
-        }
-        uint32_t node[9];
-        node[0] = hdr;
-#pragma unroll
-        for (uint32_t k = 0; k < 8; ++k) node[1 + k] = c[k];
-        out[0] = hdr;
-#pragma unroll
-        for (uint32_t k = 0; k < 8; ++k)
-            if (k < nk) out[1 + k] = c[k];
-        tlen[i] = nk + 1;
-        bkt[i] = g.bucket_from_hash(level, hash_words(node, nk + 1));
+    for (uint32_t i = 0; i < 9; ++i) {
+        if (i >= n) break;
+        uint32_t k = w[i] * 0xcc9e2d51u;
+        k = (k << 15) | (k >> 17);
+        k *= 0x1b873593u;
+        h ^= k;
+        h = (h << 13) | (h >> 19);
+        h = h * 5u + 0xe6546b64u;
     }
+    return fmix32(h ^ n);
 }
 
-__global__ void k_gc_full(TableRef T, uint32_t level, uint32_t* full_nodes, uint32_t* errors) {
-    if (blockIdx.x != 0 || threadIdx.x != 0) return;
-    const Geom& g = T.g;
-    uint32_t node[9];
-    uint32_t n, h;
+// the words of a level's full node (its children: the full node of the level below); its length
+__device__ __forceinline__ uint32_t full_words(const Geom& g, uint32_t level, const uint32_t* full_nodes, uint32_t w[9]) {
     if (level == g.leaf_level()) {
-        node[0] = node[1] = 0xFFFFFFFFu;
-        n = 2;
-        h = hash_leaf(~0ull);
-    } else {
-        const uint32_t count = level < g.color_tree_levels ? 0u : (1u << (3 * (g.levels - level)));
-        node[0] = (count << 8) | 0xFFu;
-        for (int c = 0; c < 8; ++c) node[1 + c] = full_nodes[level + 1];
-        n = 9;
-        h = hash_words(node, 9);
+        w[0] = w[1] = 0xFFFFFFFFu;
+        return 2;
     }
-    const uint32_t va = table_append(T, level, g.bucket_from_hash(level, h), node, n);
-    if (va == kAppendBucketFull) atomicOr(errors, GC_ERR_BUCKET);
-    else if (va == kAppendPoolFull) atomicOr(errors, GC_ERR_POOL);
-    else full_nodes[level] = va;
+    const uint32_t count = level < g.color_tree_levels ? 0u : (1u << (3 * (g.levels - level)));
+    w[0] = (count << 8) | 0xFFu;
+    for (uint32_t c = 0; c < 8; ++c) w[1 + c] = full_nodes[level + 1];
+    return 9;
 }
 
-// The live nodes of a level are placed bucket by bucket: each node takes a rank within its
-// bucket (the bucket from k_gc_gather, the rank from k_gc_bucket), the buckets' ranges of a level-wide order follow from a scan of the
-// bucket counts (k_gc_tile_sums, k_gc_tile_scan, k_gc_tile_apply, k_gc_order), one lane per bucket lays its nodes out in rank order
-// with the append rule of table_append (a node that does not fit in the rest of its page starts
-// the next page; k_gc_layout), and every node is then written where it was placed
-// (k_gc_write). This is what appending the nodes one at a time in rank order gives, without a
-// compare-and-swap loop on each bucket's size.
-__global__ __launch_bounds__(256) void k_gc_bucket(uint32_t level, const uint32_t* counts, uint32_t cap,
-                                                   const uint32_t* __restrict__ bkt, uint32_t* __restrict__ rank,
-                                                   uint32_t* bcount) {
-    const uint32_t n = min(counts[level], cap);
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        rank[i] = atomicAdd(&bcount[bkt[i]], 1u);
-}
+// A live node on its way to its new place: 48 bytes, so that it moves in three aligned accesses
+// and a walk along a bucket's list reads one of them per node.
+struct alignas(16) GcRow {
+    uint32_t w[9];
+    uint32_t next;  // the next row of the bucket's list, plus one; 0 ends it
+    uint32_t va;    // the node's old address
+    uint32_t len;
+};
 
-// exclusive scan of the bucket counts of one level, in tiles of 1024 buckets: the tiles' sums
-// (k_gc_tile_sums), their exclusive scan (k_gc_tile_scan, one block), then each tile scanned
-// from its offset (k_gc_tile_apply)
-constexpr uint32_t kScanTile = 1024;
-__device__ __forceinline__ uint32_t block_incl_scan1024(uint32_t v, uint32_t* lds, uint32_t& total) {
-    const uint32_t lane = threadIdx.x & 63u, wv = threadIdx.x >> 6;
+// Gather the live nodes of `level` with their children's new addresses (the forwarding array of
+// the level below) into rows, each hung into the list of the bucket it belongs to: the exchange
+// that takes the list's head is the only atomic of a node, and its answer is the row's `next`. A
+// rank per node by an atomic add, a scan of the buckets' counts in three launches and a pass that
+// put the lengths in order took nine launches more per level (11 of 3 to 5 us each where a level
+// is small) and 200 us at the largest levels of a terrain 8192 wide.
+__global__ __launch_bounds__(256) void k_gc_gather(Geom g, const uint32_t* __restrict__ vpool,
+                                                   const uint32_t* __restrict__ frontier, uint32_t* report,
+                                                   uint32_t level, uint32_t maxLevel, uint32_t cap,
+                                                   const uint32_t* __restrict__ fwd, const uint32_t* full_nodes,
+                                                   GcRow* __restrict__ rows, uint32_t* head) {
+    const uint32_t n = min(report[kRepCounts + level], cap);
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        uint32_t w[9];
+        const uint32_t len = full_words(g, level, full_nodes, w);
+        report[kRepFull + level] = g.bucket_from_hash(level, len == 2 ? hash_leaf(~0ull) : hash_node(w, len));
+    }
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
+        GcRow r;
+        r.va = frontier[i];
+        uint32_t hash;
+        if (level == g.leaf_level()) {
 #pragma unroll
-    for (uint32_t off = 1; off < 64; off <<= 1) {
-        const uint32_t t = __shfl_up(v, off, 64);
-        if (lane >= off) v += t;
-    }
-    if (lane == 63) lds[wv] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        uint32_t run = 0;
-        for (uint32_t w = 0; w < kScanTile / 64; ++w) {
-            const uint32_t x = lds[w];
-            lds[w] = run;
-            run += x;
+            for (uint32_t k = 0; k < 9; ++k) r.w[k] = k < 2 ? vpool[r.va + k] : 0u;
+            r.len = 2;
+            hash = hash_leaf((uint64_t)r.w[0] | ((uint64_t)r.w[1] << 32));
+        } else {
+            load_node(vpool, r.va, r.w);
+            r.len = __popc(r.w[0] & 0xFFu) + 1;
+            if (level != maxLevel) {
+#pragma unroll
+                for (uint32_t k = 1; k < 9; ++k)
+                    if (k < r.len) r.w[k] = fwd[r.w[k]];
+            }
+            hash = hash_node(r.w, r.len);
         }
-        lds[kScanTile / 64] = run;
-    }
-    __syncthreads();
-    v += lds[wv];
-    total = lds[kScanTile / 64];
-    __syncthreads();  // lds is reused by the caller's next call
-    return v;
-}
-__global__ __launch_bounds__(kScanTile) void k_gc_tile_sums(const uint32_t* __restrict__ bcount, uint32_t nb,
-                                                           uint32_t* __restrict__ tileSum) {
-    __shared__ uint32_t lds[kScanTile / 64 + 1];
-    const uint32_t i = blockIdx.x * kScanTile + threadIdx.x;
-    uint32_t total;
-    block_incl_scan1024(i < nb ? bcount[i] : 0u, lds, total);
-    if (threadIdx.x == 0) tileSum[blockIdx.x] = total;
-}
-__global__ __launch_bounds__(kScanTile) void k_gc_tile_scan(uint32_t* __restrict__ tileSum, uint32_t nTiles) {
-    __shared__ uint32_t lds[kScanTile / 64 + 1];
-    uint32_t carry = 0;
-    for (uint32_t t0 = 0; t0 < nTiles; t0 += kScanTile) {  // block-uniform
-        const uint32_t t = t0 + threadIdx.x;
-        const uint32_t v = t < nTiles ? tileSum[t] : 0u;
-        uint32_t total;
-        const uint32_t incl = block_incl_scan1024(v, lds, total);
-        if (t < nTiles) tileSum[t] = carry + incl - v;
-        carry += total;
+        r.next = atomicExch(&head[g.bucket_global(level, g.bucket_from_hash(level, hash))], i + 1);
+        rows[i] = r;
     }
 }
-__global__ __launch_bounds__(kScanTile) void k_gc_tile_apply(const uint32_t* __restrict__ bcount, uint32_t nb,
-                                                            const uint32_t* __restrict__ tileSum,
-                                                            uint32_t* __restrict__ bstart) {
-    __shared__ uint32_t lds[kScanTile / 64 + 1];
-    const uint32_t i = blockIdx.x * kScanTile + threadIdx.x;
-    const uint32_t v = i < nb ? bcount[i] : 0u;
-    uint32_t total;
-    const uint32_t incl = block_incl_scan1024(v, lds, total);
-    if (i < nb) bstart[i] = tileSum[blockIdx.x] + incl - v;
-}
 
-// node lengths in level-wide (bucket, rank) order
-__global__ __launch_bounds__(256) void k_gc_order(uint32_t level, const uint32_t* counts, uint32_t cap,
-                                                  const uint32_t* __restrict__ tlen, const uint32_t* __restrict__ bkt,
-                                                  const uint32_t* __restrict__ rank, const uint32_t* __restrict__ bstart,
-                                                  uint32_t* __restrict__ olen) {
-    const uint32_t n = min(counts[level], cap);
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x)
-        olen[bstart[bkt[i]] + rank[i]] = tlen[i];
+// A block lays out `per` consecutive buckets of a level: a lane per bucket starts it with the
+// level's full node where that belongs to it, then walks its list and gives each node its place by
+// the append rule of table_append (a node that does not fit in the rest of its page starts the
+// next page), mapping the pages it starts; a node that no longer fits sets the error. This is what
+// appending the nodes one at a time in list order gives, without a compare-and-swap loop on the
+// bucket's size. The nodes and places go through LDS to all lanes of the block, which copy them
+// and record old -> new; places beyond the room there are copied by the walking lane. 64 buckets
+// a block: at 65536 buckets a level, 1024 blocks, so that the copies (bound by the latency of
+// their scattered accesses) have 16 wavefronts a CU.
+constexpr uint32_t kPlaceBuckets = 64, kPlaceList = 1024;
+__device__ __forceinline__ void move_row(const GcRow* __restrict__ rows, uint32_t i, uint32_t va, uint32_t* vpool,
+                                         uint32_t* fwd) {
+    const GcRow r = rows[i];
+#pragma unroll
+    for (uint32_t k = 0; k < 9; ++k)
+        if (k < r.len) vpool[va + k] = r.w[k];
+    fwd[r.va] = va;
 }
-
-// one lane per bucket: positions of its nodes in rank order, after what the bucket holds
-// already (the level's full node); ~0 for nodes that no longer fit
-__global__ __launch_bounds__(256) void k_gc_layout(Geom g, uint32_t level, uint32_t* bucket_sizes,
-                                                   const uint32_t* __restrict__ bcount,
-                                                   const uint32_t* __restrict__ bstart,
-                                                   const uint32_t* __restrict__ olen, uint32_t* __restrict__ opos,
-                                                   uint32_t* errors) {
+__global__ __launch_bounds__(256) void k_gc_place(TableRef T, uint32_t level, const uint32_t* report,
+                                                  uint32_t* full_nodes, const GcRow* __restrict__ rows,
+                                                  const uint32_t* __restrict__ head, uint32_t* fwd, uint32_t* errors) {
+    __shared__ uint2 list[kPlaceList];
+    __shared__ uint32_t listed;
+    const Geom& g = T.g;
     const uint32_t nb = g.buckets_per_level(level), ps = g.page_size, capB = g.bucket_size(level);
-    for (uint32_t b = blockIdx.x * blockDim.x + threadIdx.x; b < nb; b += gridDim.x * blockDim.x) {
-        uint32_t* bsPtr = &bucket_sizes[g.bucket_global(level, b)];
-        uint32_t cur = *bsPtr;
-        const uint32_t k0 = bstart[b], k1 = k0 + bcount[b];
+    if (threadIdx.x == 0) listed = 0;
+    __syncthreads();
+    const uint32_t b = blockIdx.x * kPlaceBuckets + threadIdx.x;
+    if (threadIdx.x < kPlaceBuckets && b < nb) {
+        const uint32_t bg = g.bucket_global(level, b);
+        uint32_t cur = 0;
+        if (b == report[kRepFull + level]) {
+            uint32_t w[9];
+            const uint32_t len = full_words(g, level, full_nodes, w);
+            const uint32_t va = g.make_ptr(level, b, 0);
+            if (len > capB) {
+                atomicOr(errors, GC_ERR_BUCKET);
+            } else {
+                cur = len;
+                if (!table_map_page(T, va / ps)) {
+                    atomicOr(errors, GC_ERR_POOL);
+                } else {
+                    for (uint32_t k = 0; k < len; ++k) T.vpool[va + k] = w[k];
+                    full_nodes[level] = va;
+                }
+            }
+        }
         bool full = false;
-        for (uint32_t k = k0; k < k1; ++k) {
-            const uint32_t len = olen[k];
+        for (uint32_t it = head[bg]; it && !full;) {
+            const GcRow* r = &rows[it - 1];
+            const uint32_t len = r->len, after = r->next;
             const uint32_t left = ps - cur % ps;
             const uint32_t start = (left != ps && left < len) ? cur + left : cur;
-            if (full || start + len > capB) {
+            if (start + len > capB) {
                 full = true;
-                opos[k] = ~0u;
-                continue;
+                atomicOr(errors, GC_ERR_BUCKET);
+                break;
             }
-            opos[k] = start;
             cur = start + len;
+            const uint32_t va = g.make_ptr(level, b, start);
+            if (start % ps == 0 && !table_map_page(T, va / ps)) {
+                atomicOr(errors, GC_ERR_POOL);
+            } else {
+                const uint32_t at = atomicAdd(&listed, 1u);
+                if (at < kPlaceList) list[at] = make_uint2(it - 1, va);
+                else move_row(rows, it - 1, va, T.vpool, fwd);
+            }
+            it = after;
         }
-        if (full) atomicOr(errors, GC_ERR_BUCKET);
-        *bsPtr = cur;
+        T.bucket_sizes[bg] = cur;
     }
-}
-
-// every node written where it was placed; its new address into the forwarding array
-__global__ __launch_bounds__(256) void k_gc_write(TableRef T, uint32_t level, const uint32_t* counts, uint32_t cap,
-                                                  const uint32_t* __restrict__ frontier,
-                                                  const uint32_t* __restrict__ tmp, const uint32_t* __restrict__ tlen,
-                                                  const uint32_t* __restrict__ bkt, const uint32_t* __restrict__ rank,
-                                                  const uint32_t* __restrict__ bstart,
-                                                  const uint32_t* __restrict__ opos, uint32_t* __restrict__ fwd,
-                                                  uint32_t* errors) {
-    const uint32_t n = min(counts[level], cap);
-    const uint32_t ps = T.g.page_size;
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
-        const uint32_t b = bkt[i];
-        const uint32_t start = opos[bstart[b] + rank[i]];
-        if (start == ~0u) continue;  // the bucket overflowed (error set by the layout)
-        const uint32_t va = T.g.make_ptr(level, b, start);
-        if (start % ps == 0 && !table_map_page(T, va / ps)) {
-            atomicOr(errors, GC_ERR_POOL);
-            continue;
-        }
-        const uint32_t* node = tmp + (uint64_t)i * 9;
-        const uint32_t len = tlen[i];
-        for (uint32_t k = 0; k < len; ++k) T.vpool[va + k] = node[k];
-        fwd[frontier[i]] = va;
-    }
+    __syncthreads();
+    const uint32_t n = min(listed, kPlaceList);
+    for (uint32_t q = threadIdx.x; q < n; q += blockDim.x) move_row(rows, list[q].x, list[q].y, T.vpool, fwd);
 }
 
 // every kept root -> its address after GC
@@ -363,10 +334,7 @@ static uint32_t remap(const std::vector<uint32_t>& from, const std::vector<uint3
 }
 
 // GC scratch slots (fixed indices; frontier l at kSlotFrontier + l)
-enum : uint32_t {
-    kSlotBitmap, kSlotCounts, kSlotErrors, kSlotRoots, kSlotTmp, kSlotTlen, kSlotBkt, kSlotRank, kSlotOlen,
-    kSlotOpos, kSlotBcount, kSlotBstart, kSlotTileSum, kSlotFwd, kSlotUsed, kSlotFrontier
-};
+enum : uint32_t { kSlotBitmap, kSlotReport, kSlotRows, kSlotFwd, kSlotUsed, kSlotFrontier };
 
 // slot k of the context's GC scratch with at least `bytes` (grown by a quarter beyond the
 // request, so tables that grow between collections reallocate rarely)
@@ -433,29 +401,16 @@ static hd_status gc_run(hd_ctx* ctx, uint32_t max_level, uint32_t* extra, uint32
     // scratch from the context's slots (kept between calls; every kernel is given its sizes)
     auto alloc = [&](uint32_t slot, void** p, uint64_t bytes) -> hipError_t { return gc_slot(ctx, slot, bytes, p); };
     auto release = [&]() { hipStreamSynchronize(s); };
-    const uint64_t bitmapWords = (g.total_virtual() + 31) / 32;
-    uint32_t *bitmap, *counts, *errors, *tmp, *tlen, *fwd, *droots;
+    // the mark bitmap and, behind it, the list head of every bucket
+    const uint64_t bitmapWords = (g.total_virtual() + 31) / 32, headWords = g.total_buckets();
+    uint32_t *bitmap, *report, *fwd;
+    GcRow* rows;
     std::vector<uint32_t*> frontier(max_level + 1, nullptr);
-    hipError_t e = alloc(kSlotBitmap, (void**)&bitmap, bitmapWords * 4);
-    if (e == hipSuccess) e = alloc(kSlotCounts, (void**)&counts, 64 * 4);
-    if (e == hipSuccess) e = alloc(kSlotErrors, (void**)&errors, 4);
-    if (e == hipSuccess) e = alloc(kSlotRoots, (void**)&droots, (uint64_t)nRoots * 4);
+    hipError_t e = alloc(kSlotBitmap, (void**)&bitmap, (bitmapWords + headWords) * 4);
+    if (e == hipSuccess) e = alloc(kSlotReport, (void**)&report, ((uint64_t)kRepRoots + nRoots) * 4);
     for (uint32_t l = 0; l <= max_level && e == hipSuccess; ++l)
         e = alloc(kSlotFrontier + l, (void**)&frontier[l], (uint64_t)fcap(l) * 4);
-    if (e == hipSuccess) e = alloc(kSlotTmp, (void**)&tmp, (uint64_t)cap * 36);
-    if (e == hipSuccess) e = alloc(kSlotTlen, (void**)&tlen, (uint64_t)cap * 4);
-    // placement scratch: bucket and rank per node, lengths and positions in placement order,
-    // count and start per bucket of a level
-    uint32_t maxBuckets = 1;
-    for (uint32_t l = 0; l <= max_level; ++l) maxBuckets = std::max(maxBuckets, g.buckets_per_level(l));
-    uint32_t *bkt, *rank, *olen, *opos, *bcount, *bstart, *tileSum;
-    if (e == hipSuccess) e = alloc(kSlotBkt, (void**)&bkt, (uint64_t)cap * 4);
-    if (e == hipSuccess) e = alloc(kSlotRank, (void**)&rank, (uint64_t)cap * 4);
-    if (e == hipSuccess) e = alloc(kSlotOlen, (void**)&olen, (uint64_t)cap * 4);
-    if (e == hipSuccess) e = alloc(kSlotOpos, (void**)&opos, (uint64_t)cap * 4);
-    if (e == hipSuccess) e = alloc(kSlotBcount, (void**)&bcount, (uint64_t)maxBuckets * 4);
-    if (e == hipSuccess) e = alloc(kSlotBstart, (void**)&bstart, (uint64_t)maxBuckets * 4);
-    if (e == hipSuccess) e = alloc(kSlotTileSum, (void**)&tileSum, (uint64_t)(maxBuckets / kScanTile + 1) * 4);
+    if (e == hipSuccess) e = alloc(kSlotRows, (void**)&rows, (uint64_t)cap * sizeof(GcRow));
     // old address -> new address of every live node: one word per virtual address (written
     // for live nodes only, read only for them)
     if (e == hipSuccess) e = alloc(kSlotFwd, (void**)&fwd, (uint64_t)g.total_virtual() * 4);
@@ -464,16 +419,17 @@ static hd_status gc_run(hd_ctx* ctx, uint32_t max_level, uint32_t* extra, uint32
         gc_scratch_free(ctx);  // give back what a smaller call could not reuse
         return hip_fail(ctx, e, "GC scratch");
     }
-    k_gc_fill<<<1024, 256, 0, s>>>(bitmap, bitmapWords, 0u);
-    k_gc_fill<<<1, 64, 0, s>>>(errors, 1, 0u);
+    uint32_t *head = bitmap + bitmapWords, *errors = report, *counts = report + kRepCounts, *droots = report + kRepRoots;
+    auto grid = [&](uint32_t l) { return std::min((fcap(l) + 255) / 256, kGcGrid); };
+    k_gc_fill<<<2048, 256, 0, s>>>(bitmap, bitmapWords + headWords, 0u);
     e = hipMemcpyAsync(droots, roots.data(), (uint64_t)nRoots * 4, hipMemcpyHostToDevice, s);
     if (e != hipSuccess) {
         release();
         return hip_fail(ctx, e, "GC roots");
     }
-    k_gc_seed<<<(nRoots + 255) / 256, 256, 0, s>>>(frontier[0], counts, droots, nRoots, g.levels);
+    k_gc_seed<<<(nRoots + 255) / 256, 256, 0, s>>>(frontier[0], report, nRoots);
     for (uint32_t l = 0; l < max_level; ++l)
-        k_gc_mark<<<kGcGrid, 256, 0, s>>>(ctx->vpool, bitmap, frontier[l], frontier[l + 1], counts, l, fcap(l),
+        k_gc_mark<<<grid(l), 256, 0, s>>>(ctx->vpool, bitmap, frontier[l], frontier[l + 1], counts, l, fcap(l),
                                           fcap(l + 1), g.total_virtual(), errors);
     {  // nothing has been modified yet: stop here if the mark overflowed or met a bad pointer
         uint32_t markErr = 0;
@@ -487,31 +443,20 @@ static hd_status gc_run(hd_ctx* ctx, uint32_t max_level, uint32_t* extra, uint32
     }
     TableRef T{g, ctx->vpool, ctx->page_table, ctx->bucket_sizes, ctx->counters + 0, ctx->cfg.pool_pages};
     for (uint32_t l = max_level; l != (uint32_t)-1; --l) {
-        k_gc_gather<<<kGcGrid, 256, 0, s>>>(g, ctx->vpool, frontier[l], counts, l, max_level, cap, fwd, tmp, tlen, bkt);
-        // reset the level's buckets, then the full node first, then the live nodes
-        const uint32_t b0 = g.bucket_global(l, 0);
-        k_gc_fill<<<256, 256, 0, s>>>(ctx->bucket_sizes + b0, g.buckets_per_level(l), 0u);
-        k_gc_full<<<1, 1, 0, s>>>(T, l, ctx->full_nodes, errors);
-        const uint32_t nb = g.buckets_per_level(l);
-        k_gc_fill<<<256, 256, 0, s>>>(bcount, nb, 0u);
-        k_gc_bucket<<<kGcGrid, 256, 0, s>>>(l, counts, cap, bkt, rank, bcount);
-        const uint32_t nTiles = (nb + kScanTile - 1) / kScanTile;
-        k_gc_tile_sums<<<nTiles, kScanTile, 0, s>>>(bcount, nb, tileSum);
-        k_gc_tile_scan<<<1, kScanTile, 0, s>>>(tileSum, nTiles);
-        k_gc_tile_apply<<<nTiles, kScanTile, 0, s>>>(bcount, nb, tileSum, bstart);
-        k_gc_order<<<kGcGrid, 256, 0, s>>>(l, counts, cap, tlen, bkt, rank, bstart, olen);
-        k_gc_layout<<<(nb + 255) / 256, 256, 0, s>>>(g, l, ctx->bucket_sizes, bcount, bstart, olen, opos, errors);
-        k_gc_write<<<kGcGrid, 256, 0, s>>>(T, l, counts, cap, frontier[l], tmp, tlen, bkt, rank, bstart, opos, fwd,
-                                           errors);
+        k_gc_gather<<<grid(l), 256, 0, s>>>(g, ctx->vpool, frontier[l], report, l, max_level, fcap(l), fwd,
+                                            ctx->full_nodes, rows, head);
+        k_gc_place<<<(g.buckets_per_level(l) + kPlaceBuckets - 1) / kPlaceBuckets, 256, 0, s>>>(
+            T, l, report, ctx->full_nodes, rows, head, fwd, errors);
     }
     k_gc_roots<<<(nRoots + 255) / 256, 256, 0, s>>>(fwd, droots, nRoots, errors);
-    uint32_t err = 0;
-    std::vector<uint32_t> newRoots(nRoots);
-    std::vector<uint32_t> cnt(max_level + 1);
-    HD_HIP(ctx, hipMemcpyAsync(&err, errors, 4, hipMemcpyDeviceToHost, s));
-    HD_HIP(ctx, hipMemcpyAsync(newRoots.data(), droots, (uint64_t)nRoots * 4, hipMemcpyDeviceToHost, s));
-    HD_HIP(ctx, hipMemcpyAsync(cnt.data(), counts, cnt.size() * 4, hipMemcpyDeviceToHost, s));
+    if (stats)
+        k_gc_level_used<<<dim3(64, g.levels), 256, 0, s>>>(g, ctx->bucket_sizes,
+                                                           (unsigned long long*)(report + kRepUsed));
+    std::vector<uint32_t> rep(kRepRoots + nRoots);
+    HD_HIP(ctx, hipMemcpyAsync(rep.data(), report, rep.size() * 4, hipMemcpyDeviceToHost, s));
     e = hipStreamSynchronize(s);
+    const uint32_t err = rep[0];
+    const std::vector<uint32_t> newRoots(rep.begin() + kRepRoots, rep.end());
     release();
     if (e != hipSuccess || err) {
         // levels were rewritten in place up to the failure: the table no longer holds the DAG,
@@ -541,17 +486,14 @@ static hd_status gc_run(hd_ctx* ctx, uint32_t max_level, uint32_t* extra, uint32
         ctx->redo.clear();
     }
     if (stats) {
-        uint64_t live = 0;
-        for (uint32_t v : cnt) live += v;
-        uint64_t before = 0;
-        for (uint32_t l = 0; l <= max_level; ++l) before += used[l];
+        uint64_t live = 0, before = 0, after = 0;
+        for (uint32_t l = 0; l <= max_level; ++l) {
+            live += rep[kRepCounts + l];
+            before += used[l];
+            after += rep[kRepUsed + 2 * l] | (uint64_t)rep[kRepUsed + 2 * l + 1] << 32;
+        }
         stats[0] = live;
         stats[1] = before;
-        std::vector<uint64_t> used2;
-        const hd_status st = level_used(ctx, s, used2);
-        if (st != HD_OK) return st;
-        uint64_t after = 0;
-        for (uint32_t l = 0; l <= max_level; ++l) after += used2[l];
         stats[2] = after;
         stats[3] = 0;
     }
