@@ -12,6 +12,7 @@
 
 #include <algorithm>
 
+#include "hd_color_dev.h"
 #include "hd_ctx.h"
 
 namespace hd {
@@ -578,8 +579,6 @@ struct Leaf {
     uint64_t n_blocks, n_macro, offset;
 };
 
-__device__ __forceinline__ uint32_t hdr_index(uint32_t h) { return h & 16383u; }
-__device__ __forceinline__ uint32_t hdr_bpw(uint32_t h) { return (h >> 16) == 0xFFFFu ? 0u : ((h >> 14) & 3u) + 1u; }
 
 // color_utils.h:112-148 (big-endian 16-bit window over the byte-swapped weight words)
 template <bool kCount>
@@ -599,36 +598,6 @@ __device__ __forceinline__ uint32_t extract_bits(uint32_t bits, const uint32_t* 
     const uint32_t dst = (b0 << 8) | b1;
     const uint32_t shift = 16u - bits - (uint32_t)(bitPtr & 7u);
     return (dst >> shift) & ((1u << bits) - 1u);
-}
-
-// The block of blocks[lo .. hi] that holds colour `local` of its macro block: the last one that
-// starts at or before it (block starts ascend; the first starts at 0), and its position. Three
-// probes a step in flight together: half the chain of a binary search. Same block as that search,
-// since no two blocks of a macro block start at the same colour.
-__device__ __forceinline__ uint64_t block_of(const uint64_t* __restrict__ blocks, uint32_t lo, uint32_t hi,
-                                             uint32_t local, uint32_t& at) {
-    uint64_t blk = blocks[lo];
-    while (lo < hi) {
-        const uint32_t len = hi - lo + 1;
-        const uint32_t p1 = lo + max(len / 4, 1u), p2 = min(lo + max(len / 2, 1u), hi), p3 = min(p2 + max(len / 4, 1u), hi);
-        const uint64_t b1 = blocks[p1], b2 = blocks[p2], b3 = blocks[p3];
-        if (hdr_index((uint32_t)b3) <= local) {
-            lo = p3;
-            blk = b3;
-        } else if (hdr_index((uint32_t)b2) <= local) {
-            lo = p2;
-            blk = b2;
-            hi = p3 - 1;
-        } else if (hdr_index((uint32_t)b1) <= local) {
-            lo = p1;
-            blk = b1;
-            hi = p2 - 1;
-        } else {
-            hi = p1 - 1;
-        }
-    }
-    at = lo;
-    return blk;
 }
 
 // variable_weight_size_colors.h:343-413 + CompressedColor::get_color (:144-154)
