@@ -1031,56 +1031,67 @@ __device__ __forceinline__ uint32_t item_node(const Items& I, uint32_t i) {
     const uint32_t v = I.nidx[i];
     return I.state[i] == kStateDuplicate ? I.nidx[v] : v;
 }
+// the two halves of hash_words' step over one word
+__device__ __forceinline__ uint32_t hash_mix(uint32_t w) {
+    w *= 0xcc9e2d51u;
+    return ((w << 15) | (w >> 17)) * 0x1b873593u;
+}
+__device__ __forceinline__ uint32_t hash_step(uint32_t h, uint32_t mixed) {
+    h ^= mixed;
+    return ((h << 13) | (h >> 19)) * 5u + 0xe6546b64u;
+}
+// A lane per child slot, 8 lanes an item. Bound by the chain of loads behind a child that is an
+// item (kind, index, state, node, the node of the item it duplicates): walked by 8 lanes at once,
+// from coalesced slots. A thread per item walked them one after another, with the node's words in
+// scratch memory: the 11 launches of a pass over 4096 editors took 3261 us, and take 1122 us.
 __device__ __forceinline__ void d_build(const EditPass& P, uint32_t l, VGrid G) {
     const uint32_t n = min(P.count[l], P.cap[l]);
     if (*P.errors) return;
     d_hset_clear(P, l, G);
     const Items I = P.items[l];
     const Items C = P.items[l + 1];
-    const uint32_t D = P.levels, ctl = P.ctl;
-    for (uint32_t i = G.block * blockDim.x + threadIdx.x; i < n; i += G.nblocks * blockDim.x) {
-        uint32_t node[9];
-        uint32_t nn = 1, mask = 0;
-        uint64_t count = 0;
-        bool changed = false;
-        for (uint32_t c = 0; c < 8; ++c) {
-            const uint32_t slot = i * 8 + c;
-            const uint32_t kind = I.ckind[slot];
-            uint32_t idx, cnt;
-            if (kind == KIND_ITEM) {
-                const uint32_t ci = I.cval[slot];
-                idx = item_node(C, ci);
-                cnt = C.ncount[ci];
-                I.cnew[slot] = cnt;
-            } else {
-                idx = I.cval[slot];
-                cnt = I.cnew[slot];
-            }
-            changed |= idx != I.corig[slot];
-            if (idx != kInvalidNode) {
-                mask |= 1u << c;
-                node[nn++] = idx;
-                count += cnt;
-            }
+    const uint32_t c = threadIdx.x & 7u, group = threadIdx.x & 56u;  // the lane's child; its item's first lane
+    for (uint64_t t = (uint64_t)G.block * blockDim.x + threadIdx.x; t < (uint64_t)n * 8; t += (uint64_t)G.nblocks * blockDim.x) {
+        const uint32_t slot = (uint32_t)t, i = (uint32_t)(t >> 3);
+        const uint32_t kind = I.ckind[slot], val = I.cval[slot], was = I.corig[slot];
+        uint32_t idx = val, cnt;
+        if (kind == KIND_ITEM) {
+            idx = item_node(C, val);
+            cnt = C.ncount[val];
+            I.cnew[slot] = cnt;
+        } else {
+            cnt = I.cnew[slot];
         }
-        (void)D;
-        if (l >= ctl && count >= (1u << 24)) set_error(P.errors, ERR_HEADER);
-        I.ncount[i] = (uint32_t)count;
-        if (!changed) {
-            I.nidx[i] = I.orig[i];
-            I.state[i] = 0;
+        const bool has = idx != kInvalidNode;
+        const uint32_t mask = (uint32_t)(__ballot(has) >> group) & 0xFFu;
+        const bool changed = ((uint32_t)(__ballot(idx != was) >> group) & 0xFFu) != 0;
+        uint32_t count = has ? cnt : 0u;
+#pragma unroll
+        for (uint32_t d = 1; d < 8; d <<= 1) count += __shfl_xor(count, d, 8);
+        // (eight counts below 2^24 cannot wrap the sum)
+        if (l >= P.ctl && (count >= (1u << 24) || (has && cnt >= (1u << 24)))) set_error(P.errors, ERR_HEADER);
+        // hash_words over the header and the children: each lane mixes its own word, the chain
+        // takes them in child order
+        const uint32_t head = mask | (l >= P.ctl ? count << 8 : 0u);
+        const uint32_t mixed = hash_mix(idx), len = 1u + (uint32_t)__popc(mask);
+        uint32_t h = hash_step(0u, hash_mix(head));
+#pragma unroll
+        for (uint32_t k = 0; k < 8; ++k) {
+            const uint32_t m = __shfl(mixed, k, 8);
+            if ((mask >> k) & 1u) h = hash_step(h, m);
+        }
+        const bool pending = changed && mask;
+        if (pending && has) I.cont[i * 9 + 1 + __popc(mask & ((1u << c) - 1u))] = idx;
+        if (c) continue;
+        I.ncount[i] = count;
+        I.state[i] = pending ? kStatePending : kStateKnown;
+        if (!pending) {
+            I.nidx[i] = changed ? kInvalidNode : I.orig[i];
             continue;
         }
-        if (!mask) {
-            I.nidx[i] = kInvalidNode;
-            I.state[i] = 0;
-            continue;
-        }
-        node[0] = mask | (l >= ctl ? (uint32_t)(count << 8) : 0u);
-        for (uint32_t k = 0; k < nn; ++k) I.cont[i * 9 + k] = node[k];
-        I.clen[i] = nn;
-        I.hash[i] = hash_words(node, nn);
-        I.state[i] = 1;
+        I.cont[i * 9] = head;
+        I.clen[i] = len;
+        I.hash[i] = fmix32(h ^ len);
     }
 }
 __global__ __launch_bounds__(256) void k_build(EditPass P, uint32_t l) {
@@ -1205,12 +1216,7 @@ __device__ __forceinline__ uint32_t node_hash(const NodeWords& c) {
 #pragma unroll
     for (uint32_t i = 0; i < 9; ++i) {
         if (i >= c.n) break;
-        uint32_t k = c.w[i] * 0xcc9e2d51u;
-        k = (k << 15) | (k >> 17);
-        k *= 0x1b873593u;
-        h ^= k;
-        h = (h << 13) | (h >> 19);
-        h = h * 5u + 0xe6546b64u;
+        h = hash_step(h, hash_mix(c.w[i]));
     }
     return fmix32(h ^ c.n);
 }
@@ -3511,7 +3517,7 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
                 if (special) k_leaf<true><<<gl, 256, 0, s>>>(P);
                 else k_leaf<false><<<units(b, 256), 256, 0, s>>>(P);
                 break;
-            case ST_BUILD: k_build<<<units(b, 256), 256, 0, s>>>(P, l); break;  // a thread per item
+            case ST_BUILD: k_build<<<units(8 * b, 256), 256, 0, s>>>(P, l); break;  // 8 lanes an item
             case ST_NODES:
                 if (b <= kNodesItems || !bounded) {  // a wavefront per item
                     k_nodes<<<units(b, 4), 256, 0, s>>>(P, l);
