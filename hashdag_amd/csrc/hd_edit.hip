@@ -13,16 +13,21 @@
 //
 //   expand   levels 0 .. L-1, top-down: per (item, child) filter the edit list, classify the
 //            child (keep / empty / full / item), append child items (atomic slot allocation)
-//   build    levels L .. 0, bottom-up: new leaf masks (one wavefront per leaf item, one lane
-//            per voxel) and new interior nodes; unchanged nodes keep their index
+//   build    levels L .. 0, bottom-up: new leaf masks (a thread per leaf item) and new interior
+//            nodes (8 lanes an item); unchanged nodes keep their index
 //   dedup    identical new nodes of a level collapse to one representative (device hash set)
-//   find     one wavefront per representative scans its bucket in 64-word strides
+//   find     one wavefront per representative scans its bucket, as it was before the level's adds
 //   add      misses reserve space with a CAS on the bucket size (page padding rule of
 //            hash_table.h:418-442) and write the node; new pages are numbered from poolTop
+//            (dedup, find and add of a level of few items are one launch)
 //   colours  per colour subtree (level color_tree_levels item): prefix sums of new / old voxel
 //            counts, emission of every new colour (copied, filled, or folded per voxel), then
-//            one workgroup re-encodes the subtree's leaf (block / weight / macro-block rules of
-//            variable_weight_size_colors.h:557-721) into the colour arena
+//            the subtrees' leaves re-encoded in segments of 4096 colours over the whole chip:
+//            count, offsets, write (block / weight / macro-block rules of
+//            variable_weight_size_colors.h:557-721)
+//
+// The levels around the root, whose items fit LDS, go through one workgroup each way
+// (k_top_expand, k_top_nodes).
 //
 // Kernels read item counts from device memory (grid-stride loops), so a pass needs no host
 // round trip and can be captured in a HIP graph.
