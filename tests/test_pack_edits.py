@@ -37,10 +37,27 @@ def test_same_bytes(name, edits):
 
 
 @pytest.mark.parametrize("bad", [(0, (1.0, 2.0), 3.0), (0, (1.0,), 3.0), (0, (1.0, 2.0, 3.0, 4.0), 1.0), (0, None, 1.0),
-                                 (0, (1.0, 2.0, "x"), 1.0), ("k", (1.0, 2.0, 3.0), 1.0), (0, (1.0, 2.0, 3.0), None)])
+                                 (0, (1.0, 2.0, "x"), 1.0), ("k", (1.0, 2.0, 3.0), 1.0), (0, (1.0, 2.0, 3.0), None),
+                                 (0, (1.0, None, 2.0), 3.0), (0, (1.0, np.datetime64("2020"), 2.0), 3.0)])
 def test_same_refusals(bad):
     for edits in ([(0, (1.0, 2.0, 3.0), 4.0)] * 30 + [bad], [bad] * 20):
         with pytest.raises(Exception) as want:
             plain(edits)
         with pytest.raises(want.type):
             pack_edits(edits)
+
+
+def test_numpy_error_state_of_the_caller():
+    """Values that leave float32's range pack alike whatever numpy is told to do about it."""
+    edits = [(0, (1e-50, 1e300, 2.0), 1e-60)] * 20
+    with np.errstate(all="raise"):
+        assert bytes(pack_edits(edits)) == plain(edits)
+
+
+def test_centres_that_are_read_once():
+    """A centre that is an iterator is read by one of the forms only."""
+    def edits(bad=False):
+        return [(0, iter((1.0, 2.0, 3.0)), 4.0) for _ in range(19)] + [(0, (1.0, None if bad else 0.0, 2.0), 3.0)]
+    assert bytes(pack_edits(edits())) == plain(edits())
+    with pytest.raises(TypeError):
+        pack_edits(edits(bad=True))
