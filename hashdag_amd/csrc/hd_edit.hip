@@ -3414,7 +3414,7 @@ static void level_bounds(const EditPass& P, const DevEdit* e, uint32_t n, uint64
     }
 }
 
-constexpr uint32_t kWideEdits = 8, kWideItems = 512;
+constexpr uint32_t kWideEdits = 8, kWideEditsBlock = 64, kWideItems = 512;
 constexpr uint32_t kTopItems = 128, kNodesItems = 1u << 12;
 
 hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hipStream_t s, PassReadback* rb,
@@ -3434,31 +3434,36 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
         gridMax = std::max(gridMax, grid[l]);
     }
     P.single_edit = (n == 1 && !dN) ? 1u : 0u;
+    const uint32_t D = P.levels, L = D - 2;
+    // one cooperative launch for passes of at most edit_persist_max edits (not under capture);
+    // otherwise a pass with at most edit_block_max work items on every level (by the editors'
+    // boxes) is one single-workgroup launch, and any other pass a launch per step over grids
+    // sized for each level, but for its levels around the root
+    const bool cooperative = !dN && n <= ctx->edit_persist_max;
+    uint64_t largest = 0;
+    for (uint32_t l = 0; l <= L && l < kMaxEditLevels; ++l) largest = std::max(largest, bound[l]);
+    const bool smallPass = !cooperative && largest <= (uint64_t)ctx->edit_block_max;
     // a wavefront per child slot where a level's items hold long edit lists: passes over at
     // least kWideEdits editors, on levels with at most kWideItems items (the grid's two blocks
-    // per item hold a wavefront per slot)
+    // per item hold a wavefront per slot). A single workgroup has four wavefronts for all slots and
+    // takes a thread per slot until the lists are longer (8 to 48 editors: 1.6 to 4.1 ms a pass with
+    // a wavefront a slot from 8 editors on, 0.73 to 1.96 ms from 64 on).
     P.wide_levels = 0;
-    if (!dN && n >= kWideEdits)
+    if (!dN && n >= (smallPass ? kWideEditsBlock : kWideEdits))
         for (uint32_t l = 0; l < kMaxEditLevels && l < 32; ++l)
             if (bound[l] <= kWideItems) P.wide_levels |= 1u << l;
-    const uint32_t D = P.levels, L = D - 2;
     k_init_pass<<<(std::max<uint32_t>(n, 1) + 255) / 256, 256, 0, s>>>(P, ctx->d_root, ctx->root, first, n, dN);
     // a plain pass counts its edited voxels on the way; the others' are counted from the editors
     if (n > 1 || dN) launch_count_voxels(P.edits + first, n, dN, 1u << D, P.stat_voxels, s);
     StepList sl = pass_step_list(D, P.ctl, colors);
-    // one cooperative launch for passes of at most edit_persist_max edits (not under capture)
-    if (!dN && n <= ctx->edit_persist_max)
+    if (cooperative)
         return special ? launch_persistent<true>(ctx, P, sl, s) : launch_persistent<false>(ctx, P, sl, s);
-    // otherwise a pass with at most edit_block_max work items on every level (by the editors'
-    // boxes) is one single-workgroup launch, and any other pass a launch per step over grids
-    // sized for each level. (Running only a bigger pass's small levels in a workgroup was
-    // slower: a workgroup's four wavefronts scan the buckets of a level's finds one after
-    // another, where a launch gives each its own wavefront.)
-    uint64_t largest = 0;
-    for (uint32_t l = 0; l <= L && l < kMaxEditLevels; ++l) largest = std::max(largest, bound[l]);
-    const bool smallPass = largest <= (uint64_t)ctx->edit_block_max;
-    const auto small = [&](uint32_t) { return smallPass; };
-    // a wavefront per task slot (the task count is on the device), at most 2^18 of them
+    if (smallPass) {
+        if (special) k_pass_block<true><<<1, 256, 0, s>>>(P, sl, 0, sl.n, ctx->d_root);
+        else k_pass_block<false><<<1, 256, 0, s>>>(P, sl, 0, sl.n, ctx->d_root);
+        HD_HIP(ctx, hipGetLastError());
+        return HD_OK;
+    }
     const bool bounded = hostEdits && !dN;  // bound[] from the editors' boxes
     // levels [0, topExpand) expand in k_top_expand, levels topNodes .. 0 build and enter their
     // nodes in k_top_nodes (~0: none)
@@ -3477,14 +3482,6 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
     const uint32_t segBlocks =
         (uint32_t)std::min<uint64_t>(std::max<uint64_t>((maxSegs + kEncWaves - 1) / kEncWaves, 1u), 4096u);
     for (uint32_t i = 0; i < sl.n;) {
-        if (small(sl.step[i])) {
-            uint32_t j = i + 1;
-            while (j < sl.n && small(sl.step[j])) ++j;
-            if (special) k_pass_block<true><<<1, 256, 0, s>>>(P, sl, i, j, ctx->d_root);
-            else k_pass_block<false><<<1, 256, 0, s>>>(P, sl, i, j, ctx->d_root);
-            i = j;
-            continue;
-        }
         const uint32_t st = sl.step[i] >> 8;
         // the small levels around the root, together (not while bytes are counted: d_expand counts
         // the descent's)
