@@ -3415,7 +3415,8 @@ static void level_bounds(const EditPass& P, const DevEdit* e, uint32_t n, uint64
 }
 
 constexpr uint32_t kWideEdits = 8, kWideEditsBlock = 64, kWideItems = 512;
-constexpr uint32_t kTopItems = 128, kNodesItems = 1u << 12;
+constexpr uint32_t kTopItems = 128, kNodesItems = 1u << 12, kNodesEdits = 256;
+constexpr uint32_t kPieceItems = 4096;
 
 hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hipStream_t s, PassReadback* rb,
                        const uint32_t* dN, bool special, const EditScratch* scratch, const DevEdit* hostEdits) {
@@ -3521,7 +3522,7 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
                 break;
             case ST_BUILD: k_build<<<units(8 * b, 256), 256, 0, s>>>(P, l); break;  // 8 lanes an item
             case ST_NODES:
-                if (b <= kNodesItems || !bounded) {  // a wavefront per item
+                if (dN ? n < kNodesEdits : b <= kNodesItems) {  // a wavefront per item
                     k_nodes<<<units(b, 4), 256, 0, s>>>(P, l);
                 } else {
                     k_dedup<<<units(b, 256), 256, 0, s>>>(P, l);  // a thread per item
@@ -3534,7 +3535,7 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
             case ST_CTREE: k_color_tree<<<gridMax, 256, 0, s>>>(P); break;
             // colour copies: a wavefront per slot (per item at the leaf parents)
             case ST_CCOPY: {
-                const bool few = bounded && b <= 4096;
+                const bool few = bounded && b <= kPieceItems;
                 if (few) k_color_copy<<<units((8 * b) << 3, 4), 256, 0, s>>>(P, l, 3, 0);
                 else k_color_copy<<<units(bounded ? b : 8 * b, 4), 256, 0, s>>>(P, l, 0, bounded ? 3 : 0);
                 break;

@@ -103,3 +103,32 @@ def test_edit_only_graph_matches_oracle():
     assert np.array_equal(canonical(dag), before)
     graph.close()
     dag.close()
+
+
+@pytest.mark.parametrize("max_edits", [255, 256])
+def test_graph_on_both_sides_of_the_node_steps_rule(max_edits):
+    """Captured passes enter a level's nodes in one step or, from 256 editors on, in three: full
+    lists, short ones and an undone one, over and over, against the oracle."""
+    from hashdag_amd import HashDAG
+    from hashdag_amd.graph import FrameGraph
+    from oracle import OracleColors, OracleDAG
+    from tests.test_edit_gpu import assert_same
+    p, sc, g = scene("d13")
+    od = OracleDAG.from_basic(g, sc.dag, POOL_PAGES)
+    oc = OracleColors.from_scene(sc)
+    dag = HashDAG(g, pool_pages=POOL_PAGES)
+    dag.load_scene(sc)
+    graph = FrameGraph(dag, None, max_edits)
+    replays = 0
+    for k, n in enumerate((max_edits, 3, max_edits - 1)):
+        edits = random_edits(p, n, seed=300 + k, rmax=5)
+        st, ran = graph.launch(edits)
+        replays += ran
+        dag.undo()
+        st, ran = graph.launch(edits)  # now over nodes that are there
+        replays += ran
+        assert st.num_voxels == sum(od.edit(kind, c, r, oc)[1] for kind, c, r in edits)
+        assert_same(dag, sc, od, oc, f"list {k}")
+    assert replays >= 4
+    graph.close()
+    dag.close()
