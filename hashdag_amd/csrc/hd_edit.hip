@@ -1426,7 +1426,9 @@ __global__ __launch_bounds__(256) void k_add(EditPass P, uint32_t l) {
 // then the whole wavefront finds or adds the representatives among them one after another. One
 // launch where dedup, find and add need three (a launch costs a small level more than its work:
 // 2-5 us of each were the time of a level of a few items); on levels of many items the runs
-// would queue behind each other, so those keep the three.
+// would queue behind each other, so those keep the three. A pass in one launch, over one workgroup
+// or all, takes it on every level: a step more there is a barrier (cooperative passes of 2048
+// editors: 11.9 ms with undo in separate steps, 7.5 ms so).
 __device__ __forceinline__ void d_nodes(const EditPass& P, uint32_t l, VGrid G) {
     const uint32_t n = min(P.count[l], P.cap[l]);
     if (*P.errors) return;
@@ -3180,8 +3182,8 @@ __global__ __launch_bounds__(kTopBlock) void k_top_expand(EditPass P, uint32_t f
 // Build and nodes of levels first .. 0, each of at most kTopNodes items, in one workgroup: eight
 // lanes build an item's node from its children's results, which stay in LDS, and a wavefront
 // enters it into the table. The child slots of all these levels are loaded at once at the start.
-// More items on one of the levels than that (the host's bound is of the editors' boxes, rounded):
-// all levels run over the item arrays.
+// More items on one of the levels than that (spheres can touch more nodes than their boxes overlap,
+// level_bounds): all levels run over the item arrays.
 constexpr uint32_t kTopSlots = kTopNodes * 8;
 struct TopSlots {
     uint32_t cval[kTopSlots], corig[kTopSlots], cnew[kTopSlots];
@@ -3387,9 +3389,12 @@ static void fill_pass(hd_ctx* ctx, EditPass& P, const EditScratch& S) {
 // Enqueues one pass over edits [first, first + n) of the uploaded edit array.
 // dN (optional): the edit count is read from device memory (at most n), for graph replays.
 // scratch (optional): the scratch the pass runs in (default: the context's own).
-// Upper bound of the work items of each level a pass over these editors creates: an item is a
-// node some editor's box overlaps, so per editor and level the nodes of that level its box
-// overlaps, capped by the level's node count and item capacity.
+// Work items of each level a pass over these editors creates, as a rule at most: an item is a node
+// some editor touches, so per editor and level the nodes of that level its box overlaps, capped by
+// the level's item capacity. A sphere can touch more: where its radius is a step of FP32 past the
+// distance to a node's upper edge, centre - radius rounds onto the edge. What is chosen by these
+// numbers takes more items than they say (grids stride, k_top_expand and k_top_nodes go on over the
+// item arrays, an undo frame that outgrows its room goes to the host).
 static void level_bounds(const EditPass& P, const DevEdit* e, uint32_t n, uint64_t out[kMaxEditLevels]) {
     const uint32_t D = P.levels, L = D - 2;
     const double world = (double)(1ull << D);
@@ -3415,7 +3420,17 @@ static void level_bounds(const EditPass& P, const DevEdit* e, uint32_t n, uint64
 }
 
 constexpr uint32_t kWideEdits = 8, kWideEditsBlock = 64, kWideItems = 512;
-constexpr uint32_t kTopItems = 128, kNodesItems = 1u << 12, kNodesEdits = 256;
+// Levels by boxes that k_top_expand takes: half of what its LDS holds, as spheres can touch more
+// nodes. Passes of 1 to 64 editors at 32, 128, 256: 0 to 4 % slower, -, 0 to 4 % faster, within the
+// 3 % that two runs of one build differ by.
+constexpr uint32_t kTopItems = 128;
+// Nodes of a level in one launch (a wavefront per item) or three. By items: the same passes at 1024
+// and 16384 in place of 4096: within 3 %, and 0 to 3 % slower; 700,000 leaves in one launch took 85
+// ms, in three 47 ms. A captured pass does not know its items, and goes by its editors: replays of
+// 128 took 1.06 ms with one launch a level and 1.13 ms with three, of 256 2.41 and 2.20 ms.
+constexpr uint32_t kNodesItems = 1u << 12, kNodesEdits = 256;
+// Items up to which a colour copy's slots are cut into pieces: within 3 % at 1024, and at 16384 up
+// to 7 % slower (64 editors of radius 2-100: 743 against 786 us).
 constexpr uint32_t kPieceItems = 4096;
 
 hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hipStream_t s, PassReadback* rb,
