@@ -179,6 +179,7 @@ _SIGS = {
     "hd_undo": (C.c_int32, [C.c_void_p]),
     "hd_redo": (C.c_int32, [C.c_void_p]),
     "hd_undo_clear": (C.c_int32, [C.c_void_p]),
+    "hd_undo_to_host": (C.c_int32, [C.c_void_p]),
     "hd_undo_depth": (C.c_int32, [C.c_void_p, u32p, u32p]),
     "hd_reserve_edit_scratch": (C.c_int32, [C.c_void_p, C.c_uint32, C.c_uint32, C.c_uint64]),
     "hd_default_config": (None, [C.c_uint32, C.POINTER(hd_config)]),

@@ -76,7 +76,7 @@ static hd_status upload_image_impl(hd_ctx* ctx, const uint32_t* pool, const uint
     if (pool_top > ctx->cfg.pool_pages) return fail(ctx, HD_ERR_POOL_FULL, "image uses more pages than the pool budget");
     const uint64_t physWords = (uint64_t)pool_top * g.page_size;
     uint32_t* dphys = nullptr;
-    HD_HIP(ctx, hipMalloc(&dphys, std::max<uint64_t>(physWords, 1) * 4));
+    HD_HIP(ctx, dev_malloc(ctx, &dphys, std::max<uint64_t>(physWords, 1) * 4));
     hipError_t e = hipMemcpyAsync(dphys, pool, physWords * 4, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess)
         e = hipMemcpyAsync(ctx->page_table, page_table, g.total_pages() * 4, hipMemcpyHostToDevice, ctx->stream);
@@ -271,7 +271,7 @@ hd_status download_pool(hd_ctx* ctx, uint32_t* pool, uint64_t cap_words) {
         HD_HIP(ctx, hipStreamSynchronize(ctx->stream));
         const uint64_t words = (uint64_t)std::max<uint32_t>(top, 1) * g.page_size;
         uint32_t* dphys = nullptr;
-        HD_HIP(ctx, hipMalloc(&dphys, words * 4));
+        HD_HIP(ctx, dev_malloc(ctx, &dphys, words * 4));
         hipError_t e = hipMemsetAsync(dphys, 0, words * 4, ctx->stream);
         if (e == hipSuccess) {
             k_gather_pages<<<grid_for(g.total_pages()), 256, 0, ctx->stream>>>(dphys, ctx->vpool, ctx->page_table,
@@ -333,10 +333,10 @@ hd_status hd_load_colors(hd_ctx* ctx, const uint32_t* nodes, uint64_t n_nodes, c
     ctx->cleaves = nullptr;
     ctx->arena = nullptr;
     ctx->colors_loaded = false;
-    HD_HIP(ctx, hipMalloc(&ctx->cnodes, nodesCap * 4));
-    HD_HIP(ctx, hipMalloc(&ctx->coffsets, std::max<uint64_t>(n_offsets, 1) * 8));
-    HD_HIP(ctx, hipMalloc(&ctx->cleaves, leavesCap * sizeof(LeafDesc)));
-    HD_HIP(ctx, hipMalloc(&ctx->arena, arenaWords * 8));
+    HD_HIP(ctx, dev_malloc(ctx, &ctx->cnodes, nodesCap * 4));
+    HD_HIP(ctx, dev_malloc(ctx, &ctx->coffsets, std::max<uint64_t>(n_offsets, 1) * 8));
+    HD_HIP(ctx, dev_malloc(ctx, &ctx->cleaves, leavesCap * sizeof(LeafDesc)));
+    HD_HIP(ctx, dev_malloc(ctx, &ctx->arena, arenaWords * 8));
     ctx->cfg.color_arena_words = arenaWords;
     ctx->cfg.color_nodes_cap = (uint32_t)nodesCap;
     ctx->cfg.color_leaves_cap = (uint32_t)leavesCap;

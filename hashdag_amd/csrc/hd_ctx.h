@@ -38,7 +38,8 @@ struct TraceScratch {
 // Device memory for the undo history's leaf records: slabs filled from the front, each kept while
 // a frame lives in it, then held for reuse (at most kSpare of them) or freed. A pass of 4096
 // editors re-points 700,000 leaves: as host vectors its frame was 90 MB copied through pageable
-// memory, and half of that back on undo. Beyond kBytes of slabs frames go to the host.
+// memory, and half of that back on undo. Beyond kBytes of slabs frames go to the host, and so do all
+// of them (undo_to_host) when an allocation of the context fails.
 struct UndoSlab {
     UndoRecord* mem = nullptr;
     uint64_t cap = 0, used = 0;
@@ -72,6 +73,12 @@ public:
         sl->cap = want;
         bytes_ += bytes;
         return cur_ = own(sl);
+    }
+    // Gives back the slabs no frame lives in; keep: but for the present one if it is of the smallest
+    // size, for a caller that clears its history after every pass.
+    void trim(bool keep) {
+        if (cur_ && cur_.use_count() == 1 && !(keep && cur_->cap == kMinRecords)) cur_.reset();
+        drop_spares();
     }
     ~UndoPool() {
         cur_.reset();
@@ -209,6 +216,14 @@ inline uint64_t leaf_tag_bytes(const Geom& g) {
     return (uint64_t)g.buckets_per_level(g.leaf_level()) * (g.bucket_size(g.leaf_level()) / 2);
 }
 hd_status fail(hd_ctx* ctx, hd_status code, const std::string& msg);
+// moves the undo history's records to host memory and gives their device memory back
+hd_status undo_to_host(hd_ctx* ctx);
+// device memory for the context: when there is none left, the undo history makes room
+hipError_t dev_malloc_bytes(hd_ctx* ctx, void** p, uint64_t bytes);
+template <class T>
+hipError_t dev_malloc(hd_ctx* ctx, T** p, uint64_t bytes) {
+    return dev_malloc_bytes(ctx, reinterpret_cast<void**>(p), bytes);
+}
 hd_status hip_fail(hd_ctx* ctx, hipError_t e, const char* what);
 DevDag dev_dag(const hd_ctx* ctx);
 DevColors dev_colors(const hd_ctx* ctx);

@@ -1427,8 +1427,7 @@ __global__ __launch_bounds__(256) void k_add(EditPass P, uint32_t l) {
 // launch where dedup, find and add need three (a launch costs a small level more than its work:
 // 2-5 us of each were the time of a level of a few items); on levels of many items the runs
 // would queue behind each other, so those keep the three. A pass in one launch, over one workgroup
-// or all, takes it on every level: a step more there is a barrier (cooperative passes of 2048
-// editors: 11.9 ms with undo in separate steps, 7.5 ms so).
+// or all, takes it on every level: a step more there is a barrier.
 __device__ __forceinline__ void d_nodes(const EditPass& P, uint32_t l, VGrid G) {
     const uint32_t n = min(P.count[l], P.cap[l]);
     if (*P.errors) return;
@@ -2707,10 +2706,10 @@ uint64_t carve_level(Items& I, uint32_t*& elist, bool leafLevel, uint64_t c, uin
 }
 
 // One allocation per level holding its item arrays and edit list.
-static hipError_t alloc_level(EditScratch& S, uint32_t l, bool leafLevel, uint64_t c, uint64_t e) {
+static hipError_t alloc_level(hd_ctx* ctx, EditScratch& S, uint32_t l, bool leafLevel, uint64_t c, uint64_t e) {
     const uint64_t total = carve_level(S.items[l], S.elist[l], leafLevel, c, e, nullptr);
     char* mem = nullptr;
-    const hipError_t err = hipMalloc(&mem, total);
+    const hipError_t err = dev_malloc(ctx, &mem, total);
     if (err != hipSuccess) return err;
     S.level_mem[l] = mem;
     carve_level(S.items[l], S.elist[l], leafLevel, c, e, mem);
@@ -2730,7 +2729,7 @@ hd_status edit_reserve(hd_ctx* ctx, const uint32_t* items, const uint32_t* elist
         scratch_free(ctx);
         S.levels = levels;
         auto alloc = [&](void** p, uint64_t bytes) -> bool {
-            if (hipMalloc(p, std::max<uint64_t>(bytes, 16)) != hipSuccess) return false;
+            if (dev_malloc(ctx, p, std::max<uint64_t>(bytes, 16)) != hipSuccess) return false;
             S.allocs.push_back(*p);
             return true;
         };
@@ -2758,7 +2757,7 @@ hd_status edit_reserve(hd_ctx* ctx, const uint32_t* items, const uint32_t* elist
         hipFree(S.level_mem[l]);
         S.level_mem[l] = nullptr;
         S.item_cap[l] = S.elist_cap[l] = 0;
-        const hipError_t err = alloc_level(S, l, l == L, c, e);
+        const hipError_t err = alloc_level(ctx, S, l, l == L, c, e);
         if (err != hipSuccess) return hip_fail(ctx, err, "edit scratch (items)");
     }
     uint32_t hcap = 1;
@@ -2768,7 +2767,7 @@ hd_status edit_reserve(hd_ctx* ctx, const uint32_t* items, const uint32_t* elist
         hipFree(S.hset);
         S.hset = nullptr;
         S.hcap = 0;
-        const hipError_t err = hipMalloc(&S.hset, (uint64_t)hcap * 4);
+        const hipError_t err = dev_malloc(ctx, &S.hset, (uint64_t)hcap * 4);
         if (err != hipSuccess) return hip_fail(ctx, err, "edit scratch (hash set)");
         S.hcap = hcap;
     }
@@ -2780,8 +2779,8 @@ hd_status edit_reserve(hd_ctx* ctx, const uint32_t* items, const uint32_t* elist
         S.cmarks = nullptr;
         S.color_cap = 0;
         colors = (colors + 63) & ~63ull;  // whole chunks, one marker each
-        hipError_t err = hipMalloc(&S.colors, colors * 8);
-        if (err == hipSuccess) err = hipMalloc(&S.cmarks, colors / 64 * 8);
+        hipError_t err = dev_malloc(ctx, &S.colors, colors * 8);
+        if (err == hipSuccess) err = dev_malloc(ctx, &S.cmarks, colors / 64 * 8);
         if (err != hipSuccess) return hip_fail(ctx, err, "edit scratch (colours)");
         S.color_cap = colors;
     }
@@ -2794,8 +2793,8 @@ hd_status edit_reserve(hd_ctx* ctx, const uint32_t* items, const uint32_t* elist
         S.seg_task = nullptr;
         S.seg_out = nullptr;
         S.seg_cap = 0;
-        hipError_t err = segs > 0xFFFFFFFFull ? hipErrorOutOfMemory : hipMalloc(&S.seg_task, segs * 4);
-        if (err == hipSuccess) err = hipMalloc(&S.seg_out, segs * 8);
+        hipError_t err = segs > 0xFFFFFFFFull ? hipErrorOutOfMemory : dev_malloc(ctx, &S.seg_task, segs * 4);
+        if (err == hipSuccess) err = dev_malloc(ctx, &S.seg_out, segs * 8);
         if (err != hipSuccess) return hip_fail(ctx, err, "edit scratch (segments)");
         S.seg_cap = (uint32_t)segs;
     }
@@ -2815,9 +2814,9 @@ hd_status edit_reserve_undo(hd_ctx* ctx, uint64_t entries) {
     S.undo_handles = nullptr;
     S.undo_descs = S.undo_next = nullptr;
     S.undo_cap = 0;
-    hipError_t e = hipMalloc(&S.undo_handles, (uint64_t)cap * 4);
-    if (e == hipSuccess) e = hipMalloc(&S.undo_descs, (uint64_t)cap * sizeof(LeafDesc));
-    if (e == hipSuccess) e = hipMalloc(&S.undo_next, (uint64_t)cap * sizeof(LeafDesc));
+    hipError_t e = dev_malloc(ctx, &S.undo_handles, (uint64_t)cap * 4);
+    if (e == hipSuccess) e = dev_malloc(ctx, &S.undo_descs, (uint64_t)cap * sizeof(LeafDesc));
+    if (e == hipSuccess) e = dev_malloc(ctx, &S.undo_next, (uint64_t)cap * sizeof(LeafDesc));
     if (e != hipSuccess) return hip_fail(ctx, e, "undo log");
     S.undo_cap = cap;
     return HD_OK;
@@ -2829,7 +2828,7 @@ hd_status edit_ensure_edits(hd_ctx* ctx, uint32_t n) {
     if (n <= S.edits_cap) return HD_OK;
     const uint32_t cap = std::max<uint32_t>(n, 4096);
     DevEdit* ne = nullptr;
-    const hipError_t e = hipMalloc(&ne, (uint64_t)cap * sizeof(DevEdit));
+    const hipError_t e = dev_malloc(ctx, &ne, (uint64_t)cap * sizeof(DevEdit));
     if (e != hipSuccess) return hip_fail(ctx, e, "edit array");
     if (S.edits_dev) {
         hipDeviceSynchronize();
@@ -3425,8 +3424,8 @@ constexpr uint32_t kWideEdits = 8, kWideEditsBlock = 64, kWideItems = 512;
 // 3 % that two runs of one build differ by.
 constexpr uint32_t kTopItems = 128;
 // Nodes of a level in one launch (a wavefront per item) or three. By items: the same passes at 1024
-// and 16384 in place of 4096: within 3 %, and 0 to 3 % slower; 700,000 leaves in one launch took 85
-// ms, in three 47 ms. A captured pass does not know its items, and goes by its editors: replays of
+// and 16384 in place of 4096: within 3 %, and 0 to 3 % slower; a first pass of 4096 editors (17 M
+// words to add) took 85 ms with one launch a level and 47 ms with three. A captured pass does not know its items, and goes by its editors: replays of
 // 128 took 1.06 ms with one launch a level and 1.13 ms with three, of 256 2.41 and 2.20 ms.
 constexpr uint32_t kNodesItems = 1u << 12, kNodesEdits = 256;
 // Items up to which a colour copy's slots are cut into pieces: within 3 % at 1024, and at 16384 up
@@ -3619,7 +3618,7 @@ hd_status fill_prepare(hd_ctx* ctx, const hd_edit& e, DevEdit& d, FillBuffers& f
     std::vector<uint8_t> solid(n);
     {
         uint8_t* dsolid = nullptr;
-        HD_HIP(ctx, hipMalloc(&dsolid, n));
+        HD_HIP(ctx, dev_malloc(ctx, &dsolid, n));
         k_fill_load<<<(uint32_t)std::min<uint64_t>((n + 255) / 256, 65536), 256, 0, s>>>(
             ctx->vpool, ctx->d_root, ctx->g.levels, fmin[0], fmin[1], fmin[2], S, dsolid);
         hipError_t err = hipGetLastError();
@@ -3677,8 +3676,8 @@ hd_status fill_prepare(hd_ctx* ctx, const hd_edit& e, DevEdit& d, FillBuffers& f
     if (nl && ctx->colors_loaded) {
         uint32_t* dxyz = nullptr;
         uint64_t* dcol = nullptr;
-        hipError_t err = hipMalloc(&dxyz, loaded.size() * 4);
-        if (err == hipSuccess) err = hipMalloc(&dcol, (uint64_t)nl * 8);
+        hipError_t err = dev_malloc(ctx, &dxyz, loaded.size() * 4);
+        if (err == hipSuccess) err = dev_malloc(ctx, &dcol, (uint64_t)nl * 8);
         if (err == hipSuccess) err = hipMemcpyAsync(dxyz, loaded.data(), loaded.size() * 4, hipMemcpyHostToDevice, s);
         if (err == hipSuccess) {
             EditPass P{};
@@ -3711,8 +3710,8 @@ hd_status fill_prepare(hd_ctx* ctx, const hd_edit& e, DevEdit& d, FillBuffers& f
     std::vector<uint8_t> state(n);
     for (uint64_t i = 0; i < n; ++i) state[i] = (uint8_t)((st[i] == SetTrue ? 3u : 0u) | (solid[i] ? 1u : 0u));
     fb.release();
-    HD_HIP(ctx, hipMalloc(&fb.state, n));
-    HD_HIP(ctx, hipMalloc(&fb.colors, nb * 8));
+    HD_HIP(ctx, dev_malloc(ctx, &fb.state, n));
+    HD_HIP(ctx, dev_malloc(ctx, &fb.colors, nb * 8));
     HD_HIP(ctx, hipMemcpyAsync(fb.state, state.data(), n, hipMemcpyHostToDevice, s));
     HD_HIP(ctx, hipMemcpyAsync(fb.colors, colors.data(), nb * 8, hipMemcpyHostToDevice, s));
     HD_HIP(ctx, hipStreamSynchronize(s));
@@ -3763,8 +3762,8 @@ hd_status noise_prepare(hd_ctx* ctx, const hd_edit& e, DevEdit& d, FillBuffers& 
     }
     const float bounding = 1.0f / ampFractal;
     fb.release();
-    HD_HIP(ctx, hipMalloc(&fb.state, n));
-    HD_HIP(ctx, hipMalloc(&fb.tables, sizeof(tab)));
+    HD_HIP(ctx, dev_malloc(ctx, &fb.state, n));
+    HD_HIP(ctx, dev_malloc(ctx, &fb.tables, sizeof(tab)));
     HD_HIP(ctx, hipMemcpyAsync(fb.tables, tab, sizeof(tab), hipMemcpyHostToDevice, s));
     k_noise_state<<<(uint32_t)std::min<uint64_t>((n + 255) / 256, 65536), 256, 0, s>>>(
         ctx->vpool, ctx->d_root, ctx->g.levels, fmin[0], fmin[1], fmin[2], S, r, 1 / r, bounding, fb.tables,

@@ -220,7 +220,7 @@ static hd_status grow_arena(hd_ctx* ctx, uint64_t need) {
     if (ctx->arena_top + need <= cap) return HD_OK;
     const uint64_t ncap = std::max<uint64_t>(cap * 2, ctx->arena_top + need + (1u << 24));
     uint64_t* na = nullptr;
-    HD_HIP(ctx, hipMalloc(&na, ncap * 8));
+    HD_HIP(ctx, dev_malloc(ctx, &na, ncap * 8));
     HD_HIP(ctx, hipMemsetAsync(na, 0, ncap * 8, ctx->stream));
     HD_HIP(ctx, hipMemcpyAsync(na, ctx->arena, ctx->arena_top * 8, hipMemcpyDeviceToDevice, ctx->stream));
     HD_HIP(ctx, hipStreamSynchronize(ctx->stream));
@@ -240,7 +240,7 @@ static hd_status grow_color_tables(hd_ctx* ctx, uint64_t nodes, uint64_t leaves)
         const uint64_t cap = std::min<uint64_t>(std::max<uint64_t>(nodes + nodes / 2, 2ull * ctx->cfg.color_nodes_cap), 0xFFFFFFF0u);
         if (cap < nodes) return fail(ctx, HD_ERR_COLOR_FULL, "colour tree exceeds 2^32 entries");
         uint32_t* nn = nullptr;
-        HD_HIP(ctx, hipMalloc(&nn, cap * 4));
+        HD_HIP(ctx, dev_malloc(ctx, &nn, cap * 4));
         HD_HIP(ctx, hipMemset(nn, 0, cap * 4));
         HD_HIP(ctx, hipMemcpy(nn, ctx->cnodes, (uint64_t)ctx->cfg.color_nodes_cap * 4, hipMemcpyDeviceToDevice));
         hipFree(ctx->cnodes);
@@ -251,7 +251,7 @@ static hd_status grow_color_tables(hd_ctx* ctx, uint64_t nodes, uint64_t leaves)
         const uint64_t cap = std::min<uint64_t>(std::max<uint64_t>(leaves + leaves / 2, 2ull * ctx->cfg.color_leaves_cap), 0x7FFFFFFFu);
         if (cap < leaves) return fail(ctx, HD_ERR_COLOR_FULL, "more than 2^31 colour leaves");
         LeafDesc* nl = nullptr;
-        HD_HIP(ctx, hipMalloc(&nl, cap * sizeof(LeafDesc)));
+        HD_HIP(ctx, dev_malloc(ctx, &nl, cap * sizeof(LeafDesc)));
         HD_HIP(ctx, hipMemcpy(nl, ctx->cleaves, (uint64_t)ctx->cfg.color_leaves_cap * sizeof(LeafDesc), hipMemcpyDeviceToDevice));
         hipFree(ctx->cleaves);
         ctx->cleaves = nl;
@@ -293,6 +293,43 @@ static hd_status frame_commit(hd_ctx* ctx, uint32_t nu, uint32_t cap, UndoFrame&
     frame.n = nu;
     if (frame.slab) frame.slab->used = frame.first + nu;
     return HD_OK;
+}
+
+hd_status undo_to_host(hd_ctx* ctx) {
+    try {
+        std::vector<UndoRecord> rec;
+        for (auto* frames : {&ctx->undo, &ctx->redo})
+            for (UndoFrame& f : *frames) {
+                if (!f.slab) continue;
+                rec.resize(f.n);
+                if (f.n)
+                    HD_HIP(ctx, hipMemcpy(rec.data(), f.slab->mem + f.first, (uint64_t)f.n * sizeof(UndoRecord),
+                                          hipMemcpyDeviceToHost));
+                f.handles.resize(f.n);
+                f.prev.resize(f.n);
+                f.next.resize(f.n);
+                for (uint32_t k = 0; k < f.n; ++k) {
+                    f.handles[k] = rec[k].handle;
+                    f.prev[k] = rec[k].prev;
+                    f.next[k] = rec[k].next;
+                }
+                f.slab.reset();
+            }
+    } catch (const std::bad_alloc&) {
+        return fail(ctx, HD_ERR_OOM, "undo history: out of host memory");
+    }
+    ctx->undo_pool.trim(false);
+    return HD_OK;
+}
+
+hipError_t dev_malloc_bytes(hd_ctx* ctx, void** p, uint64_t bytes) {
+    hipError_t e = hipMalloc(p, bytes);
+    if (e != hipErrorOutOfMemory) return e;
+    (void)hipGetLastError();
+    if (undo_to_host(ctx) != HD_OK) return e;
+    e = hipMalloc(p, bytes);
+    if (e != hipSuccess) (void)hipGetLastError();
+    return e;
 }
 
 // Colour tree, default scratch and undo log of a context's first edit.
@@ -575,7 +612,13 @@ hd_status hd_undo_clear(hd_ctx* ctx) {
     if (!ctx) return fail(ctx, HD_ERR_INVALID, "null context");
     ctx->undo.clear();
     ctx->redo.clear();
+    ctx->undo_pool.trim(true);
     return HD_OK;
+}
+
+hd_status hd_undo_to_host(hd_ctx* ctx) {
+    if (!ctx) return fail(ctx, HD_ERR_INVALID, "null context");
+    return undo_to_host(ctx);
 }
 
 hd_status hd_undo_depth(hd_ctx* ctx, uint32_t* undo, uint32_t* redo) {
@@ -903,8 +946,8 @@ hd_status hd_frame_graph_create(hd_ctx* ctx, uint32_t max_edits, uint32_t width,
     if (e == hipSuccess) e = hipHostMalloc(&g->h_n, 4);
     if (e == hipSuccess) e = hipHostMalloc(&g->h_params, sizeof(hd_ray_params));
     if (e == hipSuccess) e = hipHostMalloc(&g->h_rb, sizeof(PassReadback));
-    if (e == hipSuccess) e = hipMalloc(&g->d_n, 4);
-    if (e == hipSuccess) e = hipMalloc(&g->d_params, sizeof(hd_ray_params));
+    if (e == hipSuccess) e = dev_malloc(ctx, &g->d_n, 4);
+    if (e == hipSuccess) e = dev_malloc(ctx, &g->d_params, sizeof(hd_ray_params));
     if (e != hipSuccess) {
         hd_frame_graph_destroy(g);
         return hip_fail(ctx, e, "frame graph buffers");

@@ -353,10 +353,10 @@ hd_status hd_checkpoint_load(hd_ctx* ctx, const char* path) {
     ctx->cleaves = nullptr;
     ctx->arena = nullptr;
     ctx->colors_loaded = false;
-    HD_HIP(ctx, hipMalloc(&ctx->cnodes, nodesCap * 4));
-    HD_HIP(ctx, hipMalloc(&ctx->coffsets, std::max<uint64_t>(offsets.size(), 1) * 8));
-    HD_HIP(ctx, hipMalloc(&ctx->cleaves, leavesCap * sizeof(LeafDesc)));
-    HD_HIP(ctx, hipMalloc(&ctx->arena, arenaWords * 8));
+    HD_HIP(ctx, dev_malloc(ctx, &ctx->cnodes, nodesCap * 4));
+    HD_HIP(ctx, dev_malloc(ctx, &ctx->coffsets, std::max<uint64_t>(offsets.size(), 1) * 8));
+    HD_HIP(ctx, dev_malloc(ctx, &ctx->cleaves, leavesCap * sizeof(LeafDesc)));
+    HD_HIP(ctx, dev_malloc(ctx, &ctx->arena, arenaWords * 8));
     ctx->cfg.color_nodes_cap = (uint32_t)nodesCap;
     ctx->cfg.color_leaves_cap = (uint32_t)leavesCap;
     ctx->cfg.color_arena_words = arenaWords;

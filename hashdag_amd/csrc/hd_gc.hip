@@ -388,7 +388,7 @@ static hipError_t gc_slot(hd_ctx* ctx, uint32_t k, uint64_t bytes, void** p) {
         }
         const uint64_t want = std::max<uint64_t>(bytes + bytes / 4, 256);
         void* q = nullptr;
-        const hipError_t e = hipMalloc(&q, want);
+        const hipError_t e = dev_malloc(ctx, &q, want);
         if (e != hipSuccess) return e;
         sl = {q, want};
     }

@@ -189,9 +189,9 @@ hd_status hd_serve_run(hd_ctx* ctx, const hd_request* reqs, uint32_t n, const hd
     for (Slot& s : slots) {
         if (e == hipSuccess) e = hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking);
         if (e == hipSuccess) e = hipEventCreateWithFlags(&s.done, hipEventDisableTiming);
-        if (e == hipSuccess) e = hipMalloc(&s.paths, maxPixels * 16);
-        if (e == hipSuccess) e = hipMalloc(&s.colors, maxPixels * 4);
-        if (e == hipSuccess) e = hipMalloc(&s.sum, 8);
+        if (e == hipSuccess) e = dev_malloc(ctx, &s.paths, maxPixels * 16);
+        if (e == hipSuccess) e = dev_malloc(ctx, &s.colors, maxPixels * 4);
+        if (e == hipSuccess) e = dev_malloc(ctx, &s.sum, 8);
         if (e == hipSuccess) e = hipHostMalloc(&s.hsum, 8);
     }
     if (e != hipSuccess) {
@@ -320,7 +320,10 @@ hd_status hd_serve_run(hd_ctx* ctx, const hd_request* reqs, uint32_t n, const hd
                 if (gcSt == HD_OK) st = hd_edit_batch(ctx, fused.data(), (uint32_t)fused.size(), 1, &es, editStream);
                 else st = gcSt;
             }
-            if (st == HD_OK && !cfg->keep_undo) hd_undo_clear(ctx);
+            if (st == HD_OK && !cfg->keep_undo) {  // its memory serves the next batch's frame
+                ctx->undo.clear();
+                ctx->redo.clear();
+            }
             const double done = now_s();
             for (uint32_t m : members) {
                 out[m].done_s = done;
@@ -377,6 +380,7 @@ hd_status hd_serve_run(hd_ctx* ctx, const hd_request* reqs, uint32_t n, const hd
     // drain
     while (finished < n && result == HD_OK) poll_slots(true);
     cleanup();
+    if (!cfg->keep_undo) ctx->undo_pool.trim(true);
     return result;
 }
 

@@ -1609,8 +1609,8 @@ hd_status trace_reserve(hd_ctx* ctx, hipStream_t s, uint32_t W, uint32_t H, Trac
         ctx->trace_scratch.push_back(TraceScratch{});
         ts = &ctx->trace_scratch.back();
         ts->stream = s;
-        HD_HIP(ctx, hipMalloc(&ts->queues, 64 * 32 * 4));
-        HD_HIP(ctx, hipMalloc(&ts->long_count, 64));
+        HD_HIP(ctx, dev_malloc(ctx, &ts->queues, 64 * 32 * 4));
+        HD_HIP(ctx, dev_malloc(ctx, &ts->long_count, 64));
     } else {
         HD_HIP(ctx, hipStreamSynchronize(s));
         hipFree(ts->rec);
@@ -1626,15 +1626,15 @@ hd_status trace_reserve(hd_ctx* ctx, hipStream_t s, uint32_t W, uint32_t H, Trac
         ts->long_items = ts->rest_items = ts->resume_items = ts->resume_state = nullptr;
         ts->tiles_cap = ts->pixels_cap = 0;
     }
-    HD_HIP(ctx, hipMalloc(&ts->rec, tiles * 64 * sizeof(uint4)));
-    HD_HIP(ctx, hipMalloc(&ts->shades, tiles * 64 * sizeof(uint2)));
-    HD_HIP(ctx, hipMalloc(&ts->cnt, tiles * sizeof(uint32_t)));
-    HD_HIP(ctx, hipMalloc(&ts->long_items, pixels * sizeof(uint32_t)));
-    HD_HIP(ctx, hipMalloc(&ts->rest_items, pixels * sizeof(uint32_t)));
+    HD_HIP(ctx, dev_malloc(ctx, &ts->rec, tiles * 64 * sizeof(uint4)));
+    HD_HIP(ctx, dev_malloc(ctx, &ts->shades, tiles * 64 * sizeof(uint2)));
+    HD_HIP(ctx, dev_malloc(ctx, &ts->cnt, tiles * sizeof(uint32_t)));
+    HD_HIP(ctx, dev_malloc(ctx, &ts->long_items, pixels * sizeof(uint32_t)));
+    HD_HIP(ctx, dev_malloc(ctx, &ts->rest_items, pixels * sizeof(uint32_t)));
     if (resume) {
         if (pixels * kStateWords >= (1ull << 32)) return fail(ctx, HD_ERR_INVALID, "frame too large for resumed walks");
-        HD_HIP(ctx, hipMalloc(&ts->resume_items, pixels * sizeof(uint32_t)));
-        HD_HIP(ctx, hipMalloc(&ts->resume_state, pixels * kStateWords * sizeof(uint32_t)));
+        HD_HIP(ctx, dev_malloc(ctx, &ts->resume_items, pixels * sizeof(uint32_t)));
+        HD_HIP(ctx, dev_malloc(ctx, &ts->resume_state, pixels * kStateWords * sizeof(uint32_t)));
     }
     ts->tiles_cap = tiles;
     ts->pixels_cap = pixels;

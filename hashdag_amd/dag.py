@@ -369,6 +369,10 @@ class HashDAG:
     def clear_undo(self) -> None:
         check(lib.hd_undo_clear(self._h), self._h)
 
+    def undo_to_host(self) -> None:
+        """Moves the undo history out of device memory (hd_undo_to_host)."""
+        check(lib.hd_undo_to_host(self._h), self._h)
+
     def undo_depth(self):
         u, r = C.c_uint32(), C.c_uint32()
         check(lib.hd_undo_depth(self._h, C.byref(u), C.byref(r)), self._h)

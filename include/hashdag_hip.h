@@ -273,10 +273,16 @@ hd_status hd_autotune_edit_launch(hd_ctx* ctx, const hd_edit* sample, uint32_t n
  * every colour of an explicit chunk (8 B each), written once and read twice by the encoder,
  * out[4] colour leaf words written. Old colours decoded are not counted. */
 hd_status hd_edit_count_bytes(hd_ctx* ctx, uint32_t on, uint64_t out[5]);
-/* HashDAGUndoRedo::undo / redo (hash_dag.h:68-120) and free (133-145). */
+/* HashDAGUndoRedo::undo / redo (hash_dag.h:68-120) and free (133-145). The history's colour-leaf
+ * records stay in device memory (136 B a leaf a pass re-pointed, at most 4 GiB a context, then in
+ * host memory). hd_undo_clear gives it back (but for 9 MB that the next passes use), and an
+ * allocation of the context that finds no device memory moves the history to the host first. */
 hd_status hd_undo(hd_ctx* ctx);
 hd_status hd_redo(hd_ctx* ctx);
 hd_status hd_undo_clear(hd_ctx* ctx);
+/* Moves the history's records to host memory and gives their device memory back; undo and redo work
+ * as before. No counterpart in the reference, whose history lives on the host (hash_dag.h:29-45). */
+hd_status hd_undo_to_host(hd_ctx* ctx);
 hd_status hd_undo_depth(hd_ctx* ctx, uint32_t* undo, uint32_t* redo);
 /* Pre-sizes the edit work-item scratch (items per level, edit-list words per level,
  * colours per pass); grown automatically when a pass overflows. Not in the reference. */
