@@ -106,8 +106,6 @@ struct Items {
     uint32_t *px, *py, *pz;   // path of the item's node
     uint32_t* old_;           // effective old node (may be a full node after a full cover)
     uint32_t* orig;           // the node the parent actually points to
-    uint32_t* parent;
-    uint8_t* slot;
     uint32_t *estart, *ecount;  // edit sub-list in elist[level]
     uint32_t* aux;              // levels < ctl: colour node; levels >= ctl: task (level-ctl item)
     uint32_t* handle;           // tasks: colour leaf handle before the pass

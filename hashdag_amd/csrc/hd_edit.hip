@@ -611,17 +611,15 @@ struct ParentRefs {
 // child item ci of a slot, all but its edit list (rest words from eo); its old node, colour mode
 // and aux come back for a caller that goes on with it
 __device__ __forceinline__ void slot_child_item(const EditPass& P, const Items& I, const Items& C, uint32_t l,
-                                                uint32_t i, uint32_t c, uint32_t slot, uint32_t ci, uint32_t eo,
-                                                uint32_t rest, const SlotRefs& r, uint32_t lastCover,
-                                                uint32_t coverKind, uint32_t coverColor, const ParentRefs& par,
+                                                uint32_t c, uint32_t slot, uint32_t ci, uint32_t eo, uint32_t rest,
+                                                const SlotRefs& r, uint32_t lastCover, uint32_t coverKind,
+                                                uint32_t coverColor, const ParentRefs& par,
                                                 uint32_t& childOld, ParentRefs& child) {
     const uint32_t ctl = P.ctl;
     C.px[ci] = r.cx;
     C.py[ci] = r.cy;
     C.pz[ci] = r.cz;
     C.orig[ci] = r.childOrig;
-    C.parent[ci] = i;
-    C.slot[ci] = (uint8_t)c;
     C.estart[ci] = eo;
     C.ecount[ci] = rest;
     childOld = r.childOld;
@@ -729,7 +727,7 @@ __device__ __forceinline__ void d_expand(const EditPass& P, uint32_t l, VGrid G)
             }
             uint32_t childOld;
             ParentRefs child;
-            slot_child_item(P, I, C, l, i, c, slot, ci, eo, rest, r, lastCover, coverKind, coverColor,
+            slot_child_item(P, I, C, l, c, slot, ci, eo, rest, r, lastCover, coverKind, coverColor,
                             ParentRefs{I.cmode[i], I.cmodeval[i], I.aux[i]}, childOld, child);
         }
         I.ckind[slot] = (uint8_t)kind;
@@ -829,7 +827,7 @@ __device__ __forceinline__ void d_expand_wide(const EditPass& P, uint32_t l, VGr
             if (lane == 0) {
                 uint32_t childOld;
                 ParentRefs child;
-                slot_child_item(P, I, C, l, i, c, (uint32_t)slot, ci, eo, rest, r, lastCover, coverKind, coverColor,
+                slot_child_item(P, I, C, l, c, (uint32_t)slot, ci, eo, rest, r, lastCover, coverKind, coverColor,
                                 ParentRefs{I.cmode[i], I.cmodeval[i], I.aux[i]}, childOld, child);
             }
         }
@@ -1106,10 +1104,6 @@ __global__ __launch_bounds__(256) void k_build(EditPass P, uint32_t l) {
 // ---------------------------------------------------------------------------------------------
 // dedup / find / add for the pending items of one level
 // ---------------------------------------------------------------------------------------------
-__global__ void k_fill(uint32_t* p, uint64_t n, uint32_t v) {
-    for (uint64_t i = (uint64_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (uint64_t)gridDim.x * blockDim.x) p[i] = v;
-}
-
 __device__ __forceinline__ bool same_content(const Items& I, uint32_t a, uint32_t b) {
     const uint32_t n = I.clen[a];
     if (n != I.clen[b]) return false;
@@ -1581,13 +1575,6 @@ __device__ uint64_t source_color(const EditPass& P, uint32_t root, uint32_t x, u
     const LeafDesc d = task_leaf(P, handle);
     if (!leaf_valid_index(d, nof)) return 0;
     return leaf_decode(P.arena, d, nof);
-}
-
-__device__ __forceinline__ uint64_t old_color(const EditPass& P, uint32_t mode, uint32_t modeval, const LeafDesc& d,
-                                              uint64_t index) {
-    if (mode == 1) return pack_color(modeval, 0, 0);
-    if (leaf_valid_index(d, index)) return leaf_decode(P.arena, d, index);
-    return 0;  // CompressedColor{}
 }
 
 // A chunk of 64 staged colours that all share one colour with no weights is stored as a marker
@@ -2603,8 +2590,6 @@ __global__ void k_init_pass(EditPass P, uint32_t* d_root, uint32_t root, uint32_
         I.px[0] = I.py[0] = I.pz[0] = 0;
         I.old_[0] = root;
         I.orig[0] = root;
-        I.parent[0] = 0;
-        I.slot[0] = 0;
         I.estart[0] = 0;
         I.ecount[0] = nEdits;
         I.aux[0] = 0;  // colour node of the root
@@ -2685,8 +2670,8 @@ uint64_t carve_level(Items& I, uint32_t*& elist, bool leafLevel, uint64_t c, uin
     I = Items{};
     const Field f[] = {
         {(void**)&I.px, c * 4},       {(void**)&I.py, c * 4},      {(void**)&I.pz, c * 4},
-        {(void**)&I.old_, c * 4},     {(void**)&I.orig, c * 4},    {(void**)&I.parent, c * 4},
-        {(void**)&I.slot, c},         {(void**)&I.estart, c * 4},  {(void**)&I.ecount, c * 4},
+        {(void**)&I.old_, c * 4},     {(void**)&I.orig, c * 4},
+        {(void**)&I.estart, c * 4},   {(void**)&I.ecount, c * 4},
         {(void**)&I.aux, c * 4},      {(void**)&I.handle, c * 4},  {(void**)&I.newhandle, c * 4},
         {(void**)&I.cmode, c * 4},    {(void**)&I.cmodeval, c * 4}, {(void**)&I.ckind, c8},
         {(void**)&I.cval, c8 * 4},    {(void**)&I.corig, c8 * 4},  {(void**)&I.cold, c8 * 4},
@@ -3142,7 +3127,7 @@ __global__ __launch_bounds__(kTopBlock) void k_top_expand(EditPass P, uint32_t f
                 P.elist[l + 1][eo + w++] = first + (uint32_t)__ffsll((long long)q) - 1u;
             uint32_t childOld;
             ParentRefs child;
-            slot_child_item(P, I, C, l, i, c, slot, ci, eo, nRest, r, lastCover, coverKind, coverColor,
+            slot_child_item(P, I, C, l, c, slot, ci, eo, nRest, r, lastCover, coverKind, coverColor,
                             ParentRefs{T.cmode[i], T.cmodeval[i], T.aux[i]}, childOld, child);
             if (ci < kTopCap && l + 1 < last) {
                 N.px[ci] = r.cx;
