@@ -1,7 +1,7 @@
 """The segmented colour encoder and the edited-voxel count at the sizes where they change path:
-colour arrays that end at, just before and just after a segment (4096 colours), arrays of more
-segments than a lane walks on its own (8), and editors that leave the scene or fall between
-voxels. Checked against the oracle, word by word."""
+colour arrays that end at, just before and just after a segment (4096 colours), arrays of up to and
+of more segments than a lane walks on its own (8), a wavefront's tasks of both kinds together, and
+editors that leave the scene or fall between voxels. Checked against the oracle, word by word."""
 import numpy as np
 import pytest
 
@@ -25,6 +25,40 @@ def test_segment_edges_match_oracle(r, where):
     total = sum(od.edit(kind, cc, rr, oc)[1] for kind, cc, rr in edits)
     assert st.num_voxels == total
     assert_same(dag, sc, od, oc, f"box of radius {r} in the {where}")
+
+
+@pytest.mark.parametrize("one", [None, BOX_CARVE, BOX_ADD])
+def test_one_colour_around_a_segment_matches_oracle(one):
+    """4096 colours in a subtree, and one less and one more."""
+    p, sc, g, dag, od, oc = make("d10w")
+    edits = [(BOX_ADD, (192.0, 960.0, 192.0), 8.0)]
+    if one is not None:  # the box's last voxel, or the one beside its face
+        edits.append((one, (199.5, 967.5, 199.5) if one == BOX_CARVE else (200.5, 960.5, 192.5), 0.5))
+    st = dag.edit_batch(edits, fused=True)
+    assert st.num_voxels == sum(od.edit(kind, c, r, oc)[1] for kind, c, r in edits)
+    assert st.colors_encoded == 4096 + {None: 0, BOX_CARVE: -1, BOX_ADD: 1}[one]
+    assert_same(dag, sc, od, oc, "around a segment")
+
+
+def test_tasks_of_few_and_many_segments_in_one_wavefront():
+    """40 colour subtrees in one workgroup's four wavefronts: more than 8 tasks each, so lanes walk
+    arrays of up to 8 segments on their own, beside one of 9 and one of 64 segments."""
+    p, sc, g, dag, od, oc = make("d10w")
+    dag.set_edit_launch(1 << 30)
+    sides = [2, 6, 16, 17, 25, 32] * 6 + [12, 20, 33, 64]  # voxels a side: 1 to 8 segments, 9, 64
+    assert sorted({(s ** 3 + 4095) // 4096 for s in sides})[-3:] == [8, 9, 64]
+    edits = []
+    for k, s in enumerate(sides):  # a subtree each, in the air: 128 voxels a side, 8 along x
+        half = s / 2
+        at = (128.0 * (k % 8) + 64, 448.0 + 128 * (k // 32), 128.0 * (k // 8 % 4) + 64)
+        c = tuple(v + (0.5 if s % 2 else 0.0) for v in at)
+        edits.append((BOX_ADD, c, half))
+        if k % 3 == 0:  # colours of their own in a corner
+            edits.append((SPHERE_PAINT, tuple(v + half for v in c), half))
+    st = dag.edit_batch(edits, fused=True)
+    assert st.passes == 1
+    assert st.num_voxels == sum(od.edit(kind, c, r, oc)[1] for kind, c, r in edits)
+    assert_same(dag, sc, od, oc, "few and many segments")
 
 
 @pytest.mark.parametrize("seed", range(3))
