@@ -3478,7 +3478,8 @@ hd_status enqueue_pass(hd_ctx* ctx, uint32_t first, uint32_t n, bool colors, hip
     };
     // encoder: a wavefront per segment of the staged colours. Their number is on the device (at
     // most what the tasks can hold): twice the wavefronts the chip keeps resident, then a stride
-    const uint64_t maxSegs = bound[P.ctl] * (((1ull << (3 * (D - P.ctl))) + kSegColors - 1) / kSegColors);
+    const uint64_t maxSegs =
+        colors ? bound[P.ctl] * (((1ull << (3 * (D - P.ctl))) + kSegColors - 1) / kSegColors) : 0u;
     const uint32_t segBlocks =
         (uint32_t)std::min<uint64_t>(std::max<uint64_t>((maxSegs + kEncWaves - 1) / kEncWaves, 1u), 4096u);
     for (uint32_t i = 0; i < sl.n;) {

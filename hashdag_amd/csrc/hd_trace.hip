@@ -326,12 +326,13 @@ __device__ __forceinline__ void walk_begin(const DevDag& dag, Walk& w, const Ray
 // height with children left. The walk has ended when w.s is 0: at a voxel, its path in (px, py,
 // pz), or with kNothingLeft in w.alive and (0, 0, 0).
 //
-// Bound by VALU issue (SQ_ACTIVE_INST_VALU fills the launch's SIMD cycles at 1080p) and, where few
-// wavefronts are in flight, by the latency of a step. Loads go through one straight path for
-// every lane (lanes inside a leaf read some word of their parent), so the child's pointer and
-// then its words are in flight while the child's intersection mask, which needs neither, is
-// computed; a node's own load per step, and the masks kept in the ray's order, take about 120
-// instructions a step where a load per branch and a permutation per child took about 175.
+// Bound by VALU issue (the VALU is busy for 0.83 / 0.85 of the capped paths / shadows launches at
+// 1080p) and, where few wavefronts are in flight, by the latency of a step. Loads go through one
+// straight path for every lane (lanes inside a leaf read some word of their parent), so the child's
+// pointer and then its words are in flight while the child's intersection mask, which needs neither,
+// is computed. With a node's own load per step and the masks kept in the ray's order a wavefront
+// issues 4920 / 5414 VALU instructions, where a load per branch and a permutation per child took
+// 5787 / 6169.
 // 1920x1080 over a 2^15 terrain 16384 wide, capped at 128 steps: paths 0.42 -> 0.28 ms, shadows
 // 0.59 -> 0.39 ms; 640x360 uncapped: 0.21 -> 0.08 and 0.22 -> 0.16 ms.
 template <bool kCount, int kFetch, bool kAxis0, bool kTame>
