@@ -15,8 +15,9 @@ def boxed(edits, side, world):
                for _, c, r in edits)
 
 
+@pytest.mark.parametrize("reserved", [False, True])
 @pytest.mark.parametrize("last", [SPHERE_CARVE, SPHERE_ADD, SPHERE_PAINT])
-def test_wide_overlapping_editors_match_oracle(last):
+def test_wide_overlapping_editors_match_oracle(last, reserved):
     from hashdag_amd import terrain_height
     p, sc, g, dag, od, oc = make("d13")
     F = p.footprint
@@ -28,10 +29,11 @@ def test_wide_overlapping_editors_match_oracle(last):
         edits.append(((SPHERE_ADD, BOX_CARVE, SPHERE_CARVE, BOX_ADD)[k % 4], c, 70.0 + k % 6))
     edits.append((BOX_ADD, (float(x), y, float(z)), 75.0))
     edits.append((last, (float(x + 3), y + 5.0, float(z + 1)), 33.0))
-    # the parents of the leaves' parents expand in rounds of 1024 slots from 2^17 items by the boxes,
-    # where the scratch holds as many (its first size would not)
+    # the leaves' parents expand in rounds of 1024 slots from 2^17 items by the boxes, where the
+    # scratch holds as many (its first size does not)
     assert boxed(edits, 8, 1 << g.levels) >= 1 << 17
-    dag.reserve_edit_scratch(1 << 18, 1 << 20, 1 << 22)
+    if reserved:
+        dag.reserve_edit_scratch(1 << 18, 1 << 20, 1 << 22)
     st = dag.edit_batch(edits, fused=True)
     total = sum(od.edit(kind, c, r, oc)[1] for kind, c, r in edits)
     assert st.passes == 1 and st.num_voxels == total
